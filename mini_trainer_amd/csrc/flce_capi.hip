@@ -10,11 +10,13 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/mt_flce.h"
 #include "flce_kernels.h"
 #include "flce_kernels_bf16.h"
+#include "flce_kernels_f32.h"
 #include "flce_probe.h"
 
 using namespace mtf;
@@ -261,14 +263,13 @@ inline uint32_t range_of(int64_t rows, int64_t ld_b) {
   return (uint32_t)std::min<uint64_t>((uint64_t)std::max<int64_t>(rows, 0) * (uint64_t)ld_b, kMaxBufferBytes);
 }
 
-// Output tiles are 256 x 256 with one workgroup per CU of four waves (bf16
-// and fp32 kernels alike); threads = workgroup size.
+// Output tiles: 256 x 256 with one workgroup per CU (bf16), 128 x 128 with two
+// (fp32).
 struct Geometry {
-  int64_t tile_m, tile_n, slots;
-  int threads;
+  int64_t tile, slots;
 };
 inline Geometry geometry(int es) {
-  return es == 2 ? Geometry{256, 256, kCUs, kThreadsBf} : Geometry{256, 256, kCUs, kThreads};
+  return es == 2 ? Geometry{256, kCUs} : Geometry{kTileF, 2 * kCUs};
 }
 
 // Algorithmic flops of one dX / dW launch (2 x rows x K x columns of the
@@ -448,8 +449,8 @@ struct FwdPlan {
 FwdPlan plan_forward(int64_t n_valid, int64_t V, int es) {
   const Geometry geo = geometry(es);
   FwdPlan p;
-  p.tiles_m = cdiv(n_valid, geo.tile_m);
-  p.vt_total = cdiv(V, geo.tile_n);
+  p.tiles_m = cdiv(n_valid, geo.tile);
+  p.vt_total = cdiv(V, geo.tile);
   if (p.tiles_m == 0) return p;
   if (es == 2) {
     // bf16: one partial per (vocabulary tile, row), tiles scheduled persistently
@@ -677,7 +678,7 @@ int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t 
   a.xy = reinterpret_cast<float*>(ws + align_up((size_t)p.splits * n_valid * 2 * sizeof(float)));
   a.S = nullptr;
   a.lds_b = 0;
-  const bool ktail = H % (sizeof(T) == 2 ? kBKBf : Elt<float>::kBK) != 0;
+  const bool ktail = H % (sizeof(T) == 2 ? kBKBf : kBKF) != 0;
   if constexpr (sizeof(T) == 2) {
     // vocabulary blocks of at most one buffer's reach; each writes the
     // partials of its own tiles, the finalize merges them all
@@ -700,7 +701,7 @@ int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t 
       a.V = (int32_t)vn;
       a.vcol0 = (int32_t)v0;
       a.w_range = range_of(vn, ldw * es);
-      a.vt_total = (int32_t)cdiv(vn, geometry(es).tile_n);
+      a.vt_total = (int32_t)cdiv(vn, geometry(es).tile);
       a.S = kb ? keep : nullptr;
       a.lds_b = kb ? keep_cols * 2 : 0;
       a.s_range = kb ? range_of(p.tiles_m * 256, keep_cols * 2) : 0;
@@ -714,9 +715,11 @@ int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t 
       v0 += vn;
     }
   } else {
-    void (*kern)(FwdArgs) = ktail ? fwd_kernel<T, true> : fwd_kernel<T, false>;
-    hipLaunchKernelGGL(kern, dim3((uint32_t)(p.tiles_m * p.splits)), dim3(kThreads), 0, stream, a);
-    MT_TRY(check_launch("fwd_kernel"));
+    void (*kern)(FwdArgs) = ktail ? fwd_f32_kernel<true> : fwd_f32_kernel<false>;
+    const int pf = prof_begin("fwd_f32_kernel", 2.0 * H * (double)V * n_valid, 0, stream);
+    hipLaunchKernelGGL(kern, dim3((uint32_t)(p.tiles_m * p.splits)), dim3(kThreadsF), 0, stream, a);
+    prof_end(pf, stream);
+    MT_TRY(check_launch("fwd_f32_kernel"));
   }
   hipLaunchKernelGGL(fwd_finalize_kernel, dim3((uint32_t)cdiv(n_valid, 4)), dim3(256), 0, stream,
                      a.part, a.xy, a.N, a.splits, row_index, loss, lse, guard);
@@ -778,16 +781,14 @@ int zero_tiles(const TiledDw& td, int64_t V, int64_t H, hipStream_t s) {
   return MT_OK;
 }
 
-template <typename T>
-int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V, int64_t ldx,
+int launch_backward_bf16(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V, int64_t ldx,
                     int64_t ldw,
                     float softcap, const int32_t* row_index, const int32_t* row_label,
                     int64_t N, const float* lse, const float* grad, int64_t gstride, void* dX,
                     int64_t lddx, float* dW, int64_t lddw, int accumulate, int dw_out, int64_t C,
                     int64_t Cv, char* ws, hipStream_t stream, char* scratch_ext = nullptr,
                     const int32_t* kept_guard = nullptr, const TiledDw* td = nullptr) {
-  constexpr int es = sizeof(T);
-  const Geometry geo = geometry(es);
+  constexpr int es = 2;
   const int64_t nv = cdiv(V, Cv);
   // scratch_ext (the narrowing entry, one row block): dX's accumulator (as
   // tiles) and X^T in the caller's scratch buffer
@@ -809,7 +810,7 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
   for (int64_t c0 = 0; c0 < N; c0 += C) {
     const int64_t cn = std::min(C, N - c0);
     const int64_t cn_pad = round_up(cn, 256);
-    hipLaunchKernelGGL(gather_t_kernel<T>, dim3((uint32_t)(cn_pad / 64), (uint32_t)cdiv(H, 64)),
+    hipLaunchKernelGGL(gather_t_kernel<__bf16>, dim3((uint32_t)(cn_pad / 64), (uint32_t)cdiv(H, 64)),
                        dim3(256), 0, stream, static_cast<const char*>(X), ldx * es, row_index + c0,
                        (int32_t)cn, (int32_t)H, XcT, ldxt_b);
     MT_TRY(check_launch("gather_t_kernel"));
@@ -839,9 +840,9 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
       r.cv = (int32_t)cv;
       r.G = G;
       r.ldg_b = ldg_b;
-      r.tiles_m = (int32_t)cdiv(cn, geo.tile_m);
-      r.tiles_n = (int32_t)cdiv(cv, geo.tile_n);
-      if constexpr (sizeof(T) == 2) r.zero_words = queue;
+      r.tiles_m = (int32_t)cdiv(cn, 256);
+      r.tiles_n = (int32_t)cdiv(cv, 256);
+      r.zero_words = queue;
       // kept_guard (one row block, softcap off): the G block of vocabulary
       // block 0 holds the forward's exponentials; they become G in place,
       // unless the guard was raised, in which case the block is recomputed
@@ -853,25 +854,19 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
         MT_TRY(check_launch("exp_to_grad_kernel"));
         r.run_if = kept_guard;
       }
-      if constexpr (sizeof(T) == 2) {
-        static void (*const kerns[2][2][2])(RecompArgs) = {
-            {{recompute_bf16_kernel<false, false, false>, recompute_bf16_kernel<false, false, true>},
-             {recompute_bf16_kernel<false, true, false>, recompute_bf16_kernel<false, true, true>}},
-            {{recompute_bf16_kernel<true, false, false>, recompute_bf16_kernel<true, false, true>},
-             {recompute_bf16_kernel<true, true, false>, recompute_bf16_kernel<true, true, true>}}};
-        // (a kept block's launch recomputes only if the guard was raised:
-        // recorded apart, without flops, so as not to inflate the rate)
-        const int pr = kept ? prof_begin("recompute_bf16_kernel<if_guard>", 0.0, 0, stream)
-                            : prof_begin("recompute_bf16_kernel", 2.0 * H * (double)cn * cv, 0, stream);
-        hipLaunchKernelGGL(kerns[softcap > 0.f][cv % 256 != 0][H % kBKBf != 0],
-                           dim3(persistent_grid(r.tiles_m * r.tiles_n)),
-                           dim3(kThreadsBf), 0, stream, r);
-        prof_end(pr, stream);
-      } else {
-        void (*kern)(RecompArgs) =
-            H % Elt<float>::kBK != 0 ? recompute_kernel<T, true> : recompute_kernel<T, false>;
-        hipLaunchKernelGGL(kern, dim3((uint32_t)(r.tiles_m * r.tiles_n)), dim3(kThreads), 0, stream, r);
-      }
+      static void (*const kerns[2][2][2])(RecompArgs) = {
+          {{recompute_bf16_kernel<false, false, false>, recompute_bf16_kernel<false, false, true>},
+           {recompute_bf16_kernel<false, true, false>, recompute_bf16_kernel<false, true, true>}},
+          {{recompute_bf16_kernel<true, false, false>, recompute_bf16_kernel<true, false, true>},
+           {recompute_bf16_kernel<true, true, false>, recompute_bf16_kernel<true, true, true>}}};
+      // (a kept block's launch recomputes only if the guard was raised:
+      // recorded apart, without flops, so as not to inflate the rate)
+      const int pr = kept ? prof_begin("recompute_bf16_kernel<if_guard>", 0.0, 0, stream)
+                          : prof_begin("recompute_bf16_kernel", 2.0 * H * (double)cn * cv, 0, stream);
+      hipLaunchKernelGGL(kerns[softcap > 0.f][cv % 256 != 0][H % kBKBf != 0],
+                         dim3(persistent_grid(r.tiles_m * r.tiles_n)),
+                         dim3(kThreadsBf), 0, stream, r);
+      prof_end(pr, stream);
       MT_TRY(check_launch("recompute_kernel"));
 
       DxArgs x;
@@ -893,8 +888,8 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
       x.dX = static_cast<char*>(dX);
       x.lddx_b = lddx * es;
       x.row_index = row_index + c0;
-      x.tiles_m = (int32_t)cdiv(cn, geo.tile_m);
-      x.tiles_n = (int32_t)cdiv(H, geo.tile_n);
+      x.tiles_m = (int32_t)cdiv(cn, 256);
+      x.tiles_n = (int32_t)cdiv(H, 256);
       // dX with fewer tiles than CUs leaves CUs idle for its whole (long) K:
       // dW then runs beside it, in the same launch.  Otherwise dX and the
       // persistent dW run one after the other on the caller's stream
@@ -905,20 +900,15 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
       // (the grid-cap test hook stands in for a smaller GPU here too, so small
       // tests reach the one-after-the-other form)
       const int64_t cus = grid_cap() > 0 ? std::min(grid_cap(), device_cus()) : device_cus();
-      const bool beside = sizeof(T) == 2 &&
-                          (dw_out == kDwNarrow || (int64_t)x.tiles_m * x.tiles_n < cus);
+      const bool beside = dw_out == kDwNarrow || (int64_t)x.tiles_m * x.tiles_n < cus;
       // dW beside dX over the work queue (as on the fused path), which the
       // recompute launch just before the fork clears
       const bool use_queue = beside && cdiv(cv, 256) * cdiv(H, 256) >= 4 * device_cus() &&
                              device_cus() % kQueueWords == 0 && cn > kBKBf;
       if (!beside) {
-        if constexpr (sizeof(T) == 2) {
-          const int px = prof_begin(dx_name(x.mode), dx_flops(x), 0, stream);
-          launch_dx_bf16(x, stream);
-          prof_end(px, stream);
-        } else
-          hipLaunchKernelGGL(dx_kernel<T>, dim3((uint32_t)(x.tiles_m * x.tiles_n)), dim3(kThreads), 0,
-                             stream, x);
+        const int px = prof_begin(dx_name(x.mode), dx_flops(x), 0, stream);
+        launch_dx_bf16(x, stream);
+        prof_end(px, stream);
         MT_TRY(check_launch("dx_kernel"));
       }
 
@@ -938,8 +928,8 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
       w.dW = dW;
       w.lddw = lddw;
       w.accumulate = (accumulate || c0 > 0) ? 1 : 0;
-      w.tiles_m = (int32_t)cdiv(cv, geo.tile_m);
-      w.tiles_n = (int32_t)cdiv(H, geo.tile_n);
+      w.tiles_m = (int32_t)cdiv(cv, 256);
+      w.tiles_n = (int32_t)cdiv(H, 256);
       if (dw_out == kDwTiles) set_tiled(w, *td, H);  // (bf16; the block's tile rows start at v0 / 256)
       if (dw_out == kDwNarrow) w.narrow = 1;  // dW: bf16 rows of pitch lddw
       if (use_queue) w.queue = queue;
@@ -947,20 +937,193 @@ int launch_backward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t
         // the next block's recompute (G) and gather (X^T) follow the join
         MT_TRY(launch_dx_dw_bf16(x, w, stream));
       } else {
-        if constexpr (sizeof(T) == 2) {
-          const int pw = prof_begin("dw_bf16_kernel", dw_flops(w), 0, stream);
-          static void (*const kd[3])(DwArgs) = {dw_bf16_kernel<false, kDwRows>,
-                                                dw_bf16_kernel<false, kDwTiles>,
-                                                dw_bf16_kernel<false, kDwNarrow>};
-          void (*kern)(DwArgs) = kd[dw_out];
-          hipLaunchKernelGGL(kern, dim3(persistent_grid(w.tiles_m * w.tiles_n)),
-                             dim3(kThreadsBf), 0, stream, w);
-          prof_end(pw, stream);
-        } else
-          hipLaunchKernelGGL(dw_kernel<T>, dim3((uint32_t)(w.tiles_m * w.tiles_n)), dim3(kThreads), 0,
-                             stream, w);
+        const int pw = prof_begin("dw_bf16_kernel", dw_flops(w), 0, stream);
+        static void (*const kd[3])(DwArgs) = {dw_bf16_kernel<false, kDwRows>,
+                                              dw_bf16_kernel<false, kDwTiles>,
+                                              dw_bf16_kernel<false, kDwNarrow>};
+        void (*kern)(DwArgs) = kd[dw_out];
+        hipLaunchKernelGGL(kern, dim3(persistent_grid(w.tiles_m * w.tiles_n)),
+                           dim3(kThreadsBf), 0, stream, w);
+        prof_end(pw, stream);
         MT_TRY(check_launch("dw_kernel"));
       }
+    }
+  }
+  return MT_OK;
+}
+
+// --------------------------------------------------------- fp32 backward
+// How one fp32 row block is worked through inside a workspace of `bytes`:
+// X^T [H, C], `planes` fp32 planes [C, H] of dX, and the rest the G block of
+// C x Cv.  dX has few output tiles (C / 128 x H / 128) that each contract a
+// whole vocabulary block, so each is split over the block's columns into S
+// slices with a plane of their own: one slice each left config 1's dX (20
+// tiles of 256 x 256 at the time) on 20 of 256 CUs, 38.6 of the step's 51.6
+// ms.  A plane costs H columns of G, i.e. more and smaller blocks; S and Cv
+// minimise the modelled time of a row block: tiles of the recompute by whole
+// rounds of CUs, dX and dW items as the dispatcher places them, and per block
+// two launches.
+struct F32Blocks {
+  int64_t S = 1, Cv = 0, planes = 0;
+};
+
+// End of n1 items of length l1, then n2 of length l2, each started on the slot
+// that frees up first (slots alike, kept as groups of equal finishing time).
+double list_makespan(int64_t slots, int64_t n1, double l1, int64_t n2, double l2) {
+  std::vector<std::pair<double, int64_t>> g{{0.0, slots}};  // ascending times
+  double end = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    int64_t n = pass ? n2 : n1;
+    const double l = pass ? l2 : l1;
+    while (n > 0) {
+      const double t = g[0].first + l;
+      const int64_t k = std::min(n, g[0].second);
+      g[0].second -= k;
+      n -= k;
+      if (g[0].second == 0) g.erase(g.begin());
+      auto it = g.begin();
+      while (it != g.end() && it->first < t) ++it;
+      if (it != g.end() && it->first == t) it->second += k;
+      else g.insert(it, {t, k});
+      end = std::max(end, t);
+    }
+  }
+  return end;
+}
+F32Blocks f32_blocks(int64_t C, int64_t cn, int64_t H, int64_t V, size_t bytes) {
+  const int64_t xt = (int64_t)align_up((size_t)H * C * 4), plane = C * H * 4;
+  const int64_t tm = cdiv(cn, kTileF), th = cdiv(H, kTileF), vt = cdiv(V, kTileF);
+  // in K entries of one CU's 128 x 128 tile (~55 ns): an item's prologue and
+  // epilogue, a launch
+  constexpr int64_t kItem = 48, kLaunchK = 90;
+  F32Blocks best;
+  double best_t = 0;
+  for (int64_t S = 1; S <= 16; ++S) {
+    for (int64_t more = 0; more <= 8; ++more) {
+      const bool emit = S == 1 && (int64_t)bytes - xt >= C * vt * kTileF * 4 && more == 0;
+      const int64_t planes = emit ? 0 : S;
+      const int64_t cap = ((int64_t)bytes - xt - planes * plane) / (C * 4) / kTileF;  // tiles
+      if (cap < 1) break;
+      const int64_t nv = cdiv(vt, std::min(cap, vt)) + more;
+      const int64_t ct = cdiv(vt, nv), cols = ct * kTileF;
+      if (S > 1 && cols / S < 2 * kBKF) break;
+      const double phase = list_makespan(2 * kCUs, tm * th * S, 2.0 * (cdiv(cols, S) + kItem), ct * th,
+                                         2.0 * (cn + kItem));
+      const double t = nv * ((double)cdiv(tm * ct, kCUs) * (H + kItem) + phase + 2 * kLaunchK);
+      if (best.Cv == 0 || t < best_t) {
+        best_t = t;
+        best.S = S;
+        best.Cv = cols;
+        best.planes = planes;
+      }
+      if (emit) break;
+    }
+  }
+  return best;
+}
+
+int launch_backward_f32(const void* X, const void* W, int64_t H, int64_t V, int64_t ldx, int64_t ldw,
+                        float softcap, const int32_t* row_index, const int32_t* row_label, int64_t N,
+                        const float* lse, const float* grad, int64_t gstride, void* dX, int64_t lddx,
+                        float* dW, int64_t lddw, int accumulate, int64_t C, char* ws, size_t ws_bytes,
+                        hipStream_t stream) {
+  for (int64_t c0 = 0; c0 < N; c0 += C) {
+    const int64_t cn = std::min(C, N - c0), cn_pad = round_up(cn, 256);
+    const F32Blocks b = f32_blocks(C, cn, H, V, ws_bytes);
+    if (b.Cv == 0)
+      return fail(MT_ERR_WORKSPACE_TOO_SMALL, "fp32 backward workspace %zu bytes holds no block", ws_bytes);
+    char* XcT = ws;
+    float* planes = reinterpret_cast<float*>(ws + align_up((size_t)H * C * 4));
+    char* G = reinterpret_cast<char*>(planes + b.planes * C * H);
+    const int64_t nv = cdiv(V, b.Cv), ldg_b = b.Cv * 4;
+    hipLaunchKernelGGL(gather_t_kernel<float>, dim3((uint32_t)(cn_pad / 64), (uint32_t)cdiv(H, 64)),
+                       dim3(256), 0, stream, static_cast<const char*>(X), ldx * 4, row_index + c0,
+                       (int32_t)cn, (int32_t)H, XcT, C * 4);
+    MT_TRY(check_launch("gather_t_kernel"));
+    int64_t j = 0;
+    for (int64_t v0 = 0; v0 < V; v0 += b.Cv, ++j) {
+      const int64_t cv = std::min(b.Cv, V - v0);
+      const char* Wv = static_cast<const char*>(W) + v0 * ldw * 4;
+      RecompArgs r;
+      r.X = static_cast<const char*>(X);
+      r.W = Wv;
+      r.ldx_b = ldx * 4;
+      r.ldw_b = ldw * 4;
+      r.H = (int32_t)H;
+      r.V = (int32_t)V;
+      r.x_range = r.w_range = r.g_range = 0;  // (64-bit addresses)
+      r.row_index = row_index + c0;
+      r.row_label = row_label + c0;
+      r.lse = lse + c0;
+      r.Cn = (int32_t)cn;
+      r.grad = grad;
+      r.gstride = gstride;
+      r.softcap = softcap;
+      r.v0 = (int32_t)v0;
+      r.cv = (int32_t)cv;
+      r.G = G;
+      r.ldg_b = ldg_b;
+      r.tiles_m = (int32_t)cdiv(cn, kTileF);
+      r.tiles_n = (int32_t)cdiv(cv, kTileF);
+      void (*rec)(RecompArgs) = H % kBKF != 0 ? recompute_f32_kernel<true> : recompute_f32_kernel<false>;
+      const int pr = prof_begin("recompute_f32_kernel", 2.0 * H * (double)cn * cv, 0, stream);
+      hipLaunchKernelGGL(rec, dim3((uint32_t)(r.tiles_m * r.tiles_n)), dim3(kThreadsF), 0, stream, r);
+      prof_end(pr, stream);
+      MT_TRY(check_launch("recompute_kernel"));
+
+      DxArgs x;
+      x.G = G;
+      x.ldg_b = ldg_b;
+      x.W = Wv;
+      x.ldw_b = ldw * 4;
+      x.g_range = x.w_range = 0;
+      x.V = (int32_t)(v0 + cv);  // K rows past the block's end repeat its last row (times zero G)
+      x.v0 = (int32_t)v0;
+      x.kv = (int32_t)cv;
+      x.H = (int32_t)H;
+      x.Cn = (int32_t)cn;
+      x.accbuf = planes;
+      x.ld_acc = H;
+      x.mode = b.S > 1 ? (j == 0 ? kDxStore : kDxAdd)
+                       : nv == 1 ? kDxEmit : (j == 0 ? kDxStore : (j == nv - 1 ? kDxAddEmit : kDxAdd));
+      x.dX = static_cast<char*>(dX);
+      x.lddx_b = lddx * 4;
+      x.row_index = row_index + c0;
+      x.tiles_m = r.tiles_m;
+      x.tiles_n = (int32_t)cdiv(H, kTileF);
+      x.nsplit = (int32_t)b.S;
+      x.kslice = (int32_t)round_up(cdiv(cv, b.S), kBKF);
+      x.split_stride = C * H;
+
+      DwArgs w;
+      w.G = G;
+      w.ldg_b = ldg_b;
+      w.g_rows = (int32_t)cn_pad;
+      w.g_cols = (int32_t)b.Cv;
+      w.XcT = XcT;
+      w.ldxt_b = C * 4;
+      w.g_range = w.xt_range = 0;
+      w.kt_rows = (int32_t)cn;
+      w.H = (int32_t)H;
+      w.cv = (int32_t)cv;
+      w.v0 = (int32_t)v0;
+      w.dW = dW;
+      w.lddw = lddw;
+      w.accumulate = (accumulate || c0 > 0) ? 1 : 0;
+      w.tiles_m = r.tiles_n;
+      w.tiles_n = x.tiles_n;
+      const int64_t dxg = (int64_t)x.tiles_m * x.tiles_n * b.S, dwg = (int64_t)w.tiles_m * w.tiles_n;
+      const int pd = prof_begin("dx_dw_f32_kernel", dx_flops(x) + dw_flops(w), 0, stream);
+      hipLaunchKernelGGL(dx_dw_f32_kernel, dim3((uint32_t)(dxg + dwg)), dim3(kThreadsF), 0, stream, x, w,
+                         (uint32_t)dxg);
+      prof_end(pd, stream);
+      MT_TRY(check_launch("dx_dw_f32_kernel"));
+    }
+    if (b.S > 1) {
+      hipLaunchKernelGGL(dx_sum_f32_kernel, dim3((uint32_t)cdiv(cn * (H / 4), 256)), dim3(256), 0, stream,
+                         planes, C * H, (int32_t)b.S, (int32_t)cn, (int32_t)H, row_index + c0,
+                         static_cast<char*>(dX), lddx * 4);
+      MT_TRY(check_launch("dx_sum_f32_kernel"));
     }
   }
   return MT_OK;
@@ -1572,15 +1735,15 @@ int backward_entry(const void* X, const void* W, int64_t T, int64_t H, int64_t V
   }
   if (dtype == MT_DTYPE_BF16) {
     char* scratch_ext = outside ? static_cast<char*>(scratch) : nullptr;
-    return launch_backward<__bf16>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
+    return launch_backward_bf16(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
                                    grad_loss, grad_stride, dX, lddx, dW,
                                    dw_out == kDwNarrow ? H : lddw, accumulate_dW, dw_out, chunk_rows,
                                    chunk_vocab, static_cast<char*>(workspace), s, scratch_ext,
                                    kept_guard, td);
   }
-  return launch_backward<float>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
-                                grad_loss, grad_stride, dX, lddx, dW, lddw, accumulate_dW, kDwRows,
-                                chunk_rows, chunk_vocab, static_cast<char*>(workspace), s);
+  return launch_backward_f32(X, W, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
+                             grad_loss, grad_stride, dX, lddx, dW, lddw, accumulate_dW, chunk_rows,
+                             static_cast<char*>(workspace), workspace_bytes, s);
 }
 
 }  // namespace

@@ -56,7 +56,7 @@
 //   row = wm * 128 + fm * 16 + (l & 15),  col = wn * 128 + fn * 16 + 4 (l >> 4) + r.
 #pragma once
 
-#include "flce_gemm.h"
+#include "flce_device.h"
 
 namespace mtf {
 
@@ -305,7 +305,7 @@ __device__ __forceinline__ void tie_frags(u32x4_t (&fr)[8]) {
 // MFMA i (0..63) of a phase: fragment row fm = i / 8, column fn = i % 8.
 __device__ __forceinline__ void mfma_one(f32x4_t (&acc)[8][8], const u32x4_t (&fa)[8],
                                          const u32x4_t (&fb)[8], int i) {
-  acc[i >> 3][i & 7] = mma_chunk<__bf16>(fb[i & 7], fa[i >> 3], acc[i >> 3][i & 7]);
+  acc[i >> 3][i & 7] = mma_chunk(fb[i & 7], fa[i >> 3], acc[i >> 3][i & 7]);
 }
 
 // Accumulators start at zero (the init hook of every kernel but dW).

@@ -1,28 +1,19 @@
 // Kernels of the fused LM-head linear + per-token cross-entropy path.
 //
-//   fwd_kernel       logits tile = X_rows . W_tile^T (MFMA), fused online
-//                    log-sum-exp over the vocabulary and label-logit capture;
-//                    no logits are written to memory.
-//   fwd_finalize     merge of the per-split (max, sum) partials -> lse, loss.
-//   recompute_kernel logits tile recomputed and turned into
-//                    G = g * (softmax - onehot) (bf16 / fp32) for one block.
-//   dx_kernel        dX_block (+)= G . W_block    (W consumed K-major)
-//   dw_kernel        dW_block (+)= G^T . X_block  (G consumed K-major)
+//   argument structures of the GEMM-shaped kernels (flce_kernels_bf16.h,
+//   flce_kernels_f32.h) and what both share of their epilogues
+//   fwd_finalize     merge of the per-split (max, sum) partials -> lse, loss
 //   small kernels    valid-row compaction, gather-transpose of X rows,
 //                    zeroing of ignored rows, per-sample segment sums.
 #pragma once
 
-#include "flce_gemm.h"
+#include "flce_device.h"
 
 namespace mtf {
 
-#define MT_GEMM_KERNEL \
-  __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
-
 // Output coordinates of this lane's accumulators for a wave tile of
 // 128 rows x (NFN * 16) columns, WC waves across the tile's columns (tile
-// width NFN * 16 * WC: 8 x 16 x 2 for the four-wave fp32 kernels, 4 x 16 x 4
-// for the eight-wave bf16 kernels).
+// width NFN * 16 * WC: 8 x 16 x 2 for the bf16 kernels).
 template <int NFN, int WC = 2>
 struct EpiCoordsT {
   static constexpr int kNF = NFN;
@@ -42,7 +33,6 @@ struct EpiCoordsT {
     return wn * (NFN * 16) + fn * 16 + 4 * (lane >> 4);
   }
 };
-typedef EpiCoordsT<8> EpiCoords;
 
 // Is column offset `rel` (label column minus this lane's column of fn = 0,
 // r = 0) one of the NFN * 4 columns this lane holds?
@@ -72,74 +62,6 @@ struct FwdArgs {
   const int32_t* run_if = nullptr;  // non-null: the kernel does nothing unless *run_if != 0
   int32_t* guard_reset = nullptr;   // non-null: set to 0 by the launch (read only after it)
 };
-
-// Columns at or beyond V are masked with a select (no separate tail variant:
-// one code path keeps the epilogue's register footprint small).
-template <typename T, int NFN, bool kCap>
-__device__ __forceinline__ void fwd_tile_epilogue(const f32x4_t (&acc)[8][NFN], float (&m2)[8],
-                                                  float (&d)[8], const int32_t (&rel)[8],
-                                                  const int32_t (&rglob)[8], int32_t ncol0,
-                                                  const FwdArgs& a, bool any_hit) {
-  const float cap = a.softcap, inv_cap = kCap ? 1.0f / a.softcap : 0.f;
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    float v[NFN][4];
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int fn = 0; fn < NFN; ++fn) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[fn][r] = acc[fm][fn][r];
-      round_pair<T>(v[fn][0], v[fn][1]);
-      round_pair<T>(v[fn][2], v[fn][3]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float x = v[fn][r];
-        if (kCap) x = cap * tanh_approx(x * inv_cap);
-        x = ncol0 + fn * 16 + r < a.V ? x : -INFINITY;
-        v[fn][r] = x;
-        tmax = fmaxf(tmax, x);
-      }
-    }
-    const float mn = fmaxf(m2[fm], tmax * kLog2e);
-    float s = 0.f;
-#pragma unroll
-    for (int fn = 0; fn < NFN; ++fn)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s += fast_exp2(fmaf(v[fn][r], kLog2e, -mn));
-    d[fm] = fmaf(d[fm], fast_exp2(m2[fm] - mn), s);
-    m2[fm] = mn;
-    if (any_hit) {
-      const int rl = rel[fm];
-      if (lane_holds<NFN>(rl) && rglob[fm] < a.N) {
-        float hitv = 0.f;
-#pragma unroll
-        for (int fn = 0; fn < NFN; ++fn)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) hitv = (rl == fn * 16 + r) ? v[fn][r] : hitv;
-        a.xy[rglob[fm]] = hitv;
-      }
-    }
-  }
-}
-
-// Online-LSE update of one finished 256 x 256 logits tile (vocabulary rows
-// vrow0 .. vrow0 + 255) plus label-logit capture.
-template <typename T, bool kCap, int NFN, int WC>
-__device__ __forceinline__ void fwd_tile_update(const f32x4_t (&acc)[8][NFN], float (&m2)[8],
-                                                float (&d)[8], const int32_t (&lbl)[8],
-                                                const int32_t (&rglob)[8], int32_t vrow0,
-                                                const EpiCoordsT<NFN, WC>& ec, const FwdArgs& a) {
-  const int32_t ncol0 = vrow0 + ec.col(0);
-  int32_t rel[8];
-  bool hit = false;
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    rel[fm] = lbl[fm] - ncol0;
-    hit |= lane_holds<NFN>(rel[fm]);
-  }
-  const bool any_hit = __builtin_amdgcn_ballot_w64(hit) != 0;
-  fwd_tile_epilogue<T, NFN, kCap>(acc, m2, d, rel, rglob, ncol0, a, any_hit);
-}
 
 // x of lane l ^ 16 and of lane l ^ 32, from one lane swap and a select
 // (v_permlane16_swap / v_permlane32_swap with x as both operands hand back
@@ -194,57 +116,6 @@ __device__ __forceinline__ void fwd_final_merge(char* lds, float (&m2)[8], float
       }
     }
   }
-}
-
-// kKTail: H is not a multiple of the K slab (the last slab is partial).
-template <typename T, bool kKTail>
-MT_GEMM_KERNEL void fwd_kernel(FwdArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
-  uint32_t tm, ts;
-  grouped_tile(xcd_remap(blockIdx.x, gridDim.x), a.tiles_m, a.splits, 4, tm, ts);
-  const EpiCoords ec;
-  FragOffsets fo;
-  fo.init();
-
-  const int32_t row0 = (int32_t)tm * 256;
-  DirectLoader la;
-  la.init([&](uint32_t r) __attribute__((always_inline)) {
-    int32_t rr = row0 + (int32_t)r;
-    rr = rr < a.N ? rr : a.N - 1;
-    return a.X + (int64_t)a.row_index[rr] * a.ldx_b;
-  });
-
-  int32_t lbl[8], rglob[8];
-  float m2[8], d[8];
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    rglob[fm] = row0 + ec.row(fm);
-    lbl[fm] = rglob[fm] < a.N ? a.row_label[rglob[fm]] : -1;
-    m2[fm] = kNegBig;
-    d[fm] = 0.f;
-  }
-
-  const int KT = (a.H + Elt<T>::kBK - 1) / Elt<T>::kBK;
-  const uint32_t c_lim = (uint32_t)(a.H - (KT - 1) * Elt<T>::kBK) / Elt<T>::kPerChunk;
-  if constexpr (kKTail) la.set_tail(c_lim);
-  const int vt0 = (int)ts * a.vt_per_split;
-  const int vt1 = min(vt0 + a.vt_per_split, a.vt_total);
-  f32x4_t acc[8][8];
-  for (int vt = vt0; vt < vt1; ++vt) {
-    const int32_t vrow0 = vt * 256;
-    DirectLoader lb;
-    lb.init([&](uint32_t r) __attribute__((always_inline)) {
-      int32_t v = vrow0 + (int32_t)r;
-      v = v < a.V ? v : a.V - 1;
-      return a.W + (int64_t)v * a.ldw_b;
-    });
-    if constexpr (kKTail) lb.set_tail(c_lim);
-    mainloop<T, kKTail>(lds, acc, la, lb, KT, fo, c_lim);
-
-    if (a.softcap > 0.f) fwd_tile_update<T, true>(acc, m2, d, lbl, rglob, vrow0, ec, a);
-    else fwd_tile_update<T, false>(acc, m2, d, lbl, rglob, vrow0, ec, a);
-  }
-  fwd_final_merge(lds, m2, d, rglob, ts, ec, a);
 }
 
 // lse and loss of each valid row from its `splits` (max, sum) partials: one
@@ -383,103 +254,6 @@ __global__ __launch_bounds__(256) void exp_to_grad_kernel(char* G, int64_t ldg_b
   }
 }
 
-template <typename T>
-__device__ __forceinline__ void store4(char* p, const float (&o)[4]);
-template <>
-__device__ __forceinline__ void store4<__bf16>(char* p, const float (&o)[4]) {
-  u32x2_t w;
-  w.x = pack_bf16x2(o[0], o[1]);
-  w.y = pack_bf16x2(o[2], o[3]);
-  *reinterpret_cast<u32x2_t*>(p) = w;
-}
-template <>
-__device__ __forceinline__ void store4<float>(char* p, const float (&o)[4]) {
-  *reinterpret_cast<f32x4_t*>(p) = f32x4_t{o[0], o[1], o[2], o[3]};
-}
-
-template <typename T, int NFN, bool kCap, int WC>
-__device__ __forceinline__ void recompute_epilogue(const f32x4_t (&acc)[8][NFN], const RecompArgs& a,
-                                                   const EpiCoordsT<NFN, WC>& ec, int32_t row0,
-                                                   int32_t col0) {
-  const float cap = a.softcap, inv_cap = kCap ? 1.0f / a.softcap : 0.f;
-  const int32_t ncol0 = col0 + ec.col(0);  // block-local column of fn = 0, r = 0
-  int32_t rel[8], rowl[8];
-  float lse2[8], g[8];
-  bool hit = false;
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    rowl[fm] = row0 + ec.row(fm);
-    const bool rv = rowl[fm] < a.Cn;
-    const int32_t rr = rv ? rowl[fm] : 0;
-    lse2[fm] = a.lse[rr] * kLog2e;
-    g[fm] = rv ? a.grad[(int64_t)a.row_index[rr] * a.gstride] : 0.f;
-    rel[fm] = rv ? a.row_label[rr] - a.v0 - ncol0 : -1;
-    hit |= lane_holds<NFN>(rel[fm]);
-  }
-  const bool any_hit = __builtin_amdgcn_ballot_w64(hit) != 0;
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    const bool rv = rowl[fm] < a.Cn;
-    char* grow = a.G + (int64_t)rowl[fm] * a.ldg_b;
-#pragma unroll
-    for (int fn = 0; fn < NFN; ++fn) {
-      float o[4];
-      float xr[4] ={acc[fm][fn][0], acc[fm][fn][1], acc[fm][fn][2], acc[fm][fn][3]};
-      round_pair<T>(xr[0], xr[1]);
-      round_pair<T>(xr[2], xr[3]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float x = xr[r];
-        float dcap = 1.f;
-        if (kCap) {
-          const float t = tanh_approx(x * inv_cap);
-          x = cap * t;
-          dcap = 1.f - t * t;
-        }
-        float p = fast_exp2(fmaf(x, kLog2e, -lse2[fm]));
-        if (any_hit) p -= (rel[fm] == fn * 16 + r) ? 1.f : 0.f;
-        const bool ok = rv && (ncol0 + fn * 16 + r < a.cv);
-        o[r] = ok ? p * g[fm] * dcap : 0.f;
-      }
-      store4<T>(grow + (int64_t)(ncol0 + fn * 16) * Elt<T>::kBytes, o);
-    }
-  }
-}
-
-template <typename T, bool kKTail>
-MT_GEMM_KERNEL void recompute_kernel(RecompArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
-  uint32_t tm, tn;
-  grouped_tile(xcd_remap(blockIdx.x, gridDim.x), a.tiles_m, a.tiles_n, 4, tm, tn);
-  const EpiCoords ec;
-  FragOffsets fo;
-  fo.init();
-  const int32_t row0 = (int32_t)tm * 256;
-  DirectLoader la;
-  la.init([&](uint32_t r) __attribute__((always_inline)) {
-    int32_t rr = row0 + (int32_t)r;
-    rr = rr < a.Cn ? rr : a.Cn - 1;
-    return a.X + (int64_t)a.row_index[rr] * a.ldx_b;
-  });
-  const int32_t vloc0 = (int32_t)tn * 256;  // rows from the block's first (W's row 0)
-  DirectLoader lb;
-  lb.init([&](uint32_t r) __attribute__((always_inline)) {
-    int32_t v = vloc0 + (int32_t)r;
-    v = v < a.cv ? v : a.cv - 1;  // rows past the block repeat its last one
-    return a.W + (int64_t)v * a.ldw_b;
-  });
-  f32x4_t acc[8][8];
-  const int KT = (a.H + Elt<T>::kBK - 1) / Elt<T>::kBK;
-  const uint32_t c_lim = (uint32_t)(a.H - (KT - 1) * Elt<T>::kBK) / Elt<T>::kPerChunk;
-  if constexpr (kKTail) {
-    la.set_tail(c_lim);
-    lb.set_tail(c_lim);
-  }
-  mainloop<T, kKTail>(lds, acc, la, lb, KT, fo, c_lim);
-  if (a.softcap > 0.f) recompute_epilogue<T, 8, true>(acc, a, ec, row0, (int32_t)tn * 256);
-  else recompute_epilogue<T, 8, false>(acc, a, ec, row0, (int32_t)tn * 256);
-}
-
 // ===========================================================================
 // Backward, step 2: dX rows of the block (+)= G . W[v0 : v0 + cv]
 // ===========================================================================
@@ -540,54 +314,6 @@ __global__ __launch_bounds__(256) void dx_split_reduce_kernel(const float* part,
   *reinterpret_cast<u32x2_t*>(dX + (int64_t)row_index[t] * lddx_b + (int64_t)h * 2) = o;
 }
 
-template <typename T, int NFN, int WC>
-__device__ __forceinline__ void dx_epilogue(const f32x4_t (&acc)[8][NFN], const DxArgs& a,
-                                            const EpiCoordsT<NFN, WC>& ec, int32_t row0, int32_t h0) {
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    const int32_t rowl = row0 + ec.row(fm);
-    if (rowl >= a.Cn) continue;
-    float* arow = a.accbuf + (int64_t)rowl * a.ld_acc;
-    char* xrow = a.dX + (int64_t)a.row_index[rowl] * a.lddx_b;
-#pragma unroll
-    for (int fn = 0; fn < NFN; ++fn) {
-      const int32_t h = h0 + ec.col(fn);
-      if (h >= a.H) continue;
-      f32x4_t v = acc[fm][fn];
-      if (a.mode == kDxStore) {
-        *reinterpret_cast<f32x4_t*>(arow + h) = v;
-      } else if (a.mode == kDxAdd) {
-        v += *reinterpret_cast<const f32x4_t*>(arow + h);
-        *reinterpret_cast<f32x4_t*>(arow + h) = v;
-      } else {
-        if (a.mode == kDxAddEmit) v += *reinterpret_cast<const f32x4_t*>(arow + h);
-        const float o[4] = {v[0], v[1], v[2], v[3]};
-        store4<T>(xrow + (int64_t)h * Elt<T>::kBytes, o);
-      }
-    }
-  }
-}
-
-template <typename T>
-MT_GEMM_KERNEL void dx_kernel(DxArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
-  uint32_t tm, tn;
-  grouped_tile(xcd_remap(blockIdx.x, gridDim.x), a.tiles_m, a.tiles_n, 4, tm, tn);
-  const EpiCoords ec;
-  FragOffsets fo;
-  fo.init();
-  const int32_t row0 = (int32_t)tm * 256;
-  DirectLoader la;
-  la.init([&](uint32_t r) __attribute__((always_inline)) { return a.G + (int64_t)(row0 + (int32_t)r) * a.ldg_b; });
-  const int32_t h0 = (int32_t)tn * 256;
-  TransLoader<T> lb;
-  lb.init(a.W + (int64_t)h0 * Elt<T>::kBytes, a.ldw_b, a.V - a.v0, a.H - h0);
-  f32x4_t acc[8][8];
-  const int KT = (a.kv + Elt<T>::kBK - 1) / Elt<T>::kBK;
-  mainloop<T>(lds, acc, la, lb, KT, fo);
-  dx_epilogue<T, 8>(acc, a, ec, row0, h0);
-}
-
 // ===========================================================================
 // Backward, step 3: dW[v0 : v0 + cv] (+)= G^T . X_block
 // ===========================================================================
@@ -630,49 +356,6 @@ struct DwArgs {
 // pitch lddw (elements) at dW, narrowed in the epilogue.
 constexpr int kDwRows = 0, kDwTiles = 1, kDwNarrow = 2;
 
-template <int NFN, int WC>
-__device__ __forceinline__ void dw_epilogue(const f32x4_t (&acc)[8][NFN], const DwArgs& a,
-                                            const EpiCoordsT<NFN, WC>& ec, int32_t m0, int32_t h0) {
-#pragma unroll
-  for (int fm = 0; fm < 8; ++fm) {
-    const int32_t vl = m0 + ec.row(fm);
-    if (vl >= a.cv) continue;
-    float* wrow = a.dW + (int64_t)(a.v0 + vl) * a.lddw;
-#pragma unroll
-    for (int fn = 0; fn < NFN; ++fn) {
-      const int32_t h = h0 + ec.col(fn);
-      if (h >= a.H) continue;
-      f32x4_t v = acc[fm][fn];
-      if (a.accumulate) v += *reinterpret_cast<const f32x4_t*>(wrow + h);
-      *reinterpret_cast<f32x4_t*>(wrow + h) = v;
-    }
-  }
-}
-
-template <typename T>
-MT_GEMM_KERNEL void dw_kernel(DwArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
-  uint32_t tm, tn;
-  grouped_tile(xcd_remap(blockIdx.x, gridDim.x), a.tiles_m, a.tiles_n, 4, tm, tn);
-  const EpiCoords ec;
-  FragOffsets fo;
-  fo.init();
-  const int32_t m0 = (int32_t)tm * 256;
-  TransLoader<T> la;
-  la.init(a.G + (int64_t)m0 * Elt<T>::kBytes, a.ldg_b, a.g_rows, a.g_cols - m0);
-  const int32_t h0 = (int32_t)tn * 256;
-  DirectLoader lb;
-  lb.init([&](uint32_t r) __attribute__((always_inline)) {
-    int32_t h = h0 + (int32_t)r;
-    h = h < a.H ? h : a.H - 1;
-    return a.XcT + (int64_t)h * a.ldxt_b;
-  });
-  f32x4_t acc[8][8];
-  const int KT = (a.kt_rows + Elt<T>::kBK - 1) / Elt<T>::kBK;
-  mainloop<T>(lds, acc, la, lb, KT, fo);
-  dw_epilogue<8>(acc, a, ec, m0, h0);
-}
-
 // ===========================================================================
 // Small kernels
 // ===========================================================================
@@ -687,7 +370,7 @@ __global__ __launch_bounds__(256) void gather_t_kernel(const char* X, int64_t ld
                                                        const int32_t* row_index, int32_t Cn,
                                                        int32_t H, char* XcT, int64_t ldxt_b,
                                                        const float* scale = nullptr) {
-  constexpr int E = Elt<T>::kBytes;
+  constexpr int E = sizeof(T);
   constexpr int PER = 16 / E;  // elements per 16-byte vector
   __shared__ T tile[64][64 + 1];
   const int32_t t0 = blockIdx.x * 64, hb = blockIdx.y * 64;

@@ -1,7 +1,5 @@
 // bf16 kernels on the four-wave main loop (flce_gemm_bf16.h): output tiles
-// of 256 x 256, wave tiles 128 x 128.  Arguments, accumulation order and
-// epilogues are those of the generic kernels in flce_kernels.h (the fp32
-// path).
+// of 256 x 256, wave tiles 128 x 128.
 #pragma once
 
 #include "flce_gemm_bf16.h"
@@ -440,8 +438,8 @@ __device__ __forceinline__ void recompute_epilogue_bf16(const f32x4_t (&acc)[8][
 #pragma unroll
     for (int fn = 0; fn < 8; ++fn) {
       float xr[4] = {acc[fm][fn][0], acc[fm][fn][1], acc[fm][fn][2], acc[fm][fn][3]};
-      round_pair<__bf16>(xr[0], xr[1]);
-      round_pair<__bf16>(xr[2], xr[3]);
+      round_pair(xr[0], xr[1]);
+      round_pair(xr[2], xr[3]);
       float o[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {

@@ -1,0 +1,58 @@
+"""fp32 kernels (128 x 128 tiles, K-split dX planes) at the sizes where a tile,
+a K stage, a vocabulary block or a dX slice ends, against the torch path in
+64 bits."""
+import pytest
+import torch
+
+from mini_trainer_amd import fused_linear_cross_entropy
+from mini_trainer_amd.flce import BACKWARD_BUDGET_ENV
+
+pytestmark = pytest.mark.gpu
+
+
+def _exact(X, W, y, grad, cap):
+    X, W = X.double().requires_grad_(True), W.double().requires_grad_(True)
+    z = X @ W.T
+    if cap:
+        z = cap * torch.tanh(z / cap)
+    loss = torch.nn.functional.cross_entropy(z, y, ignore_index=-100, reduction="none")
+    loss.backward(grad.double())
+    return loss.detach(), X.grad, W.grad
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("budget", [0, 1, 1 << 21, 1 << 28])
+@pytest.mark.parametrize("T,H,V,cap", [
+    (1, 4, 3, 0.0),          # one row, one K chunk
+    (127, 32, 129, 0.0),     # one K stage, one column into a second tile
+    (129, 36, 128, 0.0),     # a partial second K stage, one row into a second tile
+    (257, 132, 1283, 0.0),   # tails everywhere
+    (640, 128, 5000, 30.0),  # several blocks and dX slices, softcap
+    (1300, 260, 2052, 0.0),
+])
+def test_fp32_tiles_and_slices(gpu, monkeypatch, T, H, V, cap, budget):
+    """Bound: sums of at most K = max(H, V, T) terms, rounded to 24 bits at
+    every step, err like sqrt(K) 2^-24 of the result (random signs); an
+    exponent near 20 in log2 units carries 2^-24 of itself, about 20 ln 2
+    ulp of the exponential.  Four times their sum."""
+    if budget:
+        monkeypatch.setenv(BACKWARD_BUDGET_ENV, str(budget))
+    g = torch.Generator().manual_seed(T * 7 + V)
+    X = torch.randn(T, H, generator=g)
+    W = torch.randn(V, H, generator=g) * (1.3 / H ** 0.5)
+    y = torch.randint(0, V, (T,), generator=g)
+    if T > 1:
+        y[torch.rand(T, generator=g) < 0.2] = -100
+    grad = torch.rand(T, generator=g) + 0.5
+    Xd, Wd = X.to(gpu).requires_grad_(True), W.to(gpu).requires_grad_(True)
+    loss = fused_linear_cross_entropy(Xd, Wd, y.to(gpu), softcap=cap or None)
+    loss.backward(grad.to(gpu))
+    el, ex, ew = _exact(X.to(gpu), W.to(gpu), y.to(gpu), grad.to(gpu), cap)
+    bound = 4 * (max(H, V, T) ** 0.5 + 14) * 2.0 ** -24
+    assert _rel(loss.detach(), el) <= bound
+    assert _rel(Xd.grad, ex) <= bound and _rel(Wd.grad, ew) <= bound
+    masked = (y == -100).to(gpu)
+    assert torch.count_nonzero(loss[masked]) == 0 and torch.count_nonzero(Xd.grad[masked]) == 0
