@@ -110,7 +110,7 @@ MT_F32_KERNEL void fwd_f32_kernel(FwdArgs a) {
     }, ec.wn * 64);
     if constexpr (kKTail) B.set_tail(c_lim);
     f32x4_t acc[4][4];
-    mainloop_f32<kKTail>(lds, acc, A, B, KT, c_lim);
+    mainloop_f32<kKTail, false>(lds, acc, A, B, KT, c_lim);
     if (a.softcap > 0.f) fwd_tile_f32<true>(acc, m2, d, lbl, rglob, vrow0, ec, a);
     else fwd_tile_f32<false>(acc, m2, d, lbl, rglob, vrow0, ec, a);
   }
@@ -208,7 +208,7 @@ MT_F32_KERNEL void recompute_f32_kernel(RecompArgs a) {
     B.set_tail(c_lim);
   }
   f32x4_t acc[4][4];
-  mainloop_f32<kKTail>(lds, acc, A, B, KT, c_lim);
+  mainloop_f32<kKTail, false>(lds, acc, A, B, KT, c_lim);
   if (a.softcap > 0.f) recompute_epilogue_f32<true>(acc, a, ec, row0, vloc0);
   else recompute_epilogue_f32<false>(acc, a, ec, row0, vloc0);
 }
@@ -238,7 +238,7 @@ __device__ __forceinline__ void dx_f32_item(char* lds, const DxArgs& a, uint32_t
   B.init(a.W + (int64_t)k0 * a.ldw_b + (int64_t)h0 * 4, a.ldw_b, a.V - a.v0 - k0, a.H - h0,
          ec.wn * 64);
   f32x4_t acc[4][4];
-  mainloop_f32<false>(lds, acc, A, B, (kv + kBKF - 1) / kBKF);
+  mainloop_f32<false, true>(lds, acc, A, B, (kv + kBKF - 1) / kBKF);
   float* plane = a.accbuf + (int64_t)z * a.split_stride;
 #pragma unroll
   for (int fm = 0; fm < 4; ++fm) {
@@ -271,7 +271,7 @@ __device__ __forceinline__ void dw_f32_item(char* lds, const DwArgs& a, uint32_t
     return a.XcT + (int64_t)h * a.ldxt_b;
   }, ec.wn * 64);
   f32x4_t acc[4][4];
-  mainloop_f32<false>(lds, acc, A, B, (a.kt_rows + kBKF - 1) / kBKF);
+  mainloop_f32<false, true>(lds, acc, A, B, (a.kt_rows + kBKF - 1) / kBKF);
 #pragma unroll
   for (int fm = 0; fm < 4; ++fm) {
     const int32_t vl = m0 + ec.row_tr(fm);
