@@ -56,7 +56,7 @@
 extern "C" {
 #endif
 
-#define MT_FLCE_ABI_VERSION 7
+#define MT_FLCE_ABI_VERSION 8
 
 typedef struct ihipStream_t* mt_stream_t; /* == hipStream_t */
 
@@ -337,6 +337,61 @@ int mt_flce_backward_narrow(const void* X, const void* W, int64_t T, int64_t H,
  * or bad sizes).  No counterpart in the reference.
  */
 size_t mt_flce_narrow_scratch_bytes(int64_t V, int64_t H, int64_t chunk_rows);
+
+/*
+ * Training with the logits (or as many of their columns as fit) kept from the
+ * forward to the backward, bf16 only: the forward stores the bf16-rounded
+ * logits of vocabulary columns [0, keep_cols) of every counted row, the
+ * backward turns them into G in place and recomputes only the other columns,
+ * in blocks of keep_cols in the same buffer (6 H V n_valid flops in all when
+ * every column is kept).
+ *
+ * mt_flce_logits_plan writes keep_cols (a multiple of 256, at most
+ * round_up(V, 256)), the bytes of the logits buffer (round_up(n_valid, 256) x
+ * keep_cols bf16) and of the backward's scratch (X^T, the dW work queue, dX's
+ * fp32 accumulator or the planes of a dX split over the vocabulary), which fit
+ * budget_bytes (0 = 5% of T V 2) -- plus, with count_gradient != 0, the bytes
+ * (V H 2 and tile padding) by which a bf16 weight gradient is smaller than the
+ * fp32 one the other paths accumulate -- and *pays = 1 when every column is
+ * kept or a cost model expects this to beat the path that
+ * mt_flce_fused_plan's user would take under the same budget.  All 0 when
+ * nothing fits.
+ *
+ * mt_flce_forward_logits is mt_flce_forward (same loss and lse, bit for bit)
+ * that also writes the logits.  mt_flce_backward_logits consumes them (they
+ * hold G afterwards, so it runs once per forward): dX [T, H] bf16, zero at
+ * ignored rows, and the weight gradient as contiguous bf16 rows [V, H] at
+ * dW_out (V H 2 bytes), narrowed once from fp32 sums over all counted rows;
+ * grad_loss and grad_stride as in mt_flce_backward; one scalar (stride 0) is
+ * applied to the fp32 sums, a per-token gradient is part of G.  A scratch
+ * smaller than planned (but with X^T, the queue and, for keep_cols < V, the
+ * accumulator) means fewer dX slices.  n_valid >= 1, H a multiple of 8.
+ * Replaces the same reference interface as mt_flce_forward and
+ * mt_flce_backward (none_reduction_losses.py:16-23, whose Liger forward keeps
+ * each chunk's logits to form the gradients from).
+ */
+int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V,
+                        int dtype, size_t budget_bytes, int count_gradient,
+                        int64_t* keep_cols, size_t* logits_bytes,
+                        size_t* scratch_bytes, int* pays);
+int mt_flce_forward_logits(const void* X, const void* W, int64_t T, int64_t H,
+                           int64_t V, int64_t ldx, int64_t ldw, int dtype,
+                           float softcap, const int32_t* row_index,
+                           const int32_t* row_label, int64_t n_valid,
+                           float* loss, float* lse, void* workspace,
+                           size_t workspace_bytes, void* logits,
+                           int64_t keep_cols, size_t logits_bytes,
+                           mt_stream_t stream);
+int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H,
+                            int64_t V, int64_t ldx, int64_t ldw, int dtype,
+                            float softcap, const int32_t* row_index,
+                            const int32_t* row_label, int64_t n_valid,
+                            const float* lse, const float* grad_loss,
+                            int64_t grad_stride, void* dX, int64_t lddx,
+                            void* dW_out, size_t dw_out_bytes, void* logits,
+                            int64_t keep_cols, size_t logits_bytes,
+                            void* scratch, size_t scratch_bytes,
+                            mt_stream_t stream);
 
 /*
  * Layout of the tiled fp32 weight gradient that mt_flce_fused_tiles and

@@ -200,6 +200,7 @@ inline uint32_t persistent_grid(int64_t tiles) {
   return (uint32_t)std::min(tiles, cap > 0 ? std::min(cap, device_cus()) : device_cus());
 }
 inline int64_t round_up(int64_t a, int64_t b) { return cdiv(a, b) * b; }
+inline int64_t vocab_pad(int64_t V) { return round_up(V, 256); }
 
 // Grid of a bf16 logits launch over a.tiles_m x a.vt_total tiles whose
 // vocabulary block has `vn` rows: persistent over the full tile columns (the
@@ -302,6 +303,7 @@ struct DxReduce {
   int64_t stride = 0, ld = 0;
   int32_t nsplit = 1, cn = 0, H = 0;
   const float* scale = nullptr;
+  int64_t scale_stride = 1;
   const int32_t* row_index = nullptr;
   char* dX = nullptr;
   int64_t lddx_b = 0;
@@ -309,7 +311,7 @@ struct DxReduce {
 inline void launch_dx_reduce(const DxReduce& r, hipStream_t stream) {
   hipLaunchKernelGGL(dx_split_reduce_kernel, dim3((uint32_t)cdiv(r.H, 1024), (uint32_t)r.cn),
                      dim3(256), 0, stream, r.part, r.stride, r.nsplit, r.ld, r.cn, r.H, r.scale,
-                     r.row_index, r.dX, r.lddx_b);
+                     r.scale_stride, r.row_index, r.dX, r.lddx_b);
 }
 
 // dX and dW of one block side by side: dX (tiles_m x tiles_n workgroups,
@@ -653,7 +655,7 @@ int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t 
                    int64_t ldw, float softcap, const int32_t* row_index, const int32_t* row_label,
                    int64_t n_valid, float* loss, float* lse, const FwdPlan& p, char* ws,
                    hipStream_t stream, char* keep = nullptr, int64_t keep_cols = 0,
-                   int32_t* guard = nullptr) {
+                   int32_t* guard = nullptr, char* logits = nullptr) {
   constexpr int es = sizeof(T);
   FwdArgs a;
   a.X = static_cast<const char*>(X);
@@ -693,21 +695,34 @@ int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t 
     // raises for a row whose largest logit leaves [kGuardLo, kGuardHi]
     static void (*const kerns_keep[2])(FwdArgs) = {fwd_bf16_kernel<false, kStoreExp, false, false>,
                                                    fwd_bf16_kernel<false, kStoreExp, false, true>};
+    // logits: columns [0, keep_cols) first, storing their bf16-rounded logits
+    // as rows of keep_cols entries
+    static void (*const kerns_s[2][2][2])(FwdArgs) = {
+        {{fwd_bf16_kernel<false, kStoreLogits, false, false>,
+          fwd_bf16_kernel<false, kStoreLogits, false, true>},
+         {fwd_bf16_kernel<false, kStoreLogits, true, false>,
+          fwd_bf16_kernel<false, kStoreLogits, true, true>}},
+        {{fwd_bf16_kernel<true, kStoreLogits, false, false>,
+          fwd_bf16_kernel<true, kStoreLogits, false, true>},
+         {fwd_bf16_kernel<true, kStoreLogits, true, false>,
+          fwd_bf16_kernel<true, kStoreLogits, true, true>}}};
     const int64_t vb = vocab_block_rows(V, ldw);
     for (int64_t v0 = 0; v0 < V;) {
-      const bool kb = keep && v0 == 0;
-      const int64_t vn = kb ? keep_cols : std::min(vb, V - v0);
+      const bool kb = keep && v0 == 0, lb = logits && v0 == 0;
+      const int64_t vn = kb ? keep_cols : (lb ? std::min(keep_cols, V) : std::min(vb, V - v0));
       a.W = static_cast<const char*>(W) + v0 * ldw * es;
       a.V = (int32_t)vn;
       a.vcol0 = (int32_t)v0;
       a.w_range = range_of(vn, ldw * es);
       a.vt_total = (int32_t)cdiv(vn, geometry(es).tile);
-      a.S = kb ? keep : nullptr;
-      a.lds_b = kb ? keep_cols * 2 : 0;
-      a.s_range = kb ? range_of(p.tiles_m * 256, keep_cols * 2) : 0;
+      a.S = kb ? keep : (lb ? logits : nullptr);
+      a.lds_b = a.S ? keep_cols * 2 : 0;
+      a.s_range = a.S ? range_of(p.tiles_m * 256, keep_cols * 2) : 0;
       a.guard_reset = kb ? guard : nullptr;
-      void (*kern)(FwdArgs) = kb ? kerns_keep[ktail] : kerns[softcap > 0.f][vn % 256 != 0][ktail];
-      const int pf = prof_begin(kb ? "fwd_bf16_kernel<keep>" : "fwd_bf16_kernel",
+      void (*kern)(FwdArgs) = kb ? kerns_keep[ktail]
+                                 : (lb ? kerns_s : kerns)[softcap > 0.f][vn % 256 != 0][ktail];
+      const int pf = prof_begin(kb ? "fwd_bf16_kernel<keep>"
+                                   : (lb ? "fwd_bf16_kernel<store_logits>" : "fwd_bf16_kernel"),
                                 2.0 * H * (double)vn * n_valid, 0, stream);
       hipLaunchKernelGGL(kern, dim3(fwd_grid(a, vn)), dim3(kThreadsBf), 0, stream, a);
       prof_end(pf, stream);
@@ -779,6 +794,23 @@ int zero_tiles(const TiledDw& td, int64_t V, int64_t H, hipStream_t s) {
     MT_TRY(check_launch("zero_matrix_f32_kernel"));
   }
   return MT_OK;
+}
+
+// One vocabulary block's recompute.  (A kept block's launch, run_if set,
+// recomputes only if the guard was raised: recorded apart, without flops, so
+// as not to inflate the rate.)
+int launch_recompute_bf16(const RecompArgs& r, hipStream_t stream) {
+  static void (*const kerns[2][2][2])(RecompArgs) = {
+      {{recompute_bf16_kernel<false, false, false>, recompute_bf16_kernel<false, false, true>},
+       {recompute_bf16_kernel<false, true, false>, recompute_bf16_kernel<false, true, true>}},
+      {{recompute_bf16_kernel<true, false, false>, recompute_bf16_kernel<true, false, true>},
+       {recompute_bf16_kernel<true, true, false>, recompute_bf16_kernel<true, true, true>}}};
+  const int pr = r.run_if ? prof_begin("recompute_bf16_kernel<if_guard>", 0.0, 0, stream)
+                          : prof_begin("recompute_bf16_kernel", 2.0 * r.H * (double)r.Cn * r.cv, 0, stream);
+  hipLaunchKernelGGL(kerns[r.softcap > 0.f][r.cv % 256 != 0][r.H % kBKBf != 0],
+                     dim3(persistent_grid((int64_t)r.tiles_m * r.tiles_n)), dim3(kThreadsBf), 0, stream, r);
+  prof_end(pr, stream);
+  return check_launch("recompute_kernel");
 }
 
 int launch_backward_bf16(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V, int64_t ldx,
@@ -854,20 +886,7 @@ int launch_backward_bf16(const void* X, const void* W, int64_t Tn, int64_t H, in
         MT_TRY(check_launch("exp_to_grad_kernel"));
         r.run_if = kept_guard;
       }
-      static void (*const kerns[2][2][2])(RecompArgs) = {
-          {{recompute_bf16_kernel<false, false, false>, recompute_bf16_kernel<false, false, true>},
-           {recompute_bf16_kernel<false, true, false>, recompute_bf16_kernel<false, true, true>}},
-          {{recompute_bf16_kernel<true, false, false>, recompute_bf16_kernel<true, false, true>},
-           {recompute_bf16_kernel<true, true, false>, recompute_bf16_kernel<true, true, true>}}};
-      // (a kept block's launch recomputes only if the guard was raised:
-      // recorded apart, without flops, so as not to inflate the rate)
-      const int pr = kept ? prof_begin("recompute_bf16_kernel<if_guard>", 0.0, 0, stream)
-                          : prof_begin("recompute_bf16_kernel", 2.0 * H * (double)cn * cv, 0, stream);
-      hipLaunchKernelGGL(kerns[softcap > 0.f][cv % 256 != 0][H % kBKBf != 0],
-                         dim3(persistent_grid(r.tiles_m * r.tiles_n)),
-                         dim3(kThreadsBf), 0, stream, r);
-      prof_end(pr, stream);
-      MT_TRY(check_launch("recompute_kernel"));
+      MT_TRY(launch_recompute_bf16(r, stream));
 
       DxArgs x;
       x.G = G;
@@ -1146,8 +1165,6 @@ struct FusedPlan {
   size_t ws = 0;
 };
 
-inline int64_t vocab_pad(int64_t V) { return round_up(V, 256); }
-
 // K slices of a fused chunk's dX: dX has only cdiv(C, 256) x cdiv(H, 256)
 // tiles, each contracting the whole vocabulary; with fewer tiles than half
 // the CUs, dX alone would outlast dW beside it, so each tile is split over
@@ -1395,6 +1412,240 @@ int launch_fused(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V,
       w.queue = queue;
     // S and XcT are rewritten by the next chunk only after the join
     MT_TRY(launch_dx_dw_bf16(x, w, stream, nsplit > 1 ? &red : nullptr));
+  }
+  return MT_OK;
+}
+
+// ----------------------------------------------------------- kept logits
+// Forward that keeps the bf16-rounded logits of vocabulary columns [0, cols) of
+// every valid row, backward of one row block that turns them into G in place
+// (softmax_grad_kernel) and recomputes only the other columns, in blocks of
+// at most `cols`, into the same buffer.  Each dW tile is written once in bf16,
+// any per-token upstream gradient is exact, and nothing is lost by storing
+// the logits (they are bf16 values).  With every column kept that is 6 H V N
+// flops against the general path's 8.  The 5% budget alone holds few columns,
+// but a bf16 weight gradient leaves V H 2 bytes of the fp32 one that the
+// budget counts as an output (the narrowing backward puts its scratch there):
+// with them every column fits up to about H counted tokens.
+struct KeptPlan {
+  int64_t cols = 0;  // 0: does not fit, or cannot run
+  size_t logits = 0, scratch = 0;
+  DxSplit split;
+  double cost = 1e300;  // modelled seconds, forward and backward
+};
+
+// dX is split over a block's columns into split.S slices with an fp32 plane
+// [C, H] each (as the fused path's, but kept over the blocks and summed at the
+// end); with one slice and several blocks its accumulator is tiled.
+size_t kept_scratch(int64_t C, int64_t H, int64_t S, bool blocks) {
+  return align_up((size_t)H * C * 2) + align_up((kQueueWords + 1) * sizeof(uint32_t)) +
+         (S > 1 ? align_up((size_t)S * C * H * sizeof(float)) : (blocks ? align_up(tiled_acc_bytes(C, H)) : 0));
+}
+
+double kept_cost(int64_t N, int64_t H, int64_t V, int64_t cols, const DxSplit& d) {
+  const int64_t tm = cdiv(N, 256), th = cdiv(H, 256), nb = cdiv(V, cols);
+  double t = forward_cost(N, H, V) + (nb > 1 ? kLaunch : 0);
+  t += 4.0 * N * std::min(cols, V) / kBw;  // logits read, G written
+  for (int64_t v0 = 0; v0 < V; v0 += cols) {
+    const int64_t cv = std::min(cols, V - v0), tv = cdiv(cv, 256);
+    if (v0 > 0) t += gemm_time(tm * tv, H);
+    // (few columns: one dW tile over all rows can be the longest item)
+    t += std::max(phase_time(tm * th * d.S, cdiv(cv, d.S), tv * th, N, 0), tile_time(N) + 2 * kLaunch);
+  }
+  // dX planes (or the accumulator) stored, re-read and added to, then summed
+  const double plane = (double)N * H * 4;
+  if (d.S > 1 || nb > 1) t += plane * d.S * (2.0 * nb - 1.0) * 0.5 / kBw;
+  return t + 3 * kLaunch;
+}
+
+// dX's slices of a block of `cols` columns for S wanted ones: whole 64-entry
+// K stages, none empty in that (largest) block.
+DxSplit kept_split(int64_t cols, int64_t V, int64_t S) {
+  DxSplit d;
+  if (S <= 1) return d;
+  const int64_t k = std::min(cols, V);
+  d.kslice = round_up(cdiv(k, S), 64);
+  d.S = cdiv(k, d.kslice);
+  if (d.S <= 1) d = DxSplit();
+  return d;
+}
+
+// room: count in the bytes a bf16 gradient leaves of an fp32 one.  For every
+// number of dX slices (powers of two: with S a multiple of 8, or dividing 8,
+// slices keep to XCDs of their own, see fused_split) the columns that fit, and of
+// these the cheapest.  Too few slices and dX, whose tiles contract a whole
+// block, outlasts dW beside it; a plane costs 2 H columns.
+KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bool room) {
+  KeptPlan best;
+  if (N <= 0 || H % 8 != 0) return best;
+  if (budget == 0) budget = (size_t)((double)T * V * 2 * 0.05);
+  const int64_t C = round_up(N, 256), Vp = vocab_pad(V);
+  const uint64_t lim = buffer_limit();
+  if ((uint64_t)H * C * 2 > lim) return best;
+  const size_t have = budget + (room ? dw_tiles_bytes(V, H) - dw_lo_bytes(V, H) : 0);
+  const size_t fwd = forward_ws(plan_forward(N, V, 2), N);
+  // columns one buffer reaches: of the logits, and of the weight's rows
+  const int64_t reach = (int64_t)(std::min(lim / ((uint64_t)C * 2), lim / ((uint64_t)H * 2)) / 256 * 256);
+  for (int64_t S = 1; S <= 32; S *= 2) {
+    for (int blocks = 0; blocks < 2; ++blocks) {
+      const size_t other = std::max(kept_scratch(C, H, S, blocks != 0), fwd);
+      if (other > have) continue;
+      int64_t cols = std::min<int64_t>((int64_t)((have - other) / ((size_t)C * 2)) / 256 * 256, reach);
+      if (blocks == 0 && cols < Vp) continue;  // several blocks
+      cols = std::min(cols, blocks ? Vp - 256 : Vp);
+      if (cols < 256 || (S > 1 && std::min(cols, V) / S < 256)) continue;
+      const DxSplit d = kept_split(cols, V, S);
+      if (d.S != S && S > 1) continue;
+      const double t = kept_cost(N, H, V, cols, d);
+      if (t < best.cost) {
+        best.cols = cols;
+        best.logits = align_up((size_t)C * cols * 2);
+        best.scratch = kept_scratch(C, H, d.S, cols < V);
+        best.split = d;
+        best.cost = t;
+      }
+    }
+  }
+  return best;
+}
+
+// The most slices (a power of two) whose planes fit a scratch of `bytes`.
+int64_t kept_slices_in(int64_t C, int64_t H, bool blocks, size_t bytes) {
+  int64_t S = 32;
+  while (S > 1 && kept_scratch(C, H, S, blocks) > bytes) S /= 2;
+  return S;
+}
+
+int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V, int64_t ldx,
+                           int64_t ldw, float softcap, const int32_t* row_index,
+                           const int32_t* row_label, int64_t N, const float* lse, const float* grad,
+                           int64_t gstride, void* dX, int64_t lddx, void* dW, char* logits, int64_t cols,
+                           char* scratch, size_t scratch_bytes, hipStream_t stream) {
+  const int64_t C = round_up(N, 256), nb = cdiv(V, cols);
+  const int64_t ldg_b = cols * 2, ldxt_b = C * 2;
+  const DxSplit split = kept_split(cols, V, kept_slices_in(C, H, nb > 1, scratch_bytes));
+  char* XcT = scratch;
+  uint32_t* queue = reinterpret_cast<uint32_t*>(scratch + align_up((size_t)H * C * 2));
+  float* one = reinterpret_cast<float*>(queue + kQueueWords);
+  float* planes = reinterpret_cast<float*>(reinterpret_cast<char*>(queue) +
+                                           align_up((kQueueWords + 1) * sizeof(uint32_t)));
+  // one upstream scalar for every token: G is formed for a unit gradient and
+  // the scalar applied to the fp32 sums of dX and dW, so that its own rounding
+  // to bf16 does not enter G; a per-token gradient is part of G
+  const float* out_scale = gstride == 0 ? grad : nullptr;
+  const float* g = gstride == 0 ? one : grad;
+  hipLaunchKernelGGL(gather_t_kernel<__bf16>, dim3((uint32_t)(C / 64), (uint32_t)cdiv(H, 64)),
+                     dim3(256), 0, stream, static_cast<const char*>(X), ldx * 2, row_index, (int32_t)N,
+                     (int32_t)H, XcT, ldxt_b, static_cast<const float*>(nullptr), queue,
+                     (int32_t)kQueueWords, one);
+  MT_TRY(check_launch("gather_t_kernel"));
+  for (int64_t v0 = 0, j = 0; v0 < V; v0 += cols, ++j) {
+    const int64_t cv = std::min(cols, V - v0);
+    const char* Wv = static_cast<const char*>(W) + v0 * ldw * 2;
+    const uint32_t g_range = range_of(C, ldg_b), w_range = range_of(cv, ldw * 2);
+    if (j == 0) {
+      const int ps = prof_begin("softmax_grad_kernel", 0, 2.0 * C * cols * 2, stream);
+      hipLaunchKernelGGL(softcap > 0.f ? softmax_grad_kernel<true> : softmax_grad_kernel<false>,
+                         dim3((uint32_t)C), dim3(256), 0, stream, logits, ldg_b, (int32_t)cols,
+                         (int32_t)N, (int32_t)cv, lse, g, gstride, row_index, row_label, softcap,
+                         static_cast<const int32_t*>(nullptr));
+      prof_end(ps, stream);
+      MT_TRY(check_launch("softmax_grad_kernel"));
+    } else {
+      RecompArgs r;
+      r.X = static_cast<const char*>(X);
+      r.W = Wv;
+      r.ldx_b = ldx * 2;
+      r.ldw_b = ldw * 2;
+      r.H = (int32_t)H;
+      r.V = (int32_t)V;
+      r.x_range = range_of(Tn, ldx * 2);
+      r.w_range = w_range;
+      r.g_range = g_range;
+      r.row_index = row_index;
+      r.row_label = row_label;
+      r.lse = lse;
+      r.Cn = (int32_t)N;
+      r.grad = g;
+      r.gstride = gstride;
+      r.softcap = softcap;
+      r.v0 = (int32_t)v0;
+      r.cv = (int32_t)cv;
+      r.G = logits;
+      r.ldg_b = ldg_b;
+      r.tiles_m = (int32_t)cdiv(N, 256);
+      r.tiles_n = (int32_t)cdiv(cv, 256);
+      r.zero_words = queue;
+      MT_TRY(launch_recompute_bf16(r, stream));
+    }
+    DxArgs x;
+    x.G = logits;
+    x.ldg_b = ldg_b;
+    x.W = Wv;
+    x.ldw_b = ldw * 2;
+    x.g_range = g_range;
+    x.w_range = w_range;
+    x.V = (int32_t)(v0 + cv);  // K rows past the block's end repeat its last row (times zero G)
+    x.v0 = (int32_t)v0;
+    x.kv = (int32_t)cv;
+    x.H = (int32_t)H;
+    x.Cn = (int32_t)N;
+    x.accbuf = planes;
+    x.ld_acc = H;
+    if (split.S > 1) {
+      x.mode = j == 0 ? kDxStore : kDxAdd;
+      x.nsplit = (int32_t)split.S;
+      x.kslice = (int32_t)round_up(cdiv(cv, split.S), 64);
+      x.split_stride = C * H;
+    } else {
+      x.mode = nb == 1 ? kDxEmit
+                       : kDxTiledAcc + (j == 0 ? kDxStore : (j == nb - 1 ? kDxAddEmit : kDxAdd));
+    }
+    x.out_scale = out_scale;
+    x.dX = static_cast<char*>(dX);
+    x.lddx_b = lddx * 2;
+    x.row_index = row_index;
+    x.tiles_m = (int32_t)(C / 256);
+    x.tiles_n = (int32_t)cdiv(H, 256);
+    DxReduce red;
+    const bool last = split.S > 1 && j == nb - 1;
+    if (last) {
+      red.part = planes;
+      red.stride = C * H;
+      red.ld = H;
+      red.nsplit = (int32_t)split.S;
+      red.cn = (int32_t)N;
+      red.H = (int32_t)H;
+      red.scale = out_scale;
+      red.scale_stride = 0;
+      red.row_index = row_index;
+      red.dX = static_cast<char*>(dX);
+      red.lddx_b = lddx * 2;
+    }
+    DwArgs w;
+    w.G = logits;
+    w.ldg_b = ldg_b;
+    w.g_rows = (int32_t)C;
+    w.g_cols = (int32_t)cols;
+    w.XcT = XcT;
+    w.ldxt_b = ldxt_b;
+    w.g_range = g_range;
+    w.xt_range = range_of(H, ldxt_b);
+    w.kt_rows = (int32_t)N;
+    w.H = (int32_t)H;
+    w.cv = (int32_t)cv;
+    w.v0 = (int32_t)v0;
+    w.dW = static_cast<float*>(dW);
+    w.lddw = H;
+    w.accumulate = 0;
+    w.narrow = 1;
+    w.out_scale = out_scale;
+    w.tiles_m = (int32_t)cdiv(cv, 256);
+    w.tiles_n = x.tiles_n;
+    if ((int64_t)w.tiles_m * w.tiles_n >= 4 * device_cus() && device_cus() % kQueueWords == 0 && N > kBKBf)
+      w.queue = queue;
+    // the next block's recompute (G) follows the join
+    MT_TRY(launch_dx_dw_bf16(x, w, stream, last ? &red : nullptr));
   }
   return MT_OK;
 }
@@ -1841,6 +2092,131 @@ int mt_flce_backward_narrow(const void* X, const void* W, int64_t T, int64_t H, 
                         grad_loss, grad_stride, dX, lddx, static_cast<float*>(dW_out), 0, 0,
                         kDwNarrow, chunk_rows, chunk_vocab, workspace, workspace_bytes, stream,
                         kept_guard, nullptr, scratch, scratch_bytes);
+}
+
+int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,
+                        size_t budget_bytes, int count_gradient, int64_t* keep_cols,
+                        size_t* logits_bytes, size_t* scratch_bytes, int* pays) {
+  if (dtype != MT_DTYPE_BF16)
+    return fail(MT_ERR_UNSUPPORTED, "keeping logits is bf16 only (dtype %d)", dtype);
+  if (T < 0 || n_valid < 0 || n_valid > T || H <= 0 || V <= 0 || T > INT32_MAX || H > INT32_MAX ||
+      V > INT32_MAX)
+    return fail(MT_ERR_INVALID_ARGUMENT, "bad sizes T=%lld n_valid=%lld H=%lld V=%lld", (long long)T,
+                (long long)n_valid, (long long)H, (long long)V);
+  if (!keep_cols || !logits_bytes || !scratch_bytes || !pays)
+    return fail(MT_ERR_INVALID_ARGUMENT, "null output pointer");
+  const KeptPlan p = plan_kept(T, n_valid, H, V, budget_bytes, count_gradient != 0);
+  *keep_cols = p.cols;
+  *logits_bytes = p.logits;
+  *scratch_bytes = p.scratch;
+  *pays = 0;
+  if (p.cols > 0) {
+    const FusedPlan f = plan_fused(T, n_valid, H, V, budget_bytes);
+    // (the dearer estimate last: it searches the general path's blockings)
+    *pays = p.cols >= V ||
+            ((!f.C || p.cost < 0.97 * (fused_cost(n_valid, H, V, f.C) + (double)V * H * 6 / kBw)) &&
+             p.cost < 0.97 * general_cost(T, n_valid, H, V, budget_bytes, true));
+  }
+  return MT_OK;
+}
+
+}  // extern "C"
+
+namespace {
+
+// Checks shared by the two entries that take kept logits.
+int logits_args(int64_t n_valid, int64_t H, int64_t V, int64_t ldw, const void* logits,
+                int64_t keep_cols, size_t logits_bytes) {
+  if (keep_cols <= 0 || keep_cols % 256 != 0 || keep_cols > vocab_pad(V))
+    return fail(MT_ERR_INVALID_ARGUMENT,
+                "keep_cols=%lld must be a positive multiple of 256, at most V=%lld rounded up",
+                (long long)keep_cols, (long long)V);
+  const int64_t C = round_up(n_valid, 256);
+  const uint64_t need = (uint64_t)C * keep_cols * 2;
+  if (need > buffer_limit() || (uint64_t)H * C * 2 > buffer_limit() ||
+      (uint64_t)std::min(keep_cols, V) * ldw * 2 > buffer_limit())
+    return fail(MT_ERR_UNSUPPORTED, "kept logits, X^T or the block's weight rows beyond one buffer's reach");
+  if (!logits || logits_bytes < need || reinterpret_cast<uintptr_t>(logits) % 16 != 0)
+    return fail(MT_ERR_INVALID_ARGUMENT,
+                "logits need %llu bytes (round_up(n_valid, 256) x keep_cols bf16, 16-byte aligned), "
+                "got %zu", (unsigned long long)need, logits_bytes);
+  return MT_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int mt_flce_forward_logits(const void* X, const void* W, int64_t T, int64_t H, int64_t V,
+                           int64_t ldx, int64_t ldw, int dtype, float softcap,
+                           const int32_t* row_index, const int32_t* row_label, int64_t n_valid,
+                           float* loss, float* lse, void* workspace, size_t workspace_bytes,
+                           void* logits, int64_t keep_cols, size_t logits_bytes, mt_stream_t stream) {
+  if (dtype != MT_DTYPE_BF16)
+    return fail(MT_ERR_UNSUPPORTED, "keeping logits is bf16 only (dtype %d)", dtype);
+  MT_TRY(check_common(X, W, T, H, V, ldx, ldw, dtype, softcap));
+  if (n_valid < 0 || n_valid > T)
+    return fail(MT_ERR_INVALID_ARGUMENT, "n_valid=%lld outside [0, T=%lld]", (long long)n_valid, (long long)T);
+  if (T == 0) return MT_OK;
+  if (!row_index || !loss || (n_valid > 0 && (!row_label || !lse)))
+    return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
+  const FwdPlan p = plan_forward(n_valid, V, 2);
+  const size_t need = n_valid > 0 ? forward_ws(p, n_valid) : 0;
+  if (workspace_bytes < need || (need && !workspace))
+    return fail(MT_ERR_WORKSPACE_TOO_SMALL, "forward workspace %zu bytes < required %zu",
+                workspace_bytes, need);
+  if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+    return fail(MT_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
+  if (n_valid > 0) MT_TRY(logits_args(n_valid, H, V, ldw, logits, keep_cols, logits_bytes));
+  hipStream_t s = (hipStream_t)stream;
+  if (T - n_valid > 0) {
+    const int64_t n0 = T - n_valid;
+    hipLaunchKernelGGL(zero_scatter_f32_kernel, dim3((uint32_t)std::min<int64_t>(cdiv(n0, 256), 4096)),
+                       dim3(256), 0, s, loss, row_index + n_valid, n0);
+    MT_TRY(check_launch("zero_scatter_f32_kernel"));
+  }
+  if (n_valid == 0) return MT_OK;
+  return launch_forward<__bf16>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid,
+                                loss, lse, p, static_cast<char*>(workspace), s, nullptr, keep_cols,
+                                nullptr, static_cast<char*>(logits));
+}
+
+int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, int64_t V,
+                            int64_t ldx, int64_t ldw, int dtype, float softcap,
+                            const int32_t* row_index, const int32_t* row_label, int64_t n_valid,
+                            const float* lse, const float* grad_loss, int64_t grad_stride, void* dX,
+                            int64_t lddx, void* dW_out, size_t dw_out_bytes, void* logits,
+                            int64_t keep_cols, size_t logits_bytes, void* scratch,
+                            size_t scratch_bytes, mt_stream_t stream) {
+  if (dtype != MT_DTYPE_BF16)
+    return fail(MT_ERR_UNSUPPORTED, "keeping logits is bf16 only (dtype %d)", dtype);
+  MT_TRY(check_common(X, W, T, H, V, ldx, ldw, dtype, softcap));
+  if (n_valid <= 0 || n_valid > T)
+    return fail(MT_ERR_INVALID_ARGUMENT, "n_valid=%lld outside [1, T=%lld]", (long long)n_valid, (long long)T);
+  if (lddx < H || (lddx * 2) % 16 != 0)
+    return fail(MT_ERR_INVALID_ARGUMENT, "lddx=%lld must be >= H and a whole number of 16-byte chunks",
+                (long long)lddx);
+  if (grad_stride < 0) return fail(MT_ERR_INVALID_ARGUMENT, "grad_stride must be >= 0");
+  if (!dW_out || dw_out_bytes < dw_lo_bytes(V, H))
+    return fail(MT_ERR_INVALID_ARGUMENT, "dW_out %zu bytes < V H 2 = %zu", dw_out_bytes, dw_lo_bytes(V, H));
+  if (!dX || !row_index || !row_label || !lse || !grad_loss)
+    return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if ((reinterpret_cast<uintptr_t>(dX) | reinterpret_cast<uintptr_t>(dW_out) |
+       reinterpret_cast<uintptr_t>(scratch)) % 16 != 0)
+    return fail(MT_ERR_INVALID_ARGUMENT, "dX, dW_out and scratch must be 16-byte aligned");
+  MT_TRY(logits_args(n_valid, H, V, ldw, logits, keep_cols, logits_bytes));
+  const size_t need = kept_scratch(round_up(n_valid, 256), H, 1, keep_cols < V);
+  if (!scratch || scratch_bytes < need)
+    return fail(MT_ERR_WORKSPACE_TOO_SMALL, "logits scratch %zu bytes < required %zu", scratch_bytes, need);
+  hipStream_t s = (hipStream_t)stream;
+  if (T - n_valid > 0) {
+    hipLaunchKernelGGL(zero_rows_kernel, dim3((uint32_t)std::min<int64_t>(T - n_valid, 8192)), dim3(256),
+                       0, s, static_cast<char*>(dX), lddx * 2, row_index + n_valid, T - n_valid, H * 2);
+    MT_TRY(check_launch("zero_rows_kernel"));
+  }
+  return launch_backward_logits(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
+                                grad_loss, grad_stride, dX, lddx, dW_out, static_cast<char*>(logits),
+                                keep_cols, static_cast<char*>(scratch), scratch_bytes, s);
 }
 
 int mt_flce_fused_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,

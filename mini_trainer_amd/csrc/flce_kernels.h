@@ -284,6 +284,9 @@ struct DxArgs {
   // tiles_m * tiles_n * nsplit (dx_split_reduce_kernel sums the slices)
   int32_t nsplit = 1, kslice = 0;
   int64_t split_stride = 0;
+  // non-null (bf16 kDxEmit without row_scale, kDxTiledAcc + kDxAddEmit): every
+  // dX row times *out_scale
+  const float* out_scale = nullptr;
   // dX beside a work-queue dW in one launch (dx_dw_bf16_kernel), XCD-
   // partitioned: xcds > 0 gives dX whole XCDs -- workgroup b (on XCD b % 8)
   // takes logical tile (b % 8) per_xcd + b / 8 when b % 8 < xcds and
@@ -293,12 +296,13 @@ struct DxArgs {
   int32_t xcds = 0, per_xcd = 0;
 };
 
-// dX of a K-split fused chunk: row t < cn, columns h .. h + 3 of the sum of
-// the nsplit fp32 slices (in slice order), times scale[t], to bf16 at dX row
-// row_index[t].  One thread per 4 columns.
+// dX of a K-split chunk: row t < cn, columns h .. h + 3 of the sum of the
+// nsplit fp32 slices (in slice order), times scale[t * scale_stride] (null: 1),
+// to bf16 at dX row row_index[t].  One thread per 4 columns.
 __global__ __launch_bounds__(256) void dx_split_reduce_kernel(const float* part, int64_t stride,
                                                               int32_t nsplit, int64_t ld, int32_t cn,
                                                               int32_t H, const float* scale,
+                                                              int64_t scale_stride,
                                                               const int32_t* row_index, char* dX,
                                                               int64_t lddx_b) {
   const int32_t t = (int32_t)blockIdx.y;
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(256) void dx_split_reduce_kernel(const float* part,
   const float* p = part + (int64_t)t * ld + h;
   f32x4_t v = *reinterpret_cast<const f32x4_t*>(p);
   for (int32_t z = 1; z < nsplit; ++z) v += *reinterpret_cast<const f32x4_t*>(p + z * stride);
-  v *= scale[t];
+  if (scale) v *= scale[t * scale_stride];
   u32x2_t o;
   o[0] = pack_bf16x2(v[0], v[1]);
   o[1] = pack_bf16x2(v[2], v[3]);
@@ -346,8 +350,10 @@ struct DwArgs {
   float* dW_hi = nullptr;
   int32_t lo_rows = 0;
   // narrow (bf16, a dW every tile completes in one pass): dW is bf16 rows of
-  // pitch lddw elements, each tile narrowed in its epilogue (kDwNarrow)
+  // pitch lddw elements, each tile narrowed in its epilogue (kDwNarrow), times
+  // *out_scale when that is non-null
   int32_t narrow = 0;
+  const float* out_scale = nullptr;
 };
 
 // Where a bf16 dW kernel puts its tiles (template argument kOut): fp32 rows
@@ -364,12 +370,19 @@ constexpr int kDwRows = 0, kDwTiles = 1, kDwNarrow = 2;
 // 64 x 64 element tiles; 16-byte loads along h, 16-byte stores along t.
 // scale (non-null, bf16 only): row t is multiplied by scale[t] in fp32 and
 // rounded to bf16 (the fused path's per-row factor of G, see
-// fused_row_scale_kernel).
+// fused_row_scale_kernel).  zero_words[0 .. n_zero) are cleared (the work
+// queue of a later launch) and *one, where given, set to 1.
 template <typename T>
 __global__ __launch_bounds__(256) void gather_t_kernel(const char* X, int64_t ldx_b,
                                                        const int32_t* row_index, int32_t Cn,
                                                        int32_t H, char* XcT, int64_t ldxt_b,
-                                                       const float* scale = nullptr) {
+                                                       const float* scale = nullptr,
+                                                       uint32_t* zero_words = nullptr,
+                                                       int32_t n_zero = 0, float* one = nullptr) {
+  if (blockIdx.x == 0 && blockIdx.y == 0) {
+    if ((int32_t)threadIdx.x < n_zero) zero_words[threadIdx.x] = 0u;
+    if (one && threadIdx.x == 0) *one = 1.f;
+  }
   constexpr int E = sizeof(T);
   constexpr int PER = 16 / E;  // elements per 16-byte vector
   __shared__ T tile[64][64 + 1];

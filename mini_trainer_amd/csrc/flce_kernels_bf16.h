@@ -541,6 +541,7 @@ __device__ __forceinline__ void dx_epilogue_tiled_acc(const f32x4_t (&acc)[8][8]
                                                       int32_t h0) {
   constexpr int kM = kMode - kDxTiledAcc;
   const int64_t tile = (int64_t)(row0 / 256) * a.tiles_n + h0 / 256;
+  const float sc = kM == kDxAddEmit && a.out_scale ? *a.out_scale : 1.f;
   float* const base =
       a.accbuf + tile * 65536 + (int64_t)((ec.wm * 2u + ec.wn) * 16384u + ec.lane * 4u);
 #pragma unroll
@@ -562,6 +563,7 @@ __device__ __forceinline__ void dx_epilogue_tiled_acc(const f32x4_t (&acc)[8][8]
           if (kM <= kDxAdd) {
             __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(slot));
           } else {
+            v *= sc;
             u32x2_t o;
             o[0] = pack_bf16x2(v[0], v[1]);
             o[1] = pack_bf16x2(v[2], v[3]);
@@ -588,7 +590,10 @@ __device__ __forceinline__ void dx_epilogue_bf16(const f32x4_t (&acc)[8][8], con
     float* arow = a.accbuf + (int64_t)(rv ? rowl : 0) * a.ld_acc;
     char* xrow = kMode >= kDxAddEmit ? a.dX + (int64_t)a.row_index[rv ? rowl : 0] * a.lddx_b
                                      : nullptr;
-    const float sc = kMode == kDxEmit && a.row_scale ? a.row_scale[rv ? rowl : 0] : 1.f;
+    const float sc = kMode != kDxEmit ? 1.f
+                     : a.row_scale    ? a.row_scale[rv ? rowl : 0]
+                     : a.out_scale    ? *a.out_scale
+                                      : 1.f;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -817,7 +822,7 @@ __device__ __forceinline__ void dw_store_row(const f32x4_t (&accrow)[8], const D
 // columns past H) get an offset beyond that end.
 __device__ __forceinline__ void dw_narrow_row(const f32x4_t (&accrow)[8], const EpiCoordsBf& ec,
                                               const rsrc_t& dst, uint32_t rows, uint32_t cols,
-                                              uint32_t ldo_b, int fm, char* R) {
+                                              uint32_t ldo_b, float sc, int fm, char* R) {
   const uint32_t i = ec.lane & 15u, q = ec.lane >> 4;
   const uint32_t rr = ec.lane >> 5, c = ec.lane & 31u;
 #pragma unroll
@@ -831,8 +836,8 @@ __device__ __forceinline__ void dw_narrow_row(const f32x4_t (&accrow)[8], const 
     const uint32_t row = ec.wm * 128u + (uint32_t)fm * 16u + lrow;
     const f32x4_t v = __builtin_bit_cast(f32x4_t, lds_read16(R, lrow * 512u + ((c ^ lrow) & 31u) * 16u));
     u32x2_t o;
-    o[0] = pack_bf16x2(v[0], v[1]);
-    o[1] = pack_bf16x2(v[2], v[3]);
+    o[0] = pack_bf16x2(v[0] * sc, v[1] * sc);
+    o[1] = pack_bf16x2(v[2] * sc, v[3] * sc);
     const uint32_t off = row < rows && col < cols ? row * ldo_b + col * 2u : kDwOut;
     __builtin_amdgcn_raw_buffer_store_b64(o, dst, off, 0, kCpolNt);
   }
@@ -842,12 +847,14 @@ __device__ __forceinline__ void dw_narrow_row(const f32x4_t (&accrow)[8], const 
 struct DwNarrowTile {
   rsrc_t r;
   uint32_t rows, cols, ldo_b;
+  float sc;
 };
 __device__ __forceinline__ DwNarrowTile dw_narrow_tile(const DwArgs& a, int32_t m0, int32_t h0) {
   DwNarrowTile t;
   t.rows = (uint32_t)min(256, a.cv - m0);
   t.cols = (uint32_t)min(256, a.H - h0);
   t.ldo_b = (uint32_t)(a.lddw * 2);
+  t.sc = a.out_scale ? *a.out_scale : 1.f;
   t.r = make_rsrc(reinterpret_cast<char*>(a.dW) + (int64_t)(a.v0 + m0) * a.lddw * 2 + (int64_t)h0 * 2,
                   (t.rows - 1u) * t.ldo_b + t.cols * 2u);
   return t;
@@ -862,7 +869,7 @@ __device__ __forceinline__ void dw_store_acc(const f32x4_t (&acc)[8][8], const D
     char* R = scratch + (ec.wm * 2u + ec.wn) * 8192u;
 #pragma unroll
     for (int fm = 0; fm < 8; ++fm) {
-      dw_narrow_row(acc[fm], ec, t.r, t.rows, t.cols, t.ldo_b, fm, R);
+      dw_narrow_row(acc[fm], ec, t.r, t.rows, t.cols, t.ldo_b, t.sc, fm, R);
       sched_fence();
     }
     lgkm_wait0();
@@ -913,7 +920,7 @@ __device__ __forceinline__ void dw_store_then_load(f32x4_t (&acc)[8][8], const D
     char* R = scratch + (ec.wm * 2u + ec.wn) * 8192u;
 #pragma unroll
     for (int fm = 0; fm < 8; ++fm) {
-      dw_narrow_row(acc[fm], ec, t.r, t.rows, t.cols, t.ldo_b, fm, R);
+      dw_narrow_row(acc[fm], ec, t.r, t.rows, t.cols, t.ldo_b, t.sc, fm, R);
       const f32x4_t z = opaque_zero4();
 #pragma unroll
       for (int fn = 0; fn < 8; ++fn) acc[fm][fn] = z;
@@ -1199,12 +1206,12 @@ __global__ __launch_bounds__(256) void narrow_tiles_kernel(const float* scale, c
   }
 }
 
-// Fused path, chunks whose exponentials would leave bf16's range: G = g_t
-// (softmax(cap(S_t)) - onehot(y_t)) (1 - tanh^2), in place over one chunk of
-// the bf16 logits S written by fwd_bf16_kernel<*, kStoreLogits>; nothing
-// unless *run_if != 0 (run_if non-null).  One workgroup per row; rows >= cn
-// and columns >= V become 0.  HBM-bound: one 16-byte read and one 16-byte
-// write per 8 elements.
+// G = g_t (softmax(cap(S_t)) - onehot(y_t)) (1 - tanh^2), in place over the
+// bf16 logits S written by fwd_bf16_kernel<*, kStoreLogits>: the kept logits
+// of a whole call, or (run_if non-null: nothing unless *run_if != 0) a fused
+// chunk whose exponentials would leave bf16's range.  One workgroup per row;
+// rows >= cn and columns >= V become 0.  HBM-bound: one 16-byte read and one
+// 16-byte write per 8 elements.
 template <bool kCap>
 __global__ __launch_bounds__(256) void softmax_grad_kernel(char* S, int64_t lds_b, int32_t cols,
                                                            int32_t cn, int32_t V,

@@ -34,8 +34,9 @@ __all__ = [
 # Optional override of the backward workspace budget in bytes (default: 5% of
 # the materialised-logits size T * V * sizeof(dtype)).
 BACKWARD_BUDGET_ENV = "MT_FLCE_BWD_BUDGET_BYTES"
-# With grad_scale given (bf16): "auto" (default) takes the fused path when the
-# planner expects it to pay, "1" always, "0" never.
+# bf16: "auto" (default) keeps the logits where they fit (_kept_plan) and takes
+# the fused path when the planner expects it to pay, "1" always takes the fused
+# path, "0" always the recomputing general one.
 FUSED_ENV = "MT_FLCE_FUSED"
 
 
@@ -122,11 +123,32 @@ def backward_plan(T: int, n_valid: int, H: int, V: int, dtype: torch.dtype,
     return c.value, cv.value, ws.value
 
 
+# The least default workspace: 5% of the logits of a short call is less than
+# one block of whole tiles for every CU needs (a 300-token fp32 call ran 14
+# vocabulary blocks of 256 columns), and 32 MiB is 0.01% of the device memory.
+MIN_BUDGET = 32 << 20
+
+
 def _default_budget(T: int, V: int, es: int) -> int:
-    """The workspace budget the planners use when given 0: the override in
-    MT_FLCE_BWD_BUDGET_BYTES, else 5% of the T x V logits in bytes."""
+    """The workspace budget of a call: the override in
+    MT_FLCE_BWD_BUDGET_BYTES, else 5% of the T x V logits in bytes, at least
+    MIN_BUDGET."""
     env = int(os.environ.get(BACKWARD_BUDGET_ENV, "0"))
-    return env if env > 0 else int(float(T) * V * es * 0.05)
+    return env if env > 0 else max(int(float(T) * V * es * 0.05), MIN_BUDGET)
+
+
+def _kept_plan(T: int, n: int, H: int, V: int) -> Tuple[int, int, int, bool]:
+    """(columns, logits bytes, backward scratch bytes, pays) of a bf16 call
+    that keeps logits from the forward to the backward (mt_flce_logits_plan),
+    columns 0 when none fit.  The default budget counts the bytes by which a
+    bf16 weight gradient is smaller than the fp32 one of the other paths; a
+    budget set by MT_FLCE_BWD_BUDGET_BYTES is taken as it stands."""
+    room = int(int(os.environ.get(BACKWARD_BUDGET_ENV, "0")) == 0)
+    cols, lb, sb, pays = ctypes.c_int64(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int()
+    check(load().mt_flce_logits_plan(T, n, H, V, MT_DTYPE_BF16, _default_budget(T, V, 2), room,
+                                     ctypes.byref(cols), ctypes.byref(lb), ctypes.byref(sb),
+                                     ctypes.byref(pays)), "mt_flce_logits_plan")
+    return cols.value, lb.value, sb.value, bool(pays.value)
 
 
 def _grad_vector(grad: torch.Tensor, T: int) -> Tuple[torch.Tensor, int]:
@@ -206,7 +228,12 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                 its GEMM -- the forward then also keeps the first vocabulary
                 block's exponentials for it, mt_flce_forward_keep, softcap
                 off -- else mt_flce_backward_tiles, dW as 256 x 256 fp32
-                tiles narrowed by mt_flce_narrow_tiles).
+                tiles narrowed by mt_flce_narrow_tiles).  Where it pays
+                (bf16, no dw_accumulator, _kept_plan: every column fits up
+                to about H counted tokens) the forward keeps logits
+                (mt_flce_forward_logits) and the first backward recomputes
+                only the columns not kept (mt_flce_backward_logits): 6 H V n
+                flops instead of 8 when it keeps them all.
     fused       grad_scale promised the upstream gradient at the forward and
                 the planner expects the fused path to pay (bf16,
                 mt_flce_fused_plan): the forward also forms dX and dW for it
@@ -252,8 +279,17 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         loss = torch.empty(T, dtype=torch.float32, device=dev)
         ctx.path = "general"
         ctx.ranges = [(p[0], p[1], p[4]) for p in parts]
+        ctx.keep = ctx.logits = None
         plans = None
-        if dt == MT_DTYPE_BF16 and n_tot > 0 and (grad_scale is not None or allow_unit):
+        kept = None
+        if (dt == MT_DTYPE_BF16 and allow_unit and grad_scale is None and len(parts) == 1
+                and n_tot > 0 and _fused_mode() == "auto"):
+            kept = _kept_plan(T, n_tot, H, V)
+            kept = kept if kept[3] else None
+        if kept is None and dt == MT_DTYPE_BF16 and n_tot > 0 and (grad_scale is not None or allow_unit):
+            # planned at 5% of the logits, also where MIN_BUDGET gives a short
+            # call more: the general path's blocks grow with it, and its dX
+            # carries one rounding less than the fused path's
             plans = [fused_plan(t1 - t0, n, H, V, accumulator=dw_accumulator is not None)
                      if n > 0 else (0, 0, True) for t0, t1, _, _, n in parts]
             live = [pl for pl, p in zip(plans, parts) if p[4] > 0]
@@ -303,13 +339,26 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             ctx.dW = None if dw_accumulator is not None else dW
             ctx.fused_consumed = False
             return loss.view(hidden.shape[:-1])
-        ctx.keep = None
         for t0, t1, ri, rl, n in parts:
             lse = torch.empty(n, dtype=torch.float32, device=dev)
             lses.append(lse)
             Xr, lr = X[t0:t1], loss[t0:t1]
             plan = None
             ws_bytes = lib.mt_flce_forward_workspace_bytes(t1 - t0, n, H, V, dt)
+            if kept is not None:
+                # the logits live from here to the backward (or until the
+                # loss's graph is freed, when no backward follows)
+                cols, logits_bytes, scratch_bytes, _ = kept
+                logits = torch.empty(logits_bytes, dtype=torch.uint8, device=dev)
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+                check(lib.mt_flce_forward_logits(_p(Xr), _p(W), T, H, V, X.stride(0), W.stride(0),
+                                                 dt, float(softcap), _p(ri), _p(rl), n, _p(lr),
+                                                 _p(lse), _p(ws), ws_bytes, _p(logits), cols,
+                                                 logits_bytes, _stream(dev)),
+                      "mt_flce_forward_logits")
+                ctx.logits = (logits, cols, scratch_bytes)
+                del ws, logits
+                continue
             if (dt == MT_DTYPE_BF16 and allow_unit and float(softcap) == 0.0 and n > 0
                     and len(parts) == 1):
                 # the kept block sits beside the forward's own workspace: plan
@@ -369,16 +418,33 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         dev = X.device
         g, gstride = _grad_vector(grad_loss, T)
         dX = torch.empty((T, H), dtype=X.dtype, device=dev)
-        if acc is None and dt == MT_DTYPE_BF16:
+        logits, ctx.logits = ctx.logits, None
+        if logits is not None:
+            # the first backward: G from the logits its forward kept
+            (t0, t1, n, ri, rl, lse), (kept, cols, scratch_bytes) = rngs[0], logits
+            scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
+            out = torch.empty((V, H), dtype=torch.bfloat16, device=dev)
+            check(lib.mt_flce_backward_logits(_p(X), _p(W), T, H, V, X.stride(0), W.stride(0), dt,
+                                              softcap, _p(ri), _p(rl), n, _p(lse), _p(g), gstride,
+                                              _p(dX), dX.stride(0), _p(out), out.numel() * 2,
+                                              _p(kept), cols, kept.numel(), _p(scratch),
+                                              scratch_bytes, _stream(dev)),
+                  "mt_flce_backward_logits")
+            del kept, scratch, logits
+            grad_w = out if need_w else None
+        elif acc is None and dt == MT_DTYPE_BF16:
             # dW in bf16; the first backward takes the exponentials its
             # forward kept
-            keep, ctx.keep = getattr(ctx, "keep", None), None
+            keep, ctx.keep = ctx.keep, None
             grad_w = _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX, keep=keep)
             grad_w = grad_w if need_w else None
         else:
             dW = acc if acc is not None else torch.empty((V, H), dtype=torch.float32, device=dev)
             for r, (t0, t1, n, ri, rl, lse) in enumerate(rngs):
-                C, Cv, ws_bytes = backward_plan(t1 - t0, n, H, V, X.dtype)
+                budget = _default_budget(t1 - t0, V, X.element_size())
+                C, Cv, ws_bytes = backward_plan(t1 - t0, n, H, V, X.dtype, budget)
+                if dt == MT_DTYPE_F32:  # what the budget leaves holds planes of a split dX
+                    ws_bytes = max(ws_bytes, min(budget, ws_bytes + 8 * C * H * 4))
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
                 gr = g[t0:t1] if gstride else g
                 check(lib.mt_flce_backward(_p(X[t0:t1]), _p(W), t1 - t0, H, V, X.stride(0),
@@ -497,7 +563,8 @@ def _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX,
     one = len(rngs) == 1
     if one:
         n = rngs[0][2]
-        plan = keep[:3] if keep is not None else backward_plan(T, n, H, V, X.dtype, narrow=True)
+        plan = keep[:3] if keep is not None else backward_plan(
+            T, n, H, V, X.dtype, _default_budget(T, V, 2), narrow=True)
     if one and plan[0] >= n:
         (t0, t1, n, ri, rl, lse), (C, Cv, ws) = rngs[0], plan
         if keep is not None:
@@ -527,7 +594,8 @@ def _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX,
         # one range: the narrowing plan (several row blocks here); more: the
         # plan of mt_flce_backward_tiles itself (dX's accumulator and X^T in
         # the workspace)
-        C, Cv, ws_bytes = (plan if one else backward_plan(t1 - t0, n, H, V, X.dtype))
+        C, Cv, ws_bytes = (plan if one else backward_plan(t1 - t0, n, H, V, X.dtype,
+                                                          _default_budget(t1 - t0, V, 2)))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         gr = g[t0:t1] if gstride else g
         check(lib.mt_flce_backward_tiles(_p(X[t0:t1]), _p(W), t1 - t0, H, V, X.stride(0),
@@ -611,13 +679,17 @@ def fused_plan(T: int, n_valid: int, H: int, V: int, budget_bytes: Optional[int]
     return c.value, ws.value, bool(pays.value)
 
 
-def _use_fused(pays: bool) -> bool:
+def _fused_mode() -> str:
+    """"always", "never" or "auto" (MT_FLCE_FUSED)."""
     mode = os.environ.get(FUSED_ENV, "auto").strip().lower()
     if mode in ("1", "on", "always"):
-        return True
-    if mode in ("0", "off", "never"):
-        return False
-    return pays
+        return "always"
+    return "never" if mode in ("0", "off", "never") else "auto"
+
+
+def _use_fused(pays: bool) -> bool:
+    mode = _fused_mode()
+    return pays if mode == "auto" else mode == "always"
 
 
 def _promised_grad(grad_scale, T: int, dev: torch.device) -> Tuple[torch.Tensor, int]:
