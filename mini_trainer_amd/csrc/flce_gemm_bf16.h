@@ -144,7 +144,7 @@ struct KcOp {
   rsrc_t rsrc;
   uint32_t off[kNIBf];
   uint32_t frag[2];  // LDS offset of this lane's fragment 0 for K halves 0, 1
-  uint32_t tail_bad;  // bit i: DMA instruction i's chunk lies past K in the last stage
+  bool tail_bad[2];  // even / odd DMA instructions: their chunk lies past K in the last stage
 
   __device__ __forceinline__ static uint32_t row_of(uint32_t i) {
     const uint32_t l = lane_id(), q = wave_id() * kNIBf + i;
@@ -162,11 +162,10 @@ struct KcOp {
     for (uint32_t i = 0; i < kNIBf; ++i) off[i] = row_off(row_of(i)) + chunk_of(i) * 16u;
   }
   // c_lim: 16-byte chunks (of 8) of the last K stage that lie below K.
+  // (chunk_of depends on i through its parity only)
   __device__ __forceinline__ void set_tail(uint32_t c_lim) {
-    uint32_t m = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < kNIBf; ++i) m |= (chunk_of(i) >= c_lim ? 1u : 0u) << i;
-    tail_bad = m;
+    tail_bad[0] = chunk_of(0) >= c_lim;
+    tail_bad[1] = chunk_of(1) >= c_lim;
   }
   // wave_row0: first tile row of this wave's fragments.
   __device__ __forceinline__ void init_frag(uint32_t wave_row0) {
@@ -183,14 +182,12 @@ struct KcOp {
     for (int i = 0; i < kNIBf; ++i) issue_one(tile, kt, i);
   }
   // The same with a possibly partial last K stage (tail: kt is that stage):
-  // chunks past K re-read chunk 0 of their row, which is in bounds, and the
-  // fragments holding them are zeroed after they are read (mask_tail), so no
-  // byte past a row's K extent -- past the end of the array for its last
-  // row -- is touched.  Branch-free: the choice is a select on the offsets.
+  // a chunk past K gets an offset past the resource (whose size is a multiple
+  // of 16 below 4 GiB), so that its DMA touches no memory and fills the LDS
+  // with zeros: the MFMAs need no mask.
   __device__ __forceinline__ void issue_one_k(char* tile, int kt, int i, bool tail) const {
-    const bool bad = tail && ((tail_bad >> i) & 1u);
-    const uint32_t voff = bad ? off[i] - chunk_of(i) * 16u : (tail ? off[i] + (uint32_t)kt * 128u : off[i]);
-    dma16(rsrc, tile + (wave_id() * kNIBf + (uint32_t)i) * 1024u, voff, tail ? 0u : (uint32_t)kt * 128u);
+    const uint32_t voff = tail && tail_bad[i & 1] ? 0xfffffff0u : off[i];
+    dma16(rsrc, tile + (wave_id() * kNIBf + (uint32_t)i) * 1024u, voff, (uint32_t)kt * 128u);
   }
   __device__ __forceinline__ void issue_k(char* tile, int kt, bool tail) const {
 #pragma unroll
@@ -200,15 +197,6 @@ struct KcOp {
     return lds_read16(tile, frag[kk] + (uint32_t)f * 2048u);
   }
 };
-
-// Zero the fragments of K half kk of the last (partial) K stage in the lanes
-// whose 8 K values lie at or past K: lane l holds K chunk kk * 4 + (l >> 4)
-// of the stage, and the stage's first c_lim chunks lie below K.
-__device__ __forceinline__ void mask_tail(u32x4_t (&fr)[8], int kk, uint32_t c_lim) {
-  const bool bad = (uint32_t)kk * 4u + (lane_id() >> 4) >= c_lim;
-#pragma unroll
-  for (int f = 0; f < 8; ++f) fr[f] = bad ? u32x4_t{0u, 0u, 0u, 0u} : fr[f];
-}
 
 // Operand stored K-major: row-major [K, 256-column tile].  Instruction q of
 // the tile covers K rows 2 q and 2 q + 1; lane l writes LDS chunk l & 31 of
@@ -344,9 +332,11 @@ __device__ __forceinline__ void wait_vm8() {
 // Each phase is one basic block: the retarget branch sits before phase 1,
 // and every phase issues its DMA -- the two stages past the end reload the
 // last tile's final stage into slots that are never read again.
-// kKTail (both operands KcOp, K contiguous in their rows): the last K stage
-// holds only c_lim of its 8 chunks below K; its DMA keeps to the rows' K
-// extent and its fragments are masked (KcOp::issue_one_k, mask_tail).
+// kKTail (both operands KcOp, K contiguous in their rows): the last K stage is
+// partial; its DMA fills the chunks past K with zeros (KcOp::issue_one_k).
+// (Clamped addresses and fragments zeroed in registers, as it was, spilled up
+// to 269 VGPRs per lane into the K loop: 1.0 ms for 256 rows x 4264 x 43534,
+// 96 TFLOP/s.)
 // more(t): does tile t exist?  It is asked in increasing order of t, at most
 // one tile ahead of the one being multiplied when KT >= 2 (two ahead when
 // KT == 1) -- a tile stream whose length is found as it runs (a work queue)
@@ -358,7 +348,7 @@ template <bool kThreeA, bool kKTail = false, bool kCarry = false, class A, class
           class Retarget, class Epi, class Init = ZeroInit>
 __device__ __forceinline__ void mainloop_bf16_seq(char* lds, A& a, B& b, int KT, More more,
                                                   Retarget retarget, Epi epilogue,
-                                                  Init init = Init(), uint32_t c_lim = 8) {
+                                                  Init init = Init()) {
   if (KT <= 0 || !more(0)) return;
   // With a transposed operand (two ds_read_b64_tr_b16 per fragment) each DMA
   // instruction goes one MFMA into the group after the LDS read it used to
@@ -429,12 +419,6 @@ __device__ __forceinline__ void mainloop_bf16_seq(char* lds, A& a, B& b, int KT,
     if (!kCarry || tile == 0) init(tile, acc);
     for (int kt = 0; kt < KT; ++kt, ++g, g3 = (g3 == 2 ? 0 : g3 + 1)) {
       advance();
-      if constexpr (kKTail) {
-        if (kt == KT - 1) {
-          mask_tail(fa0, 0, c_lim);
-          mask_tail(fb0, 0, c_lim);
-        }
-      }
       sched_fence();
       const int g2 = g & 1, g2n = g2 ^ 1;
       const int g3n = g3 == 2 ? 0 : g3 + 1, g3p = g3 == 0 ? 2 : g3 - 1;  // (g+1)%3, (g+2)%3
@@ -475,12 +459,6 @@ __device__ __forceinline__ void mainloop_bf16_seq(char* lds, A& a, B& b, int KT,
       tie_frags<B>(fb1);
       wait_vm8();
       __builtin_amdgcn_s_barrier();
-      if constexpr (kKTail) {
-        if (kt == KT - 1) {
-          mask_tail(fa1, 1, c_lim);
-          mask_tail(fb1, 1, c_lim);
-        }
-      }
       sched_fence();
       // phase 2: MFMAs on F1(g), DMA of the two-slot operand's stage g + 2
       // into the slot of its stage g, LDS reads of F0(g + 1) (stale after the
@@ -547,11 +525,10 @@ __device__ __forceinline__ void mainloop_bf16_seq(char* lds, A& a, B& b, int KT,
 template <bool kThreeA, bool kKTail = false, class A, class B, class Retarget, class Epi,
           class Init = ZeroInit>
 __device__ __forceinline__ void mainloop_bf16(char* lds, A& a, B& b, int KT, int ntiles,
-                                              Retarget retarget, Epi epilogue, Init init = Init(),
-                                              uint32_t c_lim = 8) {
+                                              Retarget retarget, Epi epilogue, Init init = Init()) {
   mainloop_bf16_seq<kThreeA, kKTail>(
       lds, a, b, KT, [ntiles](int t) __attribute__((always_inline)) { return t < ntiles; },
-      retarget, epilogue, init, c_lim);
+      retarget, epilogue, init);
 }
 
 }  // namespace mtf

@@ -353,7 +353,7 @@ __device__ __forceinline__ void fwd_bf16_body(char* lds, const FwdArgs& a, int n
         // the merge's LDS is the ring slot refilled in the next phase 1
         __syncthreads();
       },
-      ZeroInit(), c_lim);
+      ZeroInit());
 }
 
 // kTail: V is not a multiple of 256.  Only the last vocabulary tile column
@@ -520,7 +520,7 @@ MT_GEMM_BF16_KERNEL void recompute_bf16_kernel(RecompArgs a) {
         const int32_t row0 = (int32_t)tm * 256, col0 = (int32_t)tn * 256;
         recompute_epilogue_bf16<kCap, kTail>(acc, a, ec, row0, col0);
       },
-      ZeroInit(), c_lim);
+      ZeroInit());
 }
 
 // dX tile epilogue of the bf16 kernels (one mode of dx_epilogue per
