@@ -339,6 +339,18 @@ int mt_flce_backward_narrow(const void* X, const void* W, int64_t T, int64_t H,
 size_t mt_flce_narrow_scratch_bytes(int64_t V, int64_t H, int64_t chunk_rows);
 
 /*
+ * *pays = 1 if the general path (mt_flce_forward and the blocks of
+ * mt_flce_backward_narrow_plan under general_budget) is expected to beat the
+ * fused one under fused_budget (0 = 5% of T V 2 each), for a bf16 weight
+ * gradient without an accumulator: short calls and small vocabularies, whose
+ * 5% holds fused chunks of 256 rows only, when the caller has more workspace
+ * to give.  (No reference counterpart, as mt_flce_fused_plan.)
+ */
+int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V,
+                         int dtype, size_t fused_budget, size_t general_budget,
+                         int* pays);
+
+/*
  * Training with the logits (or as many of their columns as fit) kept from the
  * forward to the backward, bf16 only: the forward stores the bf16-rounded
  * logits of vocabulary columns [0, keep_cols) of every counted row, the
@@ -352,7 +364,8 @@ size_t mt_flce_narrow_scratch_bytes(int64_t V, int64_t H, int64_t chunk_rows);
  * fp32 accumulator or the planes of a dX split over the vocabulary), which fit
  * budget_bytes (0 = 5% of T V 2) -- plus, with count_gradient != 0, the bytes
  * (V H 2 and tile padding) by which a bf16 weight gradient is smaller than the
- * fp32 one the other paths accumulate -- and *pays = 1 when every column is
+ * fp32 one the other paths accumulate (not with_accumulator: dW is then added
+ * into the caller's fp32 accumulator) -- and *pays = 1 when every column is
  * kept or a cost model expects this to beat the path that
  * mt_flce_fused_plan's user would take under the same budget.  All 0 when
  * nothing fits.
@@ -361,9 +374,11 @@ size_t mt_flce_narrow_scratch_bytes(int64_t V, int64_t H, int64_t chunk_rows);
  * that also writes the logits.  mt_flce_backward_logits consumes them (they
  * hold G afterwards, so it runs once per forward): dX [T, H] bf16, zero at
  * ignored rows, and the weight gradient as contiguous bf16 rows [V, H] at
- * dW_out (V H 2 bytes), narrowed once from fp32 sums over all counted rows;
+ * dW_out (V H 2 bytes), narrowed once from fp32 sums over all counted rows --
+ * or, with dW_acc (fp32 rows of pitch lddw_acc), added into that instead.
  * grad_loss and grad_stride as in mt_flce_backward; one scalar (stride 0) is
- * applied to the fp32 sums, a per-token gradient is part of G.  A scratch
+ * applied to the fp32 sums when dW goes to dW_out, else it is part of G, as a
+ * per-token gradient is.  A scratch
  * smaller than planned (but with X^T, the queue and, for keep_cols < V, the
  * accumulator) means fewer dX slices.  n_valid >= 1, H a multiple of 8.
  * Replaces the same reference interface as mt_flce_forward and
@@ -372,8 +387,8 @@ size_t mt_flce_narrow_scratch_bytes(int64_t V, int64_t H, int64_t chunk_rows);
  */
 int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V,
                         int dtype, size_t budget_bytes, int count_gradient,
-                        int64_t* keep_cols, size_t* logits_bytes,
-                        size_t* scratch_bytes, int* pays);
+                        int with_accumulator, int64_t* keep_cols,
+                        size_t* logits_bytes, size_t* scratch_bytes, int* pays);
 int mt_flce_forward_logits(const void* X, const void* W, int64_t T, int64_t H,
                            int64_t V, int64_t ldx, int64_t ldw, int dtype,
                            float softcap, const int32_t* row_index,
@@ -388,10 +403,10 @@ int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H,
                             const int32_t* row_label, int64_t n_valid,
                             const float* lse, const float* grad_loss,
                             int64_t grad_stride, void* dX, int64_t lddx,
-                            void* dW_out, size_t dw_out_bytes, void* logits,
-                            int64_t keep_cols, size_t logits_bytes,
-                            void* scratch, size_t scratch_bytes,
-                            mt_stream_t stream);
+                            void* dW_out, size_t dw_out_bytes, float* dW_acc,
+                            int64_t lddw_acc, void* logits, int64_t keep_cols,
+                            size_t logits_bytes, void* scratch,
+                            size_t scratch_bytes, mt_stream_t stream);
 
 /*
  * Layout of the tiled fp32 weight gradient that mt_flce_fused_tiles and

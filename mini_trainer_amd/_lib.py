@@ -72,8 +72,10 @@ SIGNATURES = {
                                         c_size_t, c_void_p, c_size_t, c_int64, c_int64, c_void_p,
                                         c_size_t, c_void_p, c_void_p]),
     "mt_flce_logits_plan": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int, c_size_t, c_int,
-                                    POINTER(c_int64), POINTER(c_size_t), POINTER(c_size_t),
+                                    c_int, POINTER(c_int64), POINTER(c_size_t), POINTER(c_size_t),
                                     POINTER(c_int)]),
+    "mt_flce_general_pays": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int, c_size_t, c_size_t,
+                                     POINTER(c_int)]),
     "mt_flce_forward_logits": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                        c_int64, c_int, c_float, c_void_p, c_void_p, c_int64,
                                        c_void_p, c_void_p, c_void_p, c_size_t, c_void_p, c_int64,
@@ -81,8 +83,8 @@ SIGNATURES = {
     "mt_flce_backward_logits": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
                                         c_int64, c_int, c_float, c_void_p, c_void_p, c_int64,
                                         c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
-                                        c_size_t, c_void_p, c_int64, c_size_t, c_void_p, c_size_t,
-                                        c_void_p]),
+                                        c_size_t, c_void_p, c_int64, c_void_p, c_int64, c_size_t,
+                                        c_void_p, c_size_t, c_void_p]),
     "mt_flce_narrow_scratch_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "mt_flce_dw_tiles_layout": (c_int, [c_int64, c_int64, POINTER(c_size_t), POINTER(c_int64),
                                         POINTER(c_size_t)]),

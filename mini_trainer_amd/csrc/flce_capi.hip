@@ -509,10 +509,10 @@ double tile_time(int64_t k, int64_t extra = 0) {
   return 2.0 * 256 * 256 * (double)(round_up(k, 64) + kEpiK + extra) / kCuRate;
 }
 
-double gemm_time(int64_t tiles, int64_t k, int64_t extra = 0) {
+double gemm_time(int64_t tiles, int64_t k, int64_t extra = 0, double idle = 0.3) {
   if (tiles <= 0) return 0.0;
   const double full = (double)tiles / kCUs, rounds = std::ceil(full);
-  return (full + 0.3 * (rounds - full)) * tile_time(k, extra) + kLaunch;
+  return (full + idle * (rounds - full)) * tile_time(k, extra) + kLaunch;
 }
 
 // dX (dx_items tiles of depth dx_k, one per CU) beside dW (dw_tiles of depth
@@ -526,23 +526,29 @@ double phase_time(int64_t dx_items, int64_t dx_k, int64_t dw_tiles, int64_t dw_k
 
 // Modelled seconds for one backward with blocks of C x Cv.  narrow: the
 // narrowing entry (one row block, dW tiles stored once in bf16, dX and dW
-// of every block in one launch).
+// of every block in one launch).  blocks: the estimate the blocks are chosen
+// by -- a launch of a few rounds is charged 60% of a busy CU for each idle one
+// (540 recompute tiles of depth 3584 run in 243 us, 2.7 rounds' time; the 30%
+// that rank the paths fit launches of many rounds), and no launch is shorter
+// than its longest tile: one dW tile over 35k rows took 0.8 ms of a block
+// whose CUs' share of the work was 0.1.
 double backward_cost(int64_t N, int64_t H, int64_t V, int64_t C, int64_t Cv, int es,
-                     bool narrow = false) {
+                     bool narrow = false, bool blocks = false) {
   (void)es;
   double t = 0, bytes = 0;
+  const double idle = blocks ? 0.6 : 0.3;
   for (int64_t c0 = 0; c0 < N; c0 += C) {
     const int64_t cn = std::min(C, N - c0);
     const int64_t nv = cdiv(V, Cv), tm = cdiv(cn, 256), th = cdiv(H, 256);
     for (int64_t v0 = 0; v0 < V; v0 += Cv) {
       const int64_t cv = std::min(Cv, V - v0), tv = cdiv(cv, 256);
-      t += gemm_time(tm * tv, H);
-      if (narrow)
-        t += phase_time(tm * th, cv, tv * th, cn, 0);
-      else if (tm * th < kCUs)
-        t += phase_time(tm * th, cv, tv * th, cn);  // dW beside dX
+      const int64_t extra = narrow ? 0 : kDwRmwK;
+      const double dw_tile = blocks ? tile_time(cn, extra) : 0.0;
+      t += blocks ? std::max(gemm_time(tm * tv, H, 0, idle), tile_time(H)) : gemm_time(tm * tv, H);
+      if (narrow || tm * th < kCUs)  // dW beside dX
+        t += std::max(phase_time(tm * th, cv, tv * th, cn, extra), dw_tile);
       else
-        t += gemm_time(tm * th, cv) + gemm_time(tv * th, cn, kDwRmwK);
+        t += gemm_time(tm * th, cv, 0, idle) + std::max(gemm_time(tv * th, cn, extra, idle), dw_tile);
     }
     if (nv > 1) bytes += (double)(2 * nv - 2) * cn * H * 4;  // dX accumulator
     t += kLaunch;
@@ -608,8 +614,11 @@ inline bool narrow_scratch_fits(int64_t V, int64_t H, int64_t C) {
 // mt_flce_backward_narrow: no dW read-modify-write, no narrowing pass, and
 // dX's accumulator in the dW buffer; more row blocks run
 // mt_flce_backward_tiles and the narrowing pass, which the cost includes.
+// blocks (a plan to run, not one to price a path with): the cost model of the
+// blocks, and for the best row blocking also a few more, smaller vocabulary
+// blocks, whose tiles may fill whole rounds better.
 BwdPlan plan_backward(int64_t T, int64_t N, int64_t H, int64_t V, int es, size_t budget,
-                      bool narrow = false) {
+                      bool narrow = false, bool blocks = false) {
   BwdPlan best;
   if (N <= 0) return best;
   if (budget == 0) budget = (size_t)((double)T * V * es * 0.05);
@@ -623,29 +632,34 @@ BwdPlan plan_backward(int64_t T, int64_t N, int64_t H, int64_t V, int es, size_t
   const int64_t max_nt = std::min<int64_t>(cdiv(N, 256), 128);
   const int64_t max_nv = std::min<int64_t>(cdiv(V, 256), 128);
   const double narrow_pass = (double)V * H * 6 / kBw + 10 * kLaunch;
+  // blocks of C x Cv: takes them if they fit and cost less; whether they fit
+  auto consider = [&](int64_t C, int64_t Cv) {
+    const bool one = narrow && C >= N;
+    const size_t ws = backward_ws(C, Cv, H, V, es, one && narrow_scratch_fits(V, H, C));
+    // G, X^T and the block's weight rows (bf16) within one buffer's reach
+    const uint64_t lim = buffer_limit();
+    if ((uint64_t)C * Cv * es > lim || (uint64_t)H * C * es > lim ||
+        (es == 2 && (uint64_t)Cv * H * es > lim))
+      return false;
+    if (ws > budget) return false;
+    const double cost =
+        backward_cost(N, H, V, C, Cv, es, one, blocks) + (narrow && !one ? narrow_pass : 0.0);
+    if (cost < best_cost * 0.999) {
+      best_cost = cost;
+      best.C = C;
+      best.Cv = Cv;
+      best.ws = ws;
+    }
+    return true;
+  };
   for (int64_t nt = 1; nt <= max_nt; ++nt) {
     const int64_t C = round_up(cdiv(N, nt), 256);
-    const bool one = narrow && nt == 1;
-    for (int64_t nv = 1; nv <= max_nv; ++nv) {
-      const int64_t Cv = round_up(cdiv(V, nv), 256);
-      const size_t ws = backward_ws(C, Cv, H, V, es, one && narrow_scratch_fits(V, H, C));
-      // G and X^T are read through 32-bit buffer offsets
-      // G, X^T and the block's weight rows (bf16) within one buffer's reach
-      const uint64_t lim = buffer_limit();
-      if ((uint64_t)C * Cv * es > lim || (uint64_t)H * C * es > lim ||
-          (es == 2 && (uint64_t)Cv * H * es > lim))
-        continue;
-      if (ws > budget) continue;
-      const double cost =
-          backward_cost(N, H, V, C, Cv, es, one) + (narrow && !one ? narrow_pass : 0.0);
-      if (cost < best_cost * 0.999) {
-        best_cost = cost;
-        best.C = C;
-        best.Cv = Cv;
-        best.ws = ws;
-      }
-      break;  // larger nv only shrinks blocks further
-    }
+    for (int64_t nv = 1; nv <= max_nv; ++nv)
+      if (consider(C, round_up(cdiv(V, nv), 256))) break;  // larger nv only shrinks blocks further
+  }
+  if (blocks && best.C) {
+    const int64_t C = best.C, nv = cdiv(V, best.Cv);
+    for (int64_t more = 1; more <= 6; ++more) consider(C, round_up(cdiv(V, nv + more), 256));
   }
   return best.C ? best : smallest;
 }
@@ -1436,13 +1450,17 @@ struct KeptPlan {
 
 // dX is split over a block's columns into split.S slices with an fp32 plane
 // [C, H] each (as the fused path's, but kept over the blocks and summed at the
-// end); with one slice and several blocks its accumulator is tiled.
-size_t kept_scratch(int64_t C, int64_t H, int64_t S, bool blocks) {
+// end); with one slice and several blocks its accumulator is one plane, or
+// (acc false: dW in bf16, whose kernels take it) tiles.
+size_t kept_scratch(int64_t C, int64_t H, int64_t S, bool blocks, bool acc) {
   return align_up((size_t)H * C * 2) + align_up((kQueueWords + 1) * sizeof(uint32_t)) +
-         (S > 1 ? align_up((size_t)S * C * H * sizeof(float)) : (blocks ? align_up(tiled_acc_bytes(C, H)) : 0));
+         (S > 1 || (blocks && acc) ? align_up((size_t)S * C * H * sizeof(float))
+                                   : (blocks ? align_up(tiled_acc_bytes(C, H)) : 0));
 }
 
-double kept_cost(int64_t N, int64_t H, int64_t V, int64_t cols, const DxSplit& d) {
+// acc: dW is added into an fp32 accumulator instead of written in bf16.
+double kept_cost(int64_t N, int64_t H, int64_t V, int64_t cols, const DxSplit& d, bool acc) {
+  const int64_t extra = acc ? kDwRmwK : 0;
   const int64_t tm = cdiv(N, 256), th = cdiv(H, 256), nb = cdiv(V, cols);
   double t = forward_cost(N, H, V) + (nb > 1 ? kLaunch : 0);
   t += 4.0 * N * std::min(cols, V) / kBw;  // logits read, G written
@@ -1450,7 +1468,8 @@ double kept_cost(int64_t N, int64_t H, int64_t V, int64_t cols, const DxSplit& d
     const int64_t cv = std::min(cols, V - v0), tv = cdiv(cv, 256);
     if (v0 > 0) t += gemm_time(tm * tv, H);
     // (few columns: one dW tile over all rows can be the longest item)
-    t += std::max(phase_time(tm * th * d.S, cdiv(cv, d.S), tv * th, N, 0), tile_time(N) + 2 * kLaunch);
+    t += std::max(phase_time(tm * th * d.S, cdiv(cv, d.S), tv * th, N, extra),
+                  tile_time(N, extra) + 2 * kLaunch);
   }
   // dX planes (or the accumulator) stored, re-read and added to, then summed
   const double plane = (double)N * H * 4;
@@ -1475,7 +1494,7 @@ DxSplit kept_split(int64_t cols, int64_t V, int64_t S) {
 // slices keep to XCDs of their own, see fused_split) the columns that fit, and of
 // these the cheapest.  Too few slices and dX, whose tiles contract a whole
 // block, outlasts dW beside it; a plane costs 2 H columns.
-KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bool room) {
+KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bool room, bool acc) {
   KeptPlan best;
   if (N <= 0 || H % 8 != 0) return best;
   if (budget == 0) budget = (size_t)((double)T * V * 2 * 0.05);
@@ -1488,7 +1507,7 @@ KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bo
   const int64_t reach = (int64_t)(std::min(lim / ((uint64_t)C * 2), lim / ((uint64_t)H * 2)) / 256 * 256);
   for (int64_t S = 1; S <= 32; S *= 2) {
     for (int blocks = 0; blocks < 2; ++blocks) {
-      const size_t other = std::max(kept_scratch(C, H, S, blocks != 0), fwd);
+      const size_t other = std::max(kept_scratch(C, H, S, blocks != 0, acc), fwd);
       if (other > have) continue;
       int64_t cols = std::min<int64_t>((int64_t)((have - other) / ((size_t)C * 2)) / 256 * 256, reach);
       if (blocks == 0 && cols < Vp) continue;  // several blocks
@@ -1496,11 +1515,11 @@ KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bo
       if (cols < 256 || (S > 1 && std::min(cols, V) / S < 256)) continue;
       const DxSplit d = kept_split(cols, V, S);
       if (d.S != S && S > 1) continue;
-      const double t = kept_cost(N, H, V, cols, d);
+      const double t = kept_cost(N, H, V, cols, d, acc);
       if (t < best.cost) {
         best.cols = cols;
         best.logits = align_up((size_t)C * cols * 2);
-        best.scratch = kept_scratch(C, H, d.S, cols < V);
+        best.scratch = kept_scratch(C, H, d.S, cols < V, acc);
         best.split = d;
         best.cost = t;
       }
@@ -1510,20 +1529,22 @@ KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bo
 }
 
 // The most slices (a power of two) whose planes fit a scratch of `bytes`.
-int64_t kept_slices_in(int64_t C, int64_t H, bool blocks, size_t bytes) {
+int64_t kept_slices_in(int64_t C, int64_t H, bool blocks, bool acc, size_t bytes) {
   int64_t S = 32;
-  while (S > 1 && kept_scratch(C, H, S, blocks) > bytes) S /= 2;
+  while (S > 1 && kept_scratch(C, H, S, blocks, acc) > bytes) S /= 2;
   return S;
 }
 
 int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V, int64_t ldx,
                            int64_t ldw, float softcap, const int32_t* row_index,
                            const int32_t* row_label, int64_t N, const float* lse, const float* grad,
-                           int64_t gstride, void* dX, int64_t lddx, void* dW, char* logits, int64_t cols,
-                           char* scratch, size_t scratch_bytes, hipStream_t stream) {
+                           int64_t gstride, void* dX, int64_t lddx, void* dW, int64_t lddw_acc,
+                           char* logits, int64_t cols, char* scratch, size_t scratch_bytes,
+                           hipStream_t stream) {
+  const bool acc = lddw_acc > 0;  // add into fp32 rows of that pitch
   const int64_t C = round_up(N, 256), nb = cdiv(V, cols);
   const int64_t ldg_b = cols * 2, ldxt_b = C * 2;
-  const DxSplit split = kept_split(cols, V, kept_slices_in(C, H, nb > 1, scratch_bytes));
+  const DxSplit split = kept_split(cols, V, kept_slices_in(C, H, nb > 1, acc, scratch_bytes));
   char* XcT = scratch;
   uint32_t* queue = reinterpret_cast<uint32_t*>(scratch + align_up((size_t)H * C * 2));
   float* one = reinterpret_cast<float*>(queue + kQueueWords);
@@ -1531,9 +1552,11 @@ int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, 
                                            align_up((kQueueWords + 1) * sizeof(uint32_t)));
   // one upstream scalar for every token: G is formed for a unit gradient and
   // the scalar applied to the fp32 sums of dX and dW, so that its own rounding
-  // to bf16 does not enter G; a per-token gradient is part of G
-  const float* out_scale = gstride == 0 ? grad : nullptr;
-  const float* g = gstride == 0 ? one : grad;
+  // to bf16 does not enter G; a per-token gradient, or one whose dW is added to
+  // others, is part of G
+  const bool unit = gstride == 0 && !acc;
+  const float* out_scale = unit ? grad : nullptr;
+  const float* g = unit ? one : grad;
   hipLaunchKernelGGL(gather_t_kernel<__bf16>, dim3((uint32_t)(C / 64), (uint32_t)cdiv(H, 64)),
                      dim3(256), 0, stream, static_cast<const char*>(X), ldx * 2, row_index, (int32_t)N,
                      (int32_t)H, XcT, ldxt_b, static_cast<const float*>(nullptr), queue,
@@ -1599,7 +1622,8 @@ int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, 
       x.split_stride = C * H;
     } else {
       x.mode = nb == 1 ? kDxEmit
-                       : kDxTiledAcc + (j == 0 ? kDxStore : (j == nb - 1 ? kDxAddEmit : kDxAdd));
+                       : (acc ? 0 : kDxTiledAcc) +
+                             (j == 0 ? kDxStore : (j == nb - 1 ? kDxAddEmit : kDxAdd));
     }
     x.out_scale = out_scale;
     x.dX = static_cast<char*>(dX);
@@ -1636,9 +1660,9 @@ int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, 
     w.cv = (int32_t)cv;
     w.v0 = (int32_t)v0;
     w.dW = static_cast<float*>(dW);
-    w.lddw = H;
-    w.accumulate = 0;
-    w.narrow = 1;
+    w.lddw = acc ? lddw_acc : H;
+    w.accumulate = acc ? 1 : 0;
+    w.narrow = acc ? 0 : 1;
     w.out_scale = out_scale;
     w.tiles_m = (int32_t)cdiv(cv, 256);
     w.tiles_n = x.tiles_n;
@@ -1873,7 +1897,7 @@ int backward_plan_entry(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dt
     return fail(MT_ERR_INVALID_ARGUMENT, "null output pointer");
   if (narrow && dtype != MT_DTYPE_BF16)
     return fail(MT_ERR_UNSUPPORTED, "the narrowing backward is bf16 only (dtype %d)", dtype);
-  const BwdPlan p = plan_backward(T, n_valid, H, V, es, budget_bytes, narrow);
+  const BwdPlan p = plan_backward(T, n_valid, H, V, es, budget_bytes, narrow, true);
   *chunk_rows = p.C;
   *chunk_vocab = p.Cv;
   *workspace_bytes = p.ws;
@@ -2094,9 +2118,30 @@ int mt_flce_backward_narrow(const void* X, const void* W, int64_t T, int64_t H, 
                         kept_guard, nullptr, scratch, scratch_bytes);
 }
 
+int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,
+                         size_t fused_budget, size_t general_budget, int* pays) {
+  if (dtype != MT_DTYPE_BF16)
+    return fail(MT_ERR_UNSUPPORTED, "the fused path is bf16 only (dtype %d)", dtype);
+  if (T < 0 || n_valid < 0 || n_valid > T || H <= 0 || V <= 0 || T > INT32_MAX || H > INT32_MAX ||
+      V > INT32_MAX)
+    return fail(MT_ERR_INVALID_ARGUMENT, "bad sizes T=%lld n_valid=%lld H=%lld V=%lld", (long long)T,
+                (long long)n_valid, (long long)H, (long long)V);
+  if (!pays) return fail(MT_ERR_INVALID_ARGUMENT, "null output pointer");
+  const FusedPlan f = plan_fused(T, n_valid, H, V, fused_budget);
+  const BwdPlan b = plan_backward(T, n_valid, H, V, 2, general_budget, true, true);
+  *pays = 0;
+  if (b.C && f.C) {
+    const bool one = b.C >= n_valid;
+    const double pass = (double)V * H * 6 / kBw + 10 * kLaunch;
+    *pays = forward_cost(n_valid, H, V) + backward_cost(n_valid, H, V, b.C, b.Cv, 2, one, true) +
+                (one ? 0.0 : pass) < 0.9 * (fused_cost(n_valid, H, V, f.C) + pass);
+  }
+  return MT_OK;
+}
+
 int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,
-                        size_t budget_bytes, int count_gradient, int64_t* keep_cols,
-                        size_t* logits_bytes, size_t* scratch_bytes, int* pays) {
+                        size_t budget_bytes, int count_gradient, int with_accumulator,
+                        int64_t* keep_cols, size_t* logits_bytes, size_t* scratch_bytes, int* pays) {
   if (dtype != MT_DTYPE_BF16)
     return fail(MT_ERR_UNSUPPORTED, "keeping logits is bf16 only (dtype %d)", dtype);
   if (T < 0 || n_valid < 0 || n_valid > T || H <= 0 || V <= 0 || T > INT32_MAX || H > INT32_MAX ||
@@ -2105,7 +2150,8 @@ int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dt
                 (long long)n_valid, (long long)H, (long long)V);
   if (!keep_cols || !logits_bytes || !scratch_bytes || !pays)
     return fail(MT_ERR_INVALID_ARGUMENT, "null output pointer");
-  const KeptPlan p = plan_kept(T, n_valid, H, V, budget_bytes, count_gradient != 0);
+  const bool acc = with_accumulator != 0;
+  const KeptPlan p = plan_kept(T, n_valid, H, V, budget_bytes, count_gradient != 0 && !acc, acc);
   *keep_cols = p.cols;
   *logits_bytes = p.logits;
   *scratch_bytes = p.scratch;
@@ -2114,8 +2160,9 @@ int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dt
     const FusedPlan f = plan_fused(T, n_valid, H, V, budget_bytes);
     // (the dearer estimate last: it searches the general path's blockings)
     *pays = p.cols >= V ||
-            ((!f.C || p.cost < 0.97 * (fused_cost(n_valid, H, V, f.C) + (double)V * H * 6 / kBw)) &&
-             p.cost < 0.97 * general_cost(T, n_valid, H, V, budget_bytes, true));
+            ((!f.C ||
+              p.cost < 0.97 * (fused_cost(n_valid, H, V, f.C) + (acc ? 0.0 : (double)V * H * 6 / kBw))) &&
+             p.cost < 0.97 * general_cost(T, n_valid, H, V, budget_bytes, !acc));
   }
   return MT_OK;
 }
@@ -2185,9 +2232,9 @@ int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, 
                             int64_t ldx, int64_t ldw, int dtype, float softcap,
                             const int32_t* row_index, const int32_t* row_label, int64_t n_valid,
                             const float* lse, const float* grad_loss, int64_t grad_stride, void* dX,
-                            int64_t lddx, void* dW_out, size_t dw_out_bytes, void* logits,
-                            int64_t keep_cols, size_t logits_bytes, void* scratch,
-                            size_t scratch_bytes, mt_stream_t stream) {
+                            int64_t lddx, void* dW_out, size_t dw_out_bytes, float* dW_acc,
+                            int64_t lddw_acc, void* logits, int64_t keep_cols, size_t logits_bytes,
+                            void* scratch, size_t scratch_bytes, mt_stream_t stream) {
   if (dtype != MT_DTYPE_BF16)
     return fail(MT_ERR_UNSUPPORTED, "keeping logits is bf16 only (dtype %d)", dtype);
   MT_TRY(check_common(X, W, T, H, V, ldx, ldw, dtype, softcap));
@@ -2197,15 +2244,19 @@ int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, 
     return fail(MT_ERR_INVALID_ARGUMENT, "lddx=%lld must be >= H and a whole number of 16-byte chunks",
                 (long long)lddx);
   if (grad_stride < 0) return fail(MT_ERR_INVALID_ARGUMENT, "grad_stride must be >= 0");
-  if (!dW_out || dw_out_bytes < dw_lo_bytes(V, H))
+  if (dW_acc && (lddw_acc < H || (lddw_acc * 4) % 16 != 0))
+    return fail(MT_ERR_INVALID_ARGUMENT, "lddw=%lld must be >= H and a whole number of 16-byte chunks",
+                (long long)lddw_acc);
+  if (!dW_acc && (!dW_out || dw_out_bytes < dw_lo_bytes(V, H)))
     return fail(MT_ERR_INVALID_ARGUMENT, "dW_out %zu bytes < V H 2 = %zu", dw_out_bytes, dw_lo_bytes(V, H));
   if (!dX || !row_index || !row_label || !lse || !grad_loss)
     return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
-  if ((reinterpret_cast<uintptr_t>(dX) | reinterpret_cast<uintptr_t>(dW_out) |
+  void* const dW = dW_acc ? static_cast<void*>(dW_acc) : dW_out;
+  if ((reinterpret_cast<uintptr_t>(dX) | reinterpret_cast<uintptr_t>(dW) |
        reinterpret_cast<uintptr_t>(scratch)) % 16 != 0)
-    return fail(MT_ERR_INVALID_ARGUMENT, "dX, dW_out and scratch must be 16-byte aligned");
+    return fail(MT_ERR_INVALID_ARGUMENT, "dX, dW and scratch must be 16-byte aligned");
   MT_TRY(logits_args(n_valid, H, V, ldw, logits, keep_cols, logits_bytes));
-  const size_t need = kept_scratch(round_up(n_valid, 256), H, 1, keep_cols < V);
+  const size_t need = kept_scratch(round_up(n_valid, 256), H, 1, keep_cols < V, dW_acc != nullptr);
   if (!scratch || scratch_bytes < need)
     return fail(MT_ERR_WORKSPACE_TOO_SMALL, "logits scratch %zu bytes < required %zu", scratch_bytes, need);
   hipStream_t s = (hipStream_t)stream;
@@ -2215,8 +2266,8 @@ int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, 
     MT_TRY(check_launch("zero_rows_kernel"));
   }
   return launch_backward_logits(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
-                                grad_loss, grad_stride, dX, lddx, dW_out, static_cast<char*>(logits),
-                                keep_cols, static_cast<char*>(scratch), scratch_bytes, s);
+                                grad_loss, grad_stride, dX, lddx, dW, dW_acc ? lddw_acc : 0,
+                                static_cast<char*>(logits), keep_cols, static_cast<char*>(scratch), scratch_bytes, s);
 }
 
 int mt_flce_fused_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,

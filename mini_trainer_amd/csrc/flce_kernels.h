@@ -846,10 +846,17 @@ __global__ __launch_bounds__(256) void ce_backward_kernel(const char* logits, in
   const char* row = logits + t * ld_b;
   char* drow = dlogits + t * ldd_b;
   constexpr int VEC = 16 / E;
-  if (((reinterpret_cast<uintptr_t>(row) | reinterpret_cast<uintptr_t>(drow)) & 15u) == 0) {
-    // 16-byte rows (the usual case): whole vectors, four loads in flight per
-    // thread, then the scalar tail of V mod VEC
-    const int64_t nvec = V / VEC;
+  if (((reinterpret_cast<uintptr_t>(row) ^ reinterpret_cast<uintptr_t>(drow)) & 15u) == 0) {
+    // logits and gradient row alike within 16 bytes (the usual case: the same
+    // pitch, also an odd one): up to VEC - 1 elements one by one to the next
+    // 16-byte boundary, whole vectors with four loads in flight per thread,
+    // then the rest of the row.  (An odd row went two elements at a time: 46 us
+    // for 1000 x 32003 bf16, 1.4 times its bytes' time at copy rate now.)
+    const int64_t mis = (int64_t)(reinterpret_cast<uintptr_t>(row) & 15u) / E;
+    const int64_t head = mis ? min<int64_t>(VEC - mis, V) : 0;
+    const int64_t nvec = (V - head) / VEC;
+    const char* vrow = row + head * E;
+    char* vdrow = drow + head * E;
     auto grad_vec = [&](float (&x)[VEC], int64_t c0) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
@@ -857,39 +864,41 @@ __global__ __launch_bounds__(256) void ce_backward_kernel(const char* logits, in
         x[j] = valid ? g * (p - (c0 + j == y ? 1.f : 0.f)) : 0.f;
       }
     };
-    int64_t i = threadIdx.x;
-    for (; i + 3 * 256 < nvec; i += 4 * 256) {
-      float x[4][VEC];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (valid) load_vec<T>(row + (i + k * 256) * 16, x[k]);
-        else
-#pragma unroll
-          for (int j = 0; j < VEC; ++j) x[k][j] = 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        grad_vec(x[k], (i + k * 256) * VEC);
-        store_vec<T>(drow + (i + k * 256) * 16, x[k]);
-      }
-    }
-    for (; i < nvec; i += 256) {
-      float x[VEC];
-      if (valid) load_vec<T>(row + i * 16, x);
-      else
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) x[j] = 0.f;
-      grad_vec(x, i * VEC);
-      store_vec<T>(drow + i * 16, x);
-    }
-    for (int64_t c = nvec * VEC + threadIdx.x; c < V; c += 256) {
+    auto grad_one = [&](int64_t c) __attribute__((always_inline)) {
       float r = 0.f;
       if (valid) r = g * (fast_exp2(fmaf(load_one<T>(row + c * E), kLog2e, -l2)) - (c == y ? 1.f : 0.f));
       if constexpr (E == 4)
         reinterpret_cast<float*>(drow)[c] = r;
       else
         *reinterpret_cast<uint16_t*>(drow + c * 2) = (uint16_t)(pack_bf16x2(r, 0.f) & 0xffffu);
+    };
+    int64_t i = threadIdx.x;
+    for (; i + 3 * 256 < nvec; i += 4 * 256) {
+      float x[4][VEC];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (valid) load_vec<T>(vrow + (i + k * 256) * 16, x[k]);
+        else
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) x[k][j] = 0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        grad_vec(x[k], head + (i + k * 256) * VEC);
+        store_vec<T>(vdrow + (i + k * 256) * 16, x[k]);
+      }
     }
+    for (; i < nvec; i += 256) {
+      float x[VEC];
+      if (valid) load_vec<T>(vrow + i * 16, x);
+      else
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) x[j] = 0.f;
+      grad_vec(x, head + i * VEC);
+      store_vec<T>(vdrow + i * 16, x);
+    }
+    if ((int64_t)threadIdx.x < head) grad_one(threadIdx.x);
+    for (int64_t c = head + nvec * VEC + threadIdx.x; c < V; c += 256) grad_one(c);
     return;
   }
   // any alignment: pairs of elements so bf16 rows are written 4 bytes at a time

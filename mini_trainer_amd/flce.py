@@ -123,10 +123,11 @@ def backward_plan(T: int, n_valid: int, H: int, V: int, dtype: torch.dtype,
     return c.value, cv.value, ws.value
 
 
-# The least default workspace: 5% of the logits of a short call is less than
-# one block of whole tiles for every CU needs (a 300-token fp32 call ran 14
-# vocabulary blocks of 256 columns), and 32 MiB is 0.01% of the device memory.
-MIN_BUDGET = 32 << 20
+# The least default workspace by element size: 5% of a short call's logits, or of
+# a small vocabulary's, holds only blocks that leave most CUs idle (18609 x 7552
+# x 6305 ran 25.8 ms in 12 MB), while these are 0.07% and 0.02% of the device
+# memory.
+MIN_BUDGET = {2: 192 << 20, 4: 56 << 20}
 
 
 def _default_budget(T: int, V: int, es: int) -> int:
@@ -134,21 +135,33 @@ def _default_budget(T: int, V: int, es: int) -> int:
     MT_FLCE_BWD_BUDGET_BYTES, else 5% of the T x V logits in bytes, at least
     MIN_BUDGET."""
     env = int(os.environ.get(BACKWARD_BUDGET_ENV, "0"))
-    return env if env > 0 else max(int(float(T) * V * es * 0.05), MIN_BUDGET)
+    return env if env > 0 else max(int(float(T) * V * es * 0.05), MIN_BUDGET[es])
 
 
-def _kept_plan(T: int, n: int, H: int, V: int) -> Tuple[int, int, int, bool]:
+def _kept_plan(T: int, n: int, H: int, V: int,
+               accumulator: bool = False) -> Tuple[int, int, int, bool]:
     """(columns, logits bytes, backward scratch bytes, pays) of a bf16 call
     that keeps logits from the forward to the backward (mt_flce_logits_plan),
     columns 0 when none fit.  The default budget counts the bytes by which a
-    bf16 weight gradient is smaller than the fp32 one of the other paths; a
-    budget set by MT_FLCE_BWD_BUDGET_BYTES is taken as it stands."""
+    bf16 weight gradient is smaller than the fp32 one of the other paths (no
+    such gradient exists with an accumulator); a budget set by MT_FLCE_BWD_BUDGET_BYTES is taken as it stands."""
     room = int(int(os.environ.get(BACKWARD_BUDGET_ENV, "0")) == 0)
     cols, lb, sb, pays = ctypes.c_int64(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int()
     check(load().mt_flce_logits_plan(T, n, H, V, MT_DTYPE_BF16, _default_budget(T, V, 2), room,
-                                     ctypes.byref(cols), ctypes.byref(lb), ctypes.byref(sb),
+                                     int(accumulator), ctypes.byref(cols), ctypes.byref(lb), ctypes.byref(sb),
                                      ctypes.byref(pays)), "mt_flce_logits_plan")
     return cols.value, lb.value, sb.value, bool(pays.value)
+
+
+def _general_pays(T: int, n: int, H: int, V: int) -> bool:
+    """Is the general path in the default budget expected to beat the fused
+    one at 5% of the logits (mt_flce_general_pays)?"""
+    pays = ctypes.c_int()
+    check(load().mt_flce_general_pays(T, n, H, V, MT_DTYPE_BF16,
+                                      int(os.environ.get(BACKWARD_BUDGET_ENV, "0")),
+                                      _default_budget(T, V, 2), ctypes.byref(pays)),
+          "mt_flce_general_pays")
+    return bool(pays.value)
 
 
 def _grad_vector(grad: torch.Tensor, T: int) -> Tuple[torch.Tensor, int]:
@@ -264,7 +277,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, hidden, weight, target, ignore_index, softcap, shift, dw_accumulator,
-                grad_scale, allow_unit, ranges):
+                grad_scale, allow_unit, recording, ranges):
         X, W, T, H, V, dt = _check_inputs(hidden, weight, target)
         lib = load()
         dev = X.device
@@ -282,20 +295,35 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         ctx.keep = ctx.logits = None
         plans = None
         kept = None
-        if (dt == MT_DTYPE_BF16 and allow_unit and grad_scale is None and len(parts) == 1
-                and n_tot > 0 and _fused_mode() == "auto"):
+        acc = dw_accumulator is not None
+        keep = (dt == MT_DTYPE_BF16 and len(parts) == 1 and n_tot > 0
+                and _fused_mode() == "auto")
+        if keep and allow_unit and grad_scale is None:
             kept = _kept_plan(T, n_tot, H, V)
             kept = kept if kept[3] else None
         if kept is None and dt == MT_DTYPE_BF16 and n_tot > 0 and (grad_scale is not None or allow_unit):
-            # planned at 5% of the logits, also where MIN_BUDGET gives a short
-            # call more: the general path's blocks grow with it, and its dX
-            # carries one rounding less than the fused path's
-            plans = [fused_plan(t1 - t0, n, H, V, accumulator=dw_accumulator is not None)
-                     if n > 0 else (0, 0, True) for t0, t1, _, _, n in parts]
+            # whether it pays is asked at 5% of the logits, also where
+            # MIN_BUDGET gives more: the general path's blocks grow with it,
+            # and its dX carries one rounding less than the fused path's
+            plans = [fused_plan(t1 - t0, n, H, V, accumulator=acc) if n > 0 else (0, 0, True)
+                     for t0, t1, _, _, n in parts]
             live = [pl for pl, p in zip(plans, parts) if p[4] > 0]
             # C = 0: the fused path cannot run that shape
             if all(pl[0] > 0 for pl in live) and _use_fused(all(pl[2] for pl in live)):
                 ctx.path = "fused" if grad_scale is not None else "fused_unit"
+                if T * V * 0.1 < MIN_BUDGET[2]:
+                    # a short call, or a small vocabulary: chunks that fit
+                    # MIN_BUDGET for the promised path; the unit one holds the
+                    # fp32 weight gradient besides and keeps to 5%, unless the
+                    # general path in MIN_BUDGET is the faster
+                    if ctx.path == "fused":
+                        plans = [fused_plan(t1 - t0, n, H, V, _default_budget(t1 - t0, V, 2), acc)
+                                 if n > 0 else (0, 0, True) for t0, t1, _, _, n in parts]
+                    elif keep and _general_pays(T, n_tot, H, V):
+                        ctx.path = "general"
+        if keep and acc and recording and ctx.path == "general":
+            kept = _kept_plan(T, n_tot, H, V, True)
+            kept = kept if kept[3] else None
         ctx.dw_accumulator = dw_accumulator
         ctx.meta = (float(softcap), hidden.shape, dt)
         lses = []
@@ -409,7 +437,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         softcap, hshape, dt = ctx.meta
         need_x, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         acc = ctx.dw_accumulator
-        none = (None,) * 8
+        none = (None,) * 9
         if not need_x and not need_w and acc is None:
             return (None, None) + none
         lib = load()
@@ -423,12 +451,13 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             # the first backward: G from the logits its forward kept
             (t0, t1, n, ri, rl, lse), (kept, cols, scratch_bytes) = rngs[0], logits
             scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
-            out = torch.empty((V, H), dtype=torch.bfloat16, device=dev)
+            out = None if acc is not None else torch.empty((V, H), dtype=torch.bfloat16, device=dev)
             check(lib.mt_flce_backward_logits(_p(X), _p(W), T, H, V, X.stride(0), W.stride(0), dt,
                                               softcap, _p(ri), _p(rl), n, _p(lse), _p(g), gstride,
-                                              _p(dX), dX.stride(0), _p(out), out.numel() * 2,
-                                              _p(kept), cols, kept.numel(), _p(scratch),
-                                              scratch_bytes, _stream(dev)),
+                                              _p(dX), dX.stride(0), _p(out), V * H * 2, _p(acc),
+                                              acc.stride(0) if acc is not None else 0, _p(kept),
+                                              cols, kept.numel(), _p(scratch), scratch_bytes,
+                                              _stream(dev)),
                   "mt_flce_backward_logits")
             del kept, scratch, logits
             grad_w = out if need_w else None
@@ -494,7 +523,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         grad_w = None
         if ctx.needs_input_grad[1] and dW is not None:
             grad_w = dW.narrow(torch.ones(1, dtype=torch.float32, device=dX.device))
-        return (grad_x, grad_w) + (None,) * 8
+        return (grad_x, grad_w) + (None,) * 9
 
     @staticmethod
     def _backward_fused_unit(ctx, grad_loss):
@@ -530,7 +559,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             dW_out = _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX, dW)
         grad_x = dX.view(hshape) if need_x else None
         grad_w = dW_out if need_w else None
-        return (grad_x, grad_w) + (None,) * 8
+        return (grad_x, grad_w) + (None,) * 9
 
 
 def _narrowed_view(dW: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
@@ -790,7 +819,8 @@ def fused_linear_cross_entropy(hidden_states: torch.Tensor, lm_head_weight: torc
             ranges = [(t0, min(T, t0 + rows)) for t0 in range(0, T, rows)]
     return _FusedLinearCrossEntropyNone.apply(hidden_states, lm_head_weight, target,
                                               int(ignore_index), cap, bool(shift_labels),
-                                              dw_accumulator, grad_scale, allow_unit, ranges)
+                                              dw_accumulator, grad_scale, allow_unit,
+                                              recording, ranges)
 
 
 class _CrossEntropyNone(torch.autograd.Function):

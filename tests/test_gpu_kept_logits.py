@@ -111,6 +111,57 @@ def test_kept_logits_host_checks():
         Hp, vt = -(-H // 256) * 256, -(-V // 256)
         room = Hp * 512 + vt * 256 * Hp * 4 - V * H * 2
         assert pays and cols == vt * 256 and lb >= -(-n // 256) * 256 * cols * 2
-        assert lb + sb <= max(0.05 * T * V * 2, 32 << 20) + room + 512
+        assert lb + sb <= max(0.05 * T * V * 2, 192 << 20) + room + 512
     cols, _, _, pays = _kept_plan(65536, 45875, 4096, 128256)
     assert cols < 128256 and not pays
+
+
+@pytest.mark.parametrize("T,H,V,cols,slices", [
+    (3, 64, 700, 0, 0),           # all kept, several dX slices
+    (700, 520, 5000, 0, 0),
+    (700, 1024, 66000, 0, 0),     # the dW work queue
+    (300, 136, 5000, 1024, 1),    # blocks after the kept one, one dX accumulator
+    (520, 264, 12500, 6144, 8),   # the same with dX slices in planes
+])
+def test_kept_logits_into_accumulator(gpu, monkeypatch, T, H, V, cols, slices):
+    """dW added into an fp32 accumulator that holds other values already,
+    against the recomputing backward into an empty one: the same G in both, so
+    only the order of the fp32 sums differs (sqrt(V) 2^-24 of dX before its
+    rounding, at most 2^-11 after; sqrt(T) 2^-24 of dW, 2^-18)."""
+    import mini_trainer_amd.flce as flce
+
+    X, W, y, grad = _inputs(T, H, V, 0.1)
+    n = int((y != -100).sum())
+    if cols:
+        C, al = -(-n // 256) * 256, lambda b: -(-b // 256) * 256  # noqa: E731
+        monkeypatch.setenv(flce.BACKWARD_BUDGET_ENV,
+                           str(C * cols * 2 + al(H * C * 2) + 256 + al(slices * C * H * 4)))
+    kept = flce._kept_plan(T, n, H, V, True)
+    assert kept[0] >= V if not cols else 0 < kept[0] < V
+    plan = flce._kept_plan
+    start = torch.randn(V, H, generator=torch.Generator().manual_seed(1)).to(gpu)
+
+    def run(keep, acc):
+        monkeypatch.setattr(flce, "_kept_plan", lambda *a: plan(*a)[:3] + (keep,))
+        Xd, Wd = X.to(gpu).requires_grad_(True), W.to(gpu).requires_grad_(True)
+        loss = fused_linear_cross_entropy(Xd, Wd, y.to(gpu), dw_accumulator=acc)
+        (loss * grad.to(gpu)).sum().backward()
+        assert Wd.grad is None
+        return loss, Xd.grad
+
+    acc, acc0 = start.clone(), torch.zeros(V, H, device=gpu)
+    profile_enable(True)
+    try:
+        loss, dX = run(True, acc)
+        torch.cuda.synchronize()
+    finally:
+        profile_enable(False)
+    rep = profile_report()
+    assert "fwd_bf16_kernel<store_logits>" in rep
+    assert ("recompute_bf16_kernel" in rep) == bool(cols)
+    loss0, dX0 = run(False, acc0)
+    assert torch.equal(loss, loss0)
+    assert _rel(dX, dX0) <= 2.0 ** -11
+    # acc - start loses 2^-24 of the start's size
+    assert float(((acc.double() - start.double()) - acc0.double()).norm()) <= \
+        2.0 ** -18 * float(acc0.double().norm()) + 2.0 ** -24 * float(start.double().norm())
