@@ -553,6 +553,20 @@ int mt_ce_forward(const void* logits, int64_t T, int64_t V, int64_t ld, int dtyp
                   const int64_t* target, int64_t ignore_index, float* loss, float* lse,
                   int32_t* status, mt_stream_t stream);
 
+/*
+ * The same in two steps, for a caller that must know whether every target is
+ * in range but need not wait for the logits to be read: mt_ce_check_targets
+ * raises *status (int32 [1], device or host-pinned memory that the caller has
+ * set to 0) if some target is neither ignore_index nor in [0, V), and
+ * mt_ce_forward_checked is mt_ce_forward without a status (such a row gets
+ * loss 0).  The caller waits for an event recorded between the two.
+ */
+int mt_ce_check_targets(const int64_t* target, int64_t T, int64_t V, int64_t ignore_index,
+                        int32_t* status, mt_stream_t stream);
+int mt_ce_forward_checked(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,
+                          const int64_t* target, int64_t ignore_index, float* loss, float* lse,
+                          mt_stream_t stream);
+
 /* dlogits[t, v] = g_t * (softmax(logits_t)[v] - [v == y_t]), 0 on ignored rows;
  * written in the logits dtype with leading dimension ldd. */
 int mt_ce_backward(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,

@@ -249,6 +249,13 @@ int check_common(const void* X, const void* W, int64_t T, int64_t H, int64_t V, 
   return MT_OK;
 }
 
+// loss[rows[i]] = +0.0 for i < n (a call without counted rows).
+int zero_loss(float* loss, const int32_t* rows, int64_t n, hipStream_t s) {
+  hipLaunchKernelGGL(zero_scatter_f32_kernel, dim3((uint32_t)std::min<int64_t>(cdiv(n, 256), 4096)),
+                     dim3(256), 0, s, loss, rows, n);
+  return check_launch("zero_scatter_f32_kernel");
+}
+
 // Vocabulary rows per block of a bf16 weight (a multiple of 256 whose rows
 // fit one buffer's reach; V itself when the whole weight does).
 int64_t vocab_block_rows(int64_t V, int64_t ldw) {
@@ -668,7 +675,7 @@ template <typename T>
 int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V, int64_t ldx,
                    int64_t ldw, float softcap, const int32_t* row_index, const int32_t* row_label,
                    int64_t n_valid, float* loss, float* lse, const FwdPlan& p, char* ws,
-                   hipStream_t stream, char* keep = nullptr, int64_t keep_cols = 0,
+                   hipStream_t stream, int64_t n_ignored = 0, char* keep = nullptr, int64_t keep_cols = 0,
                    int32_t* guard = nullptr, char* logits = nullptr) {
   constexpr int es = sizeof(T);
   FwdArgs a;
@@ -750,8 +757,9 @@ int launch_forward(const void* X, const void* W, int64_t Tn, int64_t H, int64_t 
     prof_end(pf, stream);
     MT_TRY(check_launch("fwd_f32_kernel"));
   }
-  hipLaunchKernelGGL(fwd_finalize_kernel, dim3((uint32_t)cdiv(n_valid, 4)), dim3(256), 0, stream,
-                     a.part, a.xy, a.N, a.splits, row_index, loss, lse, guard);
+  hipLaunchKernelGGL(fwd_finalize_kernel, dim3((uint32_t)(cdiv(n_valid, 4) + cdiv(n_ignored, 256))),
+                     dim3(256), 0, stream, a.part, a.xy, a.N, a.splits, row_index, loss, lse, guard,
+                     (int32_t)n_ignored);
   return check_launch("fwd_finalize_kernel");
 }
 
@@ -1557,24 +1565,42 @@ int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, 
   const bool unit = gstride == 0 && !acc;
   const float* out_scale = unit ? grad : nullptr;
   const float* g = unit ? one : grad;
-  hipLaunchKernelGGL(gather_t_kernel<__bf16>, dim3((uint32_t)(C / 64), (uint32_t)cdiv(H, 64)),
-                     dim3(256), 0, stream, static_cast<const char*>(X), ldx * 2, row_index, (int32_t)N,
-                     (int32_t)H, XcT, ldxt_b, static_cast<const float*>(nullptr), queue,
-                     (int32_t)kQueueWords, one);
-  MT_TRY(check_launch("gather_t_kernel"));
+  KeptGradArgs k;
+  k.S = logits;
+  k.lds_b = ldg_b;
+  k.cols = (int32_t)cols;
+  k.cn = (int32_t)N;
+  k.V = (int32_t)std::min(cols, V);
+  k.rows = (int32_t)round_up(N, 64);
+  k.lse = lse;
+  k.grad = unit ? nullptr : grad;
+  k.gstride = gstride;
+  k.row_index = row_index;
+  k.row_label = row_label;
+  k.softcap = softcap;
+  k.X = static_cast<const char*>(X);
+  k.ldx_b = ldx * 2;
+  k.H = (int32_t)H;
+  k.gather_m = (int32_t)(C / 64);
+  k.XcT = XcT;
+  k.ldxt_b = ldxt_b;
+  k.zero_words = queue;
+  k.n_zero = (int32_t)kQueueWords;
+  k.one = one;
+  k.dX = static_cast<char*>(dX);
+  k.lddx_b = lddx * 2;
+  k.n_ignored = (int32_t)(Tn - N);
+  const int ps = prof_begin("kept_grad_kernel", 0, 2.0 * k.rows * cols * 2, stream);
+  hipLaunchKernelGGL(softcap > 0.f ? kept_grad_kernel<true> : kept_grad_kernel<false>,
+                     dim3((uint32_t)(k.rows + k.gather_m * cdiv(H, 64) + std::min<int64_t>(Tn - N, 1024))),
+                     dim3(256), 0, stream, k);
+  prof_end(ps, stream);
+  MT_TRY(check_launch("kept_grad_kernel"));
   for (int64_t v0 = 0, j = 0; v0 < V; v0 += cols, ++j) {
     const int64_t cv = std::min(cols, V - v0);
     const char* Wv = static_cast<const char*>(W) + v0 * ldw * 2;
     const uint32_t g_range = range_of(C, ldg_b), w_range = range_of(cv, ldw * 2);
-    if (j == 0) {
-      const int ps = prof_begin("softmax_grad_kernel", 0, 2.0 * C * cols * 2, stream);
-      hipLaunchKernelGGL(softcap > 0.f ? softmax_grad_kernel<true> : softmax_grad_kernel<false>,
-                         dim3((uint32_t)C), dim3(256), 0, stream, logits, ldg_b, (int32_t)cols,
-                         (int32_t)N, (int32_t)cv, lse, g, gstride, row_index, row_label, softcap,
-                         static_cast<const int32_t*>(nullptr));
-      prof_end(ps, stream);
-      MT_TRY(check_launch("softmax_grad_kernel"));
-    } else {
+    if (j > 0) {
       RecompArgs r;
       r.X = static_cast<const char*>(X);
       r.W = Wv;
@@ -1718,18 +1744,12 @@ int mt_flce_forward(const void* X, const void* W, int64_t T, int64_t H, int64_t 
   if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(MT_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  if (T - n_valid > 0) {
-    const int64_t n0 = T - n_valid;
-    hipLaunchKernelGGL(zero_scatter_f32_kernel, dim3((uint32_t)std::min<int64_t>(cdiv(n0, 256), 4096)),
-                       dim3(256), 0, s, loss, row_index + n_valid, n0);
-    MT_TRY(check_launch("zero_scatter_f32_kernel"));
-  }
-  if (n_valid == 0) return MT_OK;
+  if (n_valid == 0) return zero_loss(loss, row_index, T, s);
   if (dtype == MT_DTYPE_BF16)
     return launch_forward<__bf16>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid,
-                                  loss, lse, p, static_cast<char*>(workspace), s);
+                                  loss, lse, p, static_cast<char*>(workspace), s, T - n_valid);
   return launch_forward<float>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, loss,
-                               lse, p, static_cast<char*>(workspace), s);
+                               lse, p, static_cast<char*>(workspace), s, T - n_valid);
 }
 
 int mt_flce_forward_keep(const void* X, const void* W, int64_t T, int64_t H, int64_t V,
@@ -1770,15 +1790,9 @@ int mt_flce_forward_keep(const void* X, const void* W, int64_t T, int64_t H, int
   if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(MT_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
   hipStream_t s = (hipStream_t)stream;
-  if (T - n_valid > 0) {
-    const int64_t n0 = T - n_valid;
-    hipLaunchKernelGGL(zero_scatter_f32_kernel, dim3((uint32_t)std::min<int64_t>(cdiv(n0, 256), 4096)),
-                       dim3(256), 0, s, loss, row_index + n_valid, n0);
-    MT_TRY(check_launch("zero_scatter_f32_kernel"));
-  }
-  if (n_valid == 0) return MT_OK;
+  if (n_valid == 0) return zero_loss(loss, row_index, T, s);
   return launch_forward<__bf16>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid,
-                                loss, lse, p, static_cast<char*>(workspace), s,
+                                loss, lse, p, static_cast<char*>(workspace), s, T - n_valid,
                                 static_cast<char*>(keep), keep_cols, guard);
 }
 
@@ -2216,16 +2230,10 @@ int mt_flce_forward_logits(const void* X, const void* W, int64_t T, int64_t H, i
     return fail(MT_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
   if (n_valid > 0) MT_TRY(logits_args(n_valid, H, V, ldw, logits, keep_cols, logits_bytes));
   hipStream_t s = (hipStream_t)stream;
-  if (T - n_valid > 0) {
-    const int64_t n0 = T - n_valid;
-    hipLaunchKernelGGL(zero_scatter_f32_kernel, dim3((uint32_t)std::min<int64_t>(cdiv(n0, 256), 4096)),
-                       dim3(256), 0, s, loss, row_index + n_valid, n0);
-    MT_TRY(check_launch("zero_scatter_f32_kernel"));
-  }
-  if (n_valid == 0) return MT_OK;
+  if (n_valid == 0) return zero_loss(loss, row_index, T, s);
   return launch_forward<__bf16>(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid,
-                                loss, lse, p, static_cast<char*>(workspace), s, nullptr, keep_cols,
-                                nullptr, static_cast<char*>(logits));
+                                loss, lse, p, static_cast<char*>(workspace), s, T - n_valid, nullptr,
+                                keep_cols, nullptr, static_cast<char*>(logits));
 }
 
 int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, int64_t V,
@@ -2260,11 +2268,6 @@ int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, 
   if (!scratch || scratch_bytes < need)
     return fail(MT_ERR_WORKSPACE_TOO_SMALL, "logits scratch %zu bytes < required %zu", scratch_bytes, need);
   hipStream_t s = (hipStream_t)stream;
-  if (T - n_valid > 0) {
-    hipLaunchKernelGGL(zero_rows_kernel, dim3((uint32_t)std::min<int64_t>(T - n_valid, 8192)), dim3(256),
-                       0, s, static_cast<char*>(dX), lddx * 2, row_index + n_valid, T - n_valid, H * 2);
-    MT_TRY(check_launch("zero_rows_kernel"));
-  }
   return launch_backward_logits(X, W, T, H, V, ldx, ldw, softcap, row_index, row_label, n_valid, lse,
                                 grad_loss, grad_stride, dX, lddx, dW, dW_acc ? lddw_acc : 0,
                                 static_cast<char*>(logits), keep_cols, static_cast<char*>(scratch), scratch_bytes, s);
@@ -2601,9 +2604,13 @@ int mt_flce_probe_mfma(int shape, int64_t workgroups, int32_t iters, const void*
   return check_launch("mfma_probe_kernel");
 }
 
-int mt_ce_forward(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,
-                  const int64_t* target, int64_t ignore_index, float* loss, float* lse,
-                  int32_t* status, mt_stream_t stream) {
+}  // extern "C"
+
+namespace {
+
+int ce_forward_entry(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,
+                     const int64_t* target, int64_t ignore_index, float* loss, float* lse,
+                     int32_t* status, bool checked, mt_stream_t stream) {
   const int es = esize_of(dtype);
   if (!es) return fail(MT_ERR_INVALID_ARGUMENT, "dtype %d is not MT_DTYPE_F32 or MT_DTYPE_BF16", dtype);
   if (T < 0 || T > INT32_MAX || V <= 0 || V > INT32_MAX || ld < V)
@@ -2611,20 +2618,47 @@ int mt_ce_forward(const void* logits, int64_t T, int64_t V, int64_t ld, int dtyp
                 (long long)ld);
   if (reinterpret_cast<uintptr_t>(logits) % es != 0)
     return fail(MT_ERR_INVALID_ARGUMENT, "logits must be aligned to its element size");
-  if (!status || (T > 0 && (!logits || !target || !loss || !lse)))
+  if ((!checked && !status) || (T > 0 && (!logits || !target || !loss || !lse)))
     return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(set_i32_kernel, dim3(1), dim3(1), 0, s, status, 0);
+  if (!checked) hipLaunchKernelGGL(set_i32_kernel, dim3(1), dim3(1), 0, s, status, 0);
   if (T == 0) return check_launch("set_i32_kernel");
-  if (dtype == MT_DTYPE_BF16)
-    hipLaunchKernelGGL(ce_forward_kernel<__bf16>, dim3((uint32_t)T), dim3(256), 0, s,
-                       static_cast<const char*>(logits), V, ld * es, target, ignore_index, loss, lse,
-                       status);
-  else
-    hipLaunchKernelGGL(ce_forward_kernel<float>, dim3((uint32_t)T), dim3(256), 0, s,
-                       static_cast<const char*>(logits), V, ld * es, target, ignore_index, loss, lse,
-                       status);
+  const bool nt = (double)T * V * es > 256e6;  // beyond the Infinity Cache (ce_forward_kernel)
+  static void (*const kern[2][2])(const char*, int64_t, int64_t, const int64_t*, int64_t, float*, float*,
+                                  int32_t*) = {
+      {ce_forward_kernel<float, false>, ce_forward_kernel<float, true>},
+      {ce_forward_kernel<__bf16, false>, ce_forward_kernel<__bf16, true>}};
+  hipLaunchKernelGGL(kern[dtype == MT_DTYPE_BF16][nt], dim3((uint32_t)T), dim3(256), 0, s,
+                     static_cast<const char*>(logits), V, ld * es, target, ignore_index, loss, lse,
+                     checked ? nullptr : status);
   return check_launch("ce_forward_kernel");
+}
+
+}  // namespace
+
+extern "C" {
+
+int mt_ce_forward(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,
+                  const int64_t* target, int64_t ignore_index, float* loss, float* lse,
+                  int32_t* status, mt_stream_t stream) {
+  return ce_forward_entry(logits, T, V, ld, dtype, target, ignore_index, loss, lse, status, false, stream);
+}
+
+int mt_ce_forward_checked(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,
+                          const int64_t* target, int64_t ignore_index, float* loss, float* lse,
+                          mt_stream_t stream) {
+  return ce_forward_entry(logits, T, V, ld, dtype, target, ignore_index, loss, lse, nullptr, true, stream);
+}
+
+int mt_ce_check_targets(const int64_t* target, int64_t T, int64_t V, int64_t ignore_index,
+                        int32_t* status, mt_stream_t stream) {
+  if (T < 0 || T > INT32_MAX || V <= 0 || V > INT32_MAX)
+    return fail(MT_ERR_INVALID_ARGUMENT, "bad sizes T=%lld V=%lld", (long long)T, (long long)V);
+  if (!status || (T > 0 && !target)) return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if (T == 0) return MT_OK;
+  hipLaunchKernelGGL(ce_check_kernel, dim3((uint32_t)cdiv(T, 256)), dim3(256), 0, (hipStream_t)stream,
+                     target, T, V, ignore_index, status);
+  return check_launch("ce_check_kernel");
 }
 
 int mt_ce_backward(const void* logits, int64_t T, int64_t V, int64_t ld, int dtype,

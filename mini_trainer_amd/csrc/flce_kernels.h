@@ -128,10 +128,20 @@ __device__ __forceinline__ void fwd_final_merge(char* lds, float (&m2)[8], float
 // (e^-87 is about the smallest), and at +48, lse <= 48 + ln V keeps the row
 // factor g exp(-lse) a normal fp32 number for g down to 1e-10 at V = 2^20.
 constexpr float kGuardLo = -48.f, kGuardHi = 48.f;
+// Rows N .. N + n_ignored of row_index (the last row block's caller passes the
+// ignored rows that follow the counted ones) get loss +0.0, by the grid's last
+// workgroups.
 __global__ __launch_bounds__(256) void fwd_finalize_kernel(const float* part, const float* xy,
                                                            int32_t N, int32_t splits,
                                                            const int32_t* row_index, float* loss,
-                                                           float* lse, int32_t* guard) {
+                                                           float* lse, int32_t* guard,
+                                                           int32_t n_ignored = 0) {
+  const uint32_t row_blocks = ((uint32_t)N + 3u) / 4u;
+  if (blockIdx.x >= row_blocks) {
+    const int32_t i = (int32_t)((blockIdx.x - row_blocks) * 256u + threadIdx.x);
+    if (i < n_ignored) loss[row_index[N + i]] = 0.0f;
+    return;
+  }
   const int32_t r = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (r >= N) return;  // uniform per wave
   const int lane = (int)(threadIdx.x & 63u);
@@ -370,23 +380,14 @@ constexpr int kDwRows = 0, kDwTiles = 1, kDwNarrow = 2;
 // 64 x 64 element tiles; 16-byte loads along h, 16-byte stores along t.
 // scale (non-null, bf16 only): row t is multiplied by scale[t] in fp32 and
 // rounded to bf16 (the fused path's per-row factor of G, see
-// fused_row_scale_kernel).  zero_words[0 .. n_zero) are cleared (the work
-// queue of a later launch) and *one, where given, set to 1.
+// fused_row_scale_kernel).
 template <typename T>
-__global__ __launch_bounds__(256) void gather_t_kernel(const char* X, int64_t ldx_b,
-                                                       const int32_t* row_index, int32_t Cn,
-                                                       int32_t H, char* XcT, int64_t ldxt_b,
-                                                       const float* scale = nullptr,
-                                                       uint32_t* zero_words = nullptr,
-                                                       int32_t n_zero = 0, float* one = nullptr) {
-  if (blockIdx.x == 0 && blockIdx.y == 0) {
-    if ((int32_t)threadIdx.x < n_zero) zero_words[threadIdx.x] = 0u;
-    if (one && threadIdx.x == 0) *one = 1.f;
-  }
+__device__ __forceinline__ void gather_t_tile(T (&tile)[64][64 + 1], int32_t t0, int32_t hb,
+                                              const char* X, int64_t ldx_b, const int32_t* row_index,
+                                              int32_t Cn, int32_t H, char* XcT, int64_t ldxt_b,
+                                              const float* scale) {
   constexpr int E = sizeof(T);
   constexpr int PER = 16 / E;  // elements per 16-byte vector
-  __shared__ T tile[64][64 + 1];
-  const int32_t t0 = blockIdx.x * 64, hb = blockIdx.y * 64;
   // load 64 rows (t) x 64 h
   for (int v = threadIdx.x; v < 64 * 64 / PER; v += 256) {
     const int tr = v / (64 / PER), hc = (v % (64 / PER)) * PER;
@@ -418,6 +419,16 @@ __global__ __launch_bounds__(256) void gather_t_kernel(const char* X, int64_t ld
     for (int j = 0; j < PER; ++j) e[j] = tile[tc + j][hr];
     *reinterpret_cast<u32x4_t*>(XcT + (int64_t)(hb + hr) * ldxt_b + (int64_t)(t0 + tc) * E) = val;
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void gather_t_kernel(const char* X, int64_t ldx_b,
+                                                       const int32_t* row_index, int32_t Cn,
+                                                       int32_t H, char* XcT, int64_t ldxt_b,
+                                                       const float* scale = nullptr) {
+  __shared__ T tile[64][64 + 1];
+  gather_t_tile<T>(tile, blockIdx.x * 64, blockIdx.y * 64, X, ldx_b, row_index, Cn, H, XcT, ldxt_b,
+                   scale);
 }
 
 // Zero `nrows` rows (ids from rows[]) of a row-major matrix, row_bytes each
@@ -749,6 +760,34 @@ __device__ __forceinline__ void store_vec(char* p, const float (&x)[16 / sizeof(
   }
 }
 
+// The same past the caches (data read once, larger than they hold).
+template <typename T>
+__device__ __forceinline__ void load_vec_nt(const char* p, float (&x)[16 / sizeof(T)]) {
+  const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+  if constexpr (sizeof(T) == 4) {
+    const f32x4_t f = __builtin_bit_cast(f32x4_t, v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = f[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t w = v[i];
+      x[2 * i] = __builtin_bit_cast(float, w << 16);
+      x[2 * i + 1] = __builtin_bit_cast(float, w & 0xffff0000u);
+    }
+  }
+}
+
+// *status = 1 (the caller has cleared it) if some target is neither ignore
+// nor in [0, V).
+__global__ __launch_bounds__(256) void ce_check_kernel(const int64_t* target, int64_t T, int64_t V,
+                                                       int64_t ignore, int32_t* status) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= T) return;
+  const int64_t y = target[t];
+  if (y != ignore && (y < 0 || y >= V)) *status = 1;
+}
+
 // Block-wide merge of per-thread (m, d) states; result valid in all threads.
 __device__ __forceinline__ void block_lse_merge(float& m, float& d, float* sm) {
 #pragma unroll
@@ -765,7 +804,13 @@ __device__ __forceinline__ void block_lse_merge(float& m, float& d, float* sm) {
   for (int i = 0; i < (int)(blockDim.x >> 6); ++i) lse_merge(m, d, sm[2 * i], sm[2 * i + 1]);
 }
 
-template <typename T>
+// HBM-bound: the logits of the counted rows are read once.  kNt: with loads
+// past the caches, for logits larger than the 256 MB Infinity Cache (2048 x
+// 151936 fp32 150 -> 137 us, 4096 x 128256 bf16 182 -> 160 us: 6.6 TB/s); smaller
+// ones may lie in it (1000 x 32003 bf16 12.9 against 13.6 us) and the backward
+// reads them again.  status null: the targets have been checked
+// (ce_check_kernel).
+template <typename T, bool kNt>
 __global__ __launch_bounds__(256) void ce_forward_kernel(const char* logits, int64_t V, int64_t ld_b,
                                                          const int64_t* target, int64_t ignore,
                                                          float* loss, float* lse, int32_t* status) {
@@ -782,7 +827,7 @@ __global__ __launch_bounds__(256) void ce_forward_kernel(const char* logits, int
   }
   if (y < 0 || y >= V) {
     if (threadIdx.x == 0) {
-      atomicOr(status, 1);
+      if (status) atomicOr(status, 1);
       loss[t] = 0.0f;
       lse[t] = 0.0f;
     }
@@ -811,7 +856,10 @@ __global__ __launch_bounds__(256) void ce_forward_kernel(const char* logits, int
   for (; i + 3 * 256 < nvec; i += 4 * 256) {
     float x[4][VEC];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) load_vec<T>(vrow + (i + k * 256) * 16, x[k]);
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (kNt) load_vec_nt<T>(vrow + (i + k * 256) * 16, x[k]);
+      else load_vec<T>(vrow + (i + k * 256) * 16, x[k]);
+    }
 #pragma unroll
     for (int k = 0; k < 4; ++k) merge_vec(x[k]);
   }

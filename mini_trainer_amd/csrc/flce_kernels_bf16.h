@@ -1213,19 +1213,14 @@ __global__ __launch_bounds__(256) void narrow_tiles_kernel(const float* scale, c
 // rows >= cn and columns >= V become 0.  HBM-bound: one 16-byte read and one
 // 16-byte write per 8 elements.
 template <bool kCap>
-__global__ __launch_bounds__(256) void softmax_grad_kernel(char* S, int64_t lds_b, int32_t cols,
-                                                           int32_t cn, int32_t V,
-                                                           const float* lse, const float* grad,
-                                                           int64_t gstride,
-                                                           const int32_t* row_index,
-                                                           const int32_t* row_label,
-                                                           float softcap,
-                                                           const int32_t* run_if) {
-  if (run_if && *run_if == 0) return;
-  const int32_t row = blockIdx.x;
+__device__ __forceinline__ void softmax_grad_row(int32_t row, char* S, int64_t lds_b, int32_t cols,
+                                                 int32_t cn, int32_t V, const float* lse,
+                                                 const float* grad, int64_t gstride,
+                                                 const int32_t* row_index, const int32_t* row_label,
+                                                 float softcap) {
   const bool rv = row < cn;
   const float lse2 = rv ? lse[row] * kLog2e : 0.f;
-  const float g = rv ? grad[(int64_t)row_index[row] * gstride] : 0.f;
+  const float g = !rv ? 0.f : (grad ? grad[(int64_t)row_index[row] * gstride] : 1.f);
   const int32_t y = rv ? row_label[row] : -1;
   const float inv_cap = kCap ? 1.0f / softcap : 0.f;
   u32x4_t* p = reinterpret_cast<u32x4_t*>(S + (int64_t)row * lds_b);
@@ -1263,6 +1258,78 @@ __global__ __launch_bounds__(256) void softmax_grad_kernel(char* S, int64_t lds_
     for (int k = 0; k < 4; ++k) p[(c + k * kStep) / 8] = grad8(v[k], c + k * kStep);
   }
   for (; c < cols; c += kStep) p[c / 8] = grad8(p[c / 8], c);
+}
+
+template <bool kCap>
+__global__ __launch_bounds__(256) void softmax_grad_kernel(char* S, int64_t lds_b, int32_t cols,
+                                                           int32_t cn, int32_t V,
+                                                           const float* lse, const float* grad,
+                                                           int64_t gstride,
+                                                           const int32_t* row_index,
+                                                           const int32_t* row_label,
+                                                           float softcap,
+                                                           const int32_t* run_if) {
+  if (run_if && *run_if == 0) return;
+  softmax_grad_row<kCap>((int32_t)blockIdx.x, S, lds_b, cols, cn, V, lse, grad, gstride, row_index,
+                         row_label, softcap);
+}
+
+// What the products of the kept-logits backward need first, in one launch (three
+// serial ones took 12 us of a 240-us call): workgroups [0, rows) turn
+// the logits of row b into G (rows a multiple of 64, as far as dW contracts;
+// dX discards the rows past cn), the next (C / 64) x ceil(H / 64) gather and
+// transpose X (XcT, see gather_t_tile), the others zero dX's ignored rows
+// (n_ignored row ids at row_index[cn ..], dx_row_bytes each).  Also clears
+// zero_words[0 .. n_zero) (the dW work queue) and sets *one to 1 (the unit
+// gradient of later recomputes).  grad null: a unit gradient.
+struct KeptGradArgs {
+  char* S;
+  int64_t lds_b;
+  int32_t cols, cn, V, rows;
+  const float* lse;
+  const float* grad;
+  int64_t gstride;
+  const int32_t* row_index;
+  const int32_t* row_label;
+  float softcap;
+  const char* X;
+  int64_t ldx_b;
+  int32_t H, gather_m;  // 64-row gather tiles: C / 64
+  char* XcT;
+  int64_t ldxt_b;
+  uint32_t* zero_words;
+  int32_t n_zero;
+  float* one;
+  char* dX;
+  int64_t lddx_b;
+  int32_t n_ignored;
+};
+template <bool kCap>
+__global__ __launch_bounds__(256) void kept_grad_kernel(KeptGradArgs a) {
+  __shared__ __bf16 tile[64][64 + 1];
+  if (blockIdx.x == 0) {
+    if ((int32_t)threadIdx.x < a.n_zero) a.zero_words[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) *a.one = 1.f;
+  }
+  int32_t b = (int32_t)blockIdx.x;
+  if (b < a.rows) {
+    softmax_grad_row<kCap>(b, a.S, a.lds_b, a.cols, a.cn, a.V, a.lse, a.grad, a.gstride, a.row_index,
+                           a.row_label, a.softcap);
+    return;
+  }
+  b -= a.rows;
+  const int32_t tiles = a.gather_m * ((a.H + 63) / 64);
+  if (b < tiles) {
+    gather_t_tile<__bf16>(tile, b % a.gather_m * 64, b / a.gather_m * 64, a.X, a.ldx_b, a.row_index,
+                          a.cn, a.H, a.XcT, a.ldxt_b, nullptr);
+    return;
+  }
+  const int32_t nb = (int32_t)gridDim.x - a.rows - tiles;
+  const int32_t nvec = a.H / 8;
+  for (int32_t r = b - tiles; r < a.n_ignored; r += nb) {
+    u32x4_t* p = reinterpret_cast<u32x4_t*>(a.dX + (int64_t)a.row_index[a.cn + r] * a.lddx_b);
+    for (int32_t v = (int32_t)threadIdx.x; v < nvec; v += 256) p[v] = u32x4_t{0u, 0u, 0u, 0u};
+  }
 }
 
 }  // namespace mtf

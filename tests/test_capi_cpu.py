@@ -404,3 +404,13 @@ def test_launch_failure_surfaces_as_flce_error(monkeypatch):
     monkeypatch.setenv("MT_FLCE_TEST_FAIL_LAUNCH", "prepare")
     rc = lib.mt_flce_prepare(p, 10, 100, -100, 0, p, p, p, None)
     assert rc == 4 and "injected launch failure" in lib.mt_flce_last_error().decode()
+
+
+def test_binding_declares_every_argument():
+    """Each ctypes signature has as many arguments as the header's declaration
+    (one too few is passed on as a 32-bit int)."""
+    text = re.sub(r"/\*.*?\*/", "", HEADER.read_text(), flags=re.S)
+    for name, (_, args) in _lib.SIGNATURES.items():
+        decl = re.search(r"\b" + name + r"\s*\(([^)]*)\)", text).group(1)
+        want = [a for a in decl.split(",") if a.strip() and a.strip() != "void"]
+        assert len(args) == len(want), name
