@@ -52,8 +52,10 @@ def _p(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None or t.numel() == 0 else t.data_ptr()
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    # the handle without a Stream object around it: 0.3 instead of 2 us, several
+    # times a call
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _require_device(name: str, t: torch.Tensor) -> None:
@@ -65,7 +67,7 @@ def _require_device(name: str, t: torch.Tensor) -> None:
 
 def _rows(t: torch.Tensor, name: str) -> torch.Tensor:
     """2-D view with unit stride along the last dim and a 16-byte row pitch."""
-    t2 = t.reshape(-1, t.shape[-1])
+    t2 = t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
     es = t2.element_size()
     if (t2.stride(1) != 1 or (t2.stride(0) * es) % 16 != 0 or t2.data_ptr() % 16 != 0
             or t2.stride(0) < t2.shape[1]):
@@ -84,14 +86,13 @@ def prepare_targets(target: torch.Tensor, vocab_size: int, ignore_index: int = -
     """
     _require_device("target", target)
     lib = load()
-    tgt = target.reshape(-1)
+    tgt = target if target.dim() == 1 else target.reshape(-1)
     if tgt.dtype != torch.int64:
         tgt = tgt.to(torch.int64)
     tgt = tgt.contiguous()
     T = tgt.numel()
     dev = tgt.device
-    row_index = torch.empty(T, dtype=torch.int32, device=dev)
-    row_label = torch.empty(T, dtype=torch.int32, device=dev)
+    row_index, row_label = torch.empty((2, T), dtype=torch.int32, device=dev).unbind(0)
     counts = torch.empty(4, dtype=torch.int32, device=dev)
     check(lib.mt_flce_prepare(_p(tgt), T, int(vocab_size), int(ignore_index), int(bool(shift)),
                               _p(row_index), _p(row_label), _p(counts), _stream(dev)),
@@ -286,7 +287,8 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             ranges = [(0, T)]
         parts = []  # (t0, t1, row_index, row_label, n) per range
         for t0, t1 in ranges:
-            ri, rl, n = prepare_targets(tgt[t0:t1], V, ignore_index, shift)
+            part = tgt if t1 - t0 == T else tgt[t0:t1]
+            ri, rl, n = prepare_targets(part, V, ignore_index, shift)
             parts.append((t0, t1, ri, rl, n))
         n_tot = sum(p[4] for p in parts)
         loss = torch.empty(T, dtype=torch.float32, device=dev)
@@ -370,7 +372,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         for t0, t1, ri, rl, n in parts:
             lse = torch.empty(n, dtype=torch.float32, device=dev)
             lses.append(lse)
-            Xr, lr = X[t0:t1], loss[t0:t1]
+            Xr, lr = (X, loss) if t1 - t0 == T else (X[t0:t1], loss[t0:t1])
             plan = None
             ws_bytes = lib.mt_flce_forward_workspace_bytes(t1 - t0, n, H, V, dt)
             if kept is not None:
@@ -500,11 +502,15 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             if n == 0:
                 continue
             if gl.stride(0) == 0 and gstride == 0:  # one scalar against one scalar
-                got, want = gl[:1].float(), g
+                # on the host, after one copy (fp32 differences of values this
+                # close are exact, so this is _within_promise's answer)
+                got, want = torch.cat([gl[:1].float(), g]).tolist()
+                kept = abs(got - want) <= abs(want) * (PROMISE_ULPS * 2.0 ** -23)
             else:
                 valid = ri[:n].long() + t0
-                got, want = gl[valid].float(), (g.expand(n) if gstride == 0 else g[valid])
-            if not _within_promise(got, want):
+                kept = _within_promise(gl[valid].float(),
+                                       g.expand(n) if gstride == 0 else g[valid])
+            if not kept:
                 raise RuntimeError(
                     "the upstream gradient of the loss differs from the grad_scale promised to "
                     "fused_linear_cross_entropy by more than "
