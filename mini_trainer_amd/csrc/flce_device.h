@@ -70,12 +70,18 @@ __device__ __forceinline__ void round_pair(float& lo, float& hi) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 
-// tanh(x) from exp2: 1 - 2 / (exp(2|x|) + 1), sign restored.
+// tanh(x) from exp2: 1 - 2 / (exp(2|x|) + 1), sign restored.  The quotient is
+// the reciprocal instruction (1 ulp) and one Newton step (rounded like a
+// division but for its last bit) instead of the division's ten instructions:
+// softcapped forward -3.5%, recompute -6%, the in-place pass over kept logits
+// -16% (121 -> 101 us for 2400 x 50257).  |x| is capped where tanh is 1 in fp32,
+// so that the step never sees an infinity.  NaN stays NaN.
 __device__ __forceinline__ float tanh_approx(float x) {
-  float ax = fabsf(x);
-  float e = fast_exp2(ax * (2.0f * kLog2e));
-  float t = 1.0f - 2.0f / (e + 1.0f);
-  return copysignf(t, x);
+  const float ax = fabsf(x);
+  const float d = fast_exp2((ax > 20.f ? 20.f : ax) * (2.0f * kLog2e)) + 1.0f;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  return copysignf(fmaf(-2.0f, r, 1.0f), x);
 }
 
 // Online log-sum-exp state merge in the log2 domain: (m, d) represents

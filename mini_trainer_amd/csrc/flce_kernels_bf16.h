@@ -124,6 +124,17 @@ __device__ __forceinline__ void fwd_epilogue_bf16(const f32x4_t (&acc)[8][8], fl
     if (kTail) asm volatile("" : "+v"(lim));
     float v[8][4];
     uint32_t slo[8], shi[8];
+    const uint32_t soff = (uint32_t)rglob[fm] * (uint32_t)a.lds_b + scol * 2u;
+    auto store_pair = [&](int p) __attribute__((always_inline)) {
+      const auto l2 = __builtin_amdgcn_permlane16_swap(slo[2 * p], slo[2 * p + 1], false, false);
+      const auto h2 = __builtin_amdgcn_permlane16_swap(shi[2 * p], shi[2 * p + 1], false, false);
+      u32x4_t o;
+      o[0] = l2[0];
+      o[1] = h2[0];
+      o[2] = l2[1];
+      o[3] = h2[1];
+      __builtin_amdgcn_raw_buffer_store_b128(o, srs, soff + (uint32_t)p * 64u, 0, 0);
+    };
     float tmax = -INFINITY;
 #pragma unroll
     for (int fn = 0; fn < 8; ++fn) {
@@ -143,20 +154,16 @@ __device__ __forceinline__ void fwd_epilogue_bf16(const f32x4_t (&acc)[8][8], fl
         v[fn][r] = x;
         tmax = fmaxf(tmax, x);
       }
-    }
-    if (kStoreS) {
-      const uint32_t soff = (uint32_t)rglob[fm] * (uint32_t)a.lds_b + scol * 2u;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const auto l2 = __builtin_amdgcn_permlane16_swap(slo[2 * p], slo[2 * p + 1], false, false);
-        const auto h2 = __builtin_amdgcn_permlane16_swap(shi[2 * p], shi[2 * p + 1], false, false);
-        u32x4_t o;
-        o[0] = l2[0];
-        o[1] = h2[0];
-        o[2] = l2[1];
-        o[3] = h2[1];
-        __builtin_amdgcn_raw_buffer_store_b128(o, srs, soff + (uint32_t)p * 64u, 0, 0);
+      // (softcapped rows store each fragment pair at once: held until the row's
+      // last tanh the packed logits made the allocator spill up to 50 VGPRs)
+      if (kCap && kStoreS && (fn & 1)) {
+        store_pair(fn >> 1);
+        sched_fence();
       }
+    }
+    if (kStoreS && !kCap) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p) store_pair(p);
     }
     const float mn = fmaxf(m2[fm], tmax * kLog2e);
     float sum = 0.f;
