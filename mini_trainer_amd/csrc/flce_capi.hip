@@ -531,32 +531,71 @@ double phase_time(int64_t dx_items, int64_t dx_k, int64_t dw_tiles, int64_t dw_k
   return std::max(cu / kCUs, tile_time(dx_k)) + 2 * kLaunch;
 }
 
+// End of n1 items of length l1, then n2 of length l2, each started on the slot
+// that frees up first (slots alike, kept as groups of equal finishing time).
+double list_makespan(int64_t slots, int64_t n1, double l1, int64_t n2, double l2) {
+  std::vector<std::pair<double, int64_t>> g{{0.0, slots}};  // ascending times
+  double end = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    int64_t n = pass ? n2 : n1;
+    const double l = pass ? l2 : l1;
+    while (n > 0) {
+      const double t = g[0].first + l;
+      const int64_t k = std::min(n, g[0].second);
+      g[0].second -= k;
+      n -= k;
+      if (g[0].second == 0) g.erase(g.begin());
+      auto it = g.begin();
+      while (it != g.end() && it->first < t) ++it;
+      if (it != g.end() && it->first == t) it->second += k;
+      else g.insert(it, {t, k});
+      end = std::max(end, t);
+    }
+  }
+  return end;
+}
+// The same phase as the dispatcher places it, dX's tiles first, each on the CU
+// that frees up first: with a few dW tiles per CU the last round counts
+// (252 dX tiles of depth 10240 beside 560 dW tiles over 4505 rows: 610 us
+// measured, 26k K-entries; their share of the CUs' time is 21.8k).  Over many
+// rounds that is the share and half a tile more.
+double phase_makespan(int64_t dx_items, int64_t dx_k, int64_t dw_tiles, int64_t dw_k, int64_t dw_extra) {
+  if (dx_items + dw_tiles > 6 * kCUs) {
+    const double a = tile_time(dx_k), b = tile_time(dw_k, dw_extra);
+    return std::max({(dx_items * a + dw_tiles * b) / kCUs + 0.5 * std::min(a, b), a, b}) + 2 * kLaunch;
+  }
+  return list_makespan(kCUs, dx_items, tile_time(dx_k), dw_tiles, tile_time(dw_k, dw_extra)) + 2 * kLaunch;
+}
+
 // Modelled seconds for one backward with blocks of C x Cv.  narrow: the
 // narrowing entry (one row block, dW tiles stored once in bf16, dX and dW
 // of every block in one launch).  blocks: the estimate the blocks are chosen
 // by -- a launch of a few rounds is charged 60% of a busy CU for each idle one
 // (540 recompute tiles of depth 3584 run in 243 us, 2.7 rounds' time; the 30%
-// that rank the paths fit launches of many rounds), and no launch is shorter
-// than its longest tile: one dW tile over 35k rows took 0.8 ms of a block
-// whose CUs' share of the work was 0.1.
+// that rank the paths fit launches of many rounds), dX beside dW takes its
+// makespan, and no launch is shorter than its longest tile: one dW tile over
+// 35k rows took 0.8 ms of a block whose CUs' share of the work was 0.1.
 double backward_cost(int64_t N, int64_t H, int64_t V, int64_t C, int64_t Cv, int es,
                      bool narrow = false, bool blocks = false) {
   (void)es;
   double t = 0, bytes = 0;
-  const double idle = blocks ? 0.6 : 0.3;
+  const int64_t nv = cdiv(V, Cv), th = cdiv(H, 256), extra = narrow ? 0 : kDwRmwK;
+  // one block of cn rows and cv columns
+  auto block = [&](int64_t cn, int64_t cv) {
+    const int64_t tm = cdiv(cn, 256), tv = cdiv(cv, 256);
+    const bool beside = narrow || tm * th < kCUs;  // dW beside dX
+    if (!blocks)
+      return gemm_time(tm * tv, H) + (beside ? phase_time(tm * th, cv, tv * th, cn, extra)
+                                             : gemm_time(tm * th, cv) + gemm_time(tv * th, cn, extra));
+    const double dw_tile = tile_time(cn, extra);
+    return std::max(gemm_time(tm * tv, H, 0, 0.6), tile_time(H)) +
+           (beside ? phase_makespan(tm * th, cv, tv * th, cn, extra)
+                   : gemm_time(tm * th, cv, 0, 0.6) + std::max(gemm_time(tv * th, cn, extra, 0.6), dw_tile));
+  };
   for (int64_t c0 = 0; c0 < N; c0 += C) {
     const int64_t cn = std::min(C, N - c0);
-    const int64_t nv = cdiv(V, Cv), tm = cdiv(cn, 256), th = cdiv(H, 256);
-    for (int64_t v0 = 0; v0 < V; v0 += Cv) {
-      const int64_t cv = std::min(Cv, V - v0), tv = cdiv(cv, 256);
-      const int64_t extra = narrow ? 0 : kDwRmwK;
-      const double dw_tile = blocks ? tile_time(cn, extra) : 0.0;
-      t += blocks ? std::max(gemm_time(tm * tv, H, 0, idle), tile_time(H)) : gemm_time(tm * tv, H);
-      if (narrow || tm * th < kCUs)  // dW beside dX
-        t += std::max(phase_time(tm * th, cv, tv * th, cn, extra), dw_tile);
-      else
-        t += gemm_time(tm * th, cv, 0, idle) + std::max(gemm_time(tv * th, cn, extra, idle), dw_tile);
-    }
+    if (nv > 1) t += (double)(nv - 1) * block(cn, Cv);
+    t += block(cn, V - (nv - 1) * Cv);
     if (nv > 1) bytes += (double)(2 * nv - 2) * cn * H * 4;  // dX accumulator
     t += kLaunch;
   }
@@ -622,8 +661,8 @@ inline bool narrow_scratch_fits(int64_t V, int64_t H, int64_t C) {
 // dX's accumulator in the dW buffer; more row blocks run
 // mt_flce_backward_tiles and the narrowing pass, which the cost includes.
 // blocks (a plan to run, not one to price a path with): the cost model of the
-// blocks, and for the best row blocking also a few more, smaller vocabulary
-// blocks, whose tiles may fill whole rounds better.
+// blocks, and for a few row blocks also vocabulary blocks a few tiles
+// narrower, whose tiles may fill whole rounds better.
 BwdPlan plan_backward(int64_t T, int64_t N, int64_t H, int64_t V, int es, size_t budget,
                       bool narrow = false, bool blocks = false) {
   BwdPlan best;
@@ -659,14 +698,16 @@ BwdPlan plan_backward(int64_t T, int64_t N, int64_t H, int64_t V, int es, size_t
     }
     return true;
   };
-  for (int64_t nt = 1; nt <= max_nt; ++nt) {
+  for (int64_t nt = 1; nt <= max_nt; nt += blocks && nt >= 16 ? nt / 8 : 1) {
     const int64_t C = round_up(cdiv(N, nt), 256);
-    for (int64_t nv = 1; nv <= max_nv; ++nv)
-      if (consider(C, round_up(cdiv(V, nv), 256))) break;  // larger nv only shrinks blocks further
-  }
-  if (blocks && best.C) {
-    const int64_t C = best.C, nv = cdiv(V, best.Cv);
-    for (int64_t more = 1; more <= 6; ++more) consider(C, round_up(cdiv(V, nv + more), 256));
+    for (int64_t nv = 1; nv <= max_nv; ++nv) {
+      const int64_t Cv = round_up(cdiv(V, nv), 256);
+      if (!consider(C, Cv)) continue;
+      // (larger nv only shrinks blocks further)
+      if (blocks && nt <= 4)
+        for (int64_t less = 1; less <= 12 && Cv - 256 * less >= 256; ++less) consider(C, Cv - 256 * less);
+      break;
+    }
   }
   return best.C ? best : smallest;
 }
@@ -1008,29 +1049,6 @@ struct F32Blocks {
   int64_t S = 1, Cv = 0, planes = 0;
 };
 
-// End of n1 items of length l1, then n2 of length l2, each started on the slot
-// that frees up first (slots alike, kept as groups of equal finishing time).
-double list_makespan(int64_t slots, int64_t n1, double l1, int64_t n2, double l2) {
-  std::vector<std::pair<double, int64_t>> g{{0.0, slots}};  // ascending times
-  double end = 0;
-  for (int pass = 0; pass < 2; ++pass) {
-    int64_t n = pass ? n2 : n1;
-    const double l = pass ? l2 : l1;
-    while (n > 0) {
-      const double t = g[0].first + l;
-      const int64_t k = std::min(n, g[0].second);
-      g[0].second -= k;
-      n -= k;
-      if (g[0].second == 0) g.erase(g.begin());
-      auto it = g.begin();
-      while (it != g.end() && it->first < t) ++it;
-      if (it != g.end() && it->first == t) it->second += k;
-      else g.insert(it, {t, k});
-      end = std::max(end, t);
-    }
-  }
-  return end;
-}
 F32Blocks f32_blocks(int64_t C, int64_t cn, int64_t H, int64_t V, size_t bytes) {
   const int64_t xt = (int64_t)align_up((size_t)H * C * 4), plane = C * H * 4;
   const int64_t tm = cdiv(cn, kTileF), th = cdiv(H, kTileF), vt = cdiv(V, kTileF);
@@ -1472,13 +1490,15 @@ double kept_cost(int64_t N, int64_t H, int64_t V, int64_t cols, const DxSplit& d
   const int64_t tm = cdiv(N, 256), th = cdiv(H, 256), nb = cdiv(V, cols);
   double t = forward_cost(N, H, V) + (nb > 1 ? kLaunch : 0);
   t += 4.0 * N * std::min(cols, V) / kBw;  // logits read, G written
-  for (int64_t v0 = 0; v0 < V; v0 += cols) {
-    const int64_t cv = std::min(cols, V - v0), tv = cdiv(cv, 256);
-    if (v0 > 0) t += gemm_time(tm * tv, H);
-    // (few columns: one dW tile over all rows can be the longest item)
-    t += std::max(phase_time(tm * th * d.S, cdiv(cv, d.S), tv * th, N, extra),
-                  tile_time(N, extra) + 2 * kLaunch);
-  }
+  auto block = [&](int64_t cv, bool recompute) {
+    const int64_t tv = cdiv(cv, 256);
+    return (recompute ? std::max(gemm_time(tm * tv, H, 0, 0.6), tile_time(H)) : 0.0) +
+           phase_makespan(tm * th * d.S, cdiv(cv, d.S), tv * th, N, extra);
+  };
+  const int64_t last = V - (nb - 1) * cols;
+  t += block(nb == 1 ? last : cols, false);
+  if (nb > 2) t += (double)(nb - 2) * block(cols, true);
+  if (nb > 1) t += block(last, true);
   // dX planes (or the accumulator) stored, re-read and added to, then summed
   const double plane = (double)N * H * 4;
   if (d.S > 1 || nb > 1) t += plane * d.S * (2.0 * nb - 1.0) * 0.5 / kBw;
