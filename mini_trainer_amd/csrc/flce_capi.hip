@@ -1363,26 +1363,39 @@ int launch_fused(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V,
     hipLaunchKernelGGL(fwd_finalize_kernel, dim3((uint32_t)cdiv(cn, 4)), dim3(256), 0, stream,
                        part, xy, (int32_t)cn, (int32_t)vt, row_index + c0, loss, lse + c0, guard);
     MT_TRY(check_launch("fwd_finalize_kernel"));
-    // the guarded recomputation: logits stored, G formed in place (both
-    // return at once unless the guard was raised)
+    // the guarded recomputation: logits stored, which fused_grad_kernel turns
+    // into G (it returns at once unless the guard was raised)
     a.guard_reset = nullptr;
     a.run_if = guard;
     hipLaunchKernelGGL(kerns_s[ci][ti][ki], fgrid, dim3(kThreadsBf), 0, stream, a);
     MT_TRY(check_launch("fwd_bf16_kernel"));
-    hipLaunchKernelGGL(softcap > 0.f ? softmax_grad_kernel<true> : softmax_grad_kernel<false>,
-                       dim3((uint32_t)cn_pad), dim3(256), 0, stream, S, lds_b,
-                       (int32_t)Vp, (int32_t)cn, (int32_t)V, lse + c0, grad, gstride,
-                       row_index + c0, row_label + c0, softcap, guard);
-    MT_TRY(check_launch("softmax_grad_kernel"));
-    // (also clears dW's work queue: dW runs after the fork below)
-    hipLaunchKernelGGL(fused_row_scale_kernel, dim3((uint32_t)(cn_pad / 256)), dim3(256), 0, stream,
-                       (int32_t)cn, (int32_t)cn_pad, lse + c0, xy, grad, gstride, row_index + c0,
-                       row_label + c0, guard, softcap, S, lds_b, scale, queue, (int32_t)kQueueWords);
-    MT_TRY(check_launch("fused_row_scale_kernel"));
-    hipLaunchKernelGGL(gather_t_kernel<__bf16>, dim3((uint32_t)(cn_pad / 64), (uint32_t)cdiv(H, 64)),
-                       dim3(256), 0, stream, static_cast<const char*>(X), ldx * 2, row_index + c0,
-                       (int32_t)cn, (int32_t)H, XcT, ldxt_b, static_cast<const float*>(scale));
-    MT_TRY(check_launch("gather_t_kernel"));
+    // G or the row factors, X^T, and dW's work queue cleared
+    FusedGradArgs fg;
+    fg.S = S;
+    fg.lds_b = lds_b;
+    fg.cols = (int32_t)Vp;
+    fg.cn = (int32_t)cn;
+    fg.rows = (int32_t)cn_pad;
+    fg.V = (int32_t)V;
+    fg.lse = lse + c0;
+    fg.xy = xy;
+    fg.grad = grad;
+    fg.gstride = gstride;
+    fg.row_index = row_index + c0;
+    fg.row_label = row_label + c0;
+    fg.guard = guard;
+    fg.softcap = softcap;
+    fg.scale = scale;
+    fg.X = static_cast<const char*>(X);
+    fg.ldx_b = ldx * 2;
+    fg.H = (int32_t)H;
+    fg.XcT = XcT;
+    fg.ldxt_b = ldxt_b;
+    fg.zero_words = queue;
+    fg.n_zero = (int32_t)kQueueWords;
+    hipLaunchKernelGGL(softcap > 0.f ? fused_grad_kernel<true> : fused_grad_kernel<false>,
+                       dim3((uint32_t)(cn_pad + cn_pad / 64 * cdiv(H, 64))), dim3(256), 0, stream, fg);
+    MT_TRY(check_launch("fused_grad_kernel"));
 
     DxArgs x;
     x.G = S;
@@ -1459,7 +1472,7 @@ int launch_fused(const void* X, const void* W, int64_t Tn, int64_t H, int64_t V,
 // ----------------------------------------------------------- kept logits
 // Forward that keeps the bf16-rounded logits of vocabulary columns [0, cols) of
 // every valid row, backward of one row block that turns them into G in place
-// (softmax_grad_kernel) and recomputes only the other columns, in blocks of
+// (softmax_grad_row) and recomputes only the other columns, in blocks of
 // at most `cols`, into the same buffer.  Each dW tile is written once in bf16,
 // any per-token upstream gradient is exact, and nothing is lost by storing
 // the logits (they are bf16 values).  With every column kept that is 6 H V N
@@ -1734,7 +1747,7 @@ int mt_flce_prepare(const int64_t* labels, int64_t T, int64_t V, int64_t ignore_
   if (V <= 0 || V > INT32_MAX) return fail(MT_ERR_INVALID_ARGUMENT, "V=%lld out of range", (long long)V);
   if (!counts || (T > 0 && (!labels || !row_index || !row_label)))
     return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
-  hipLaunchKernelGGL(prepare_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, labels, T, V,
+  hipLaunchKernelGGL(prepare_kernel, dim3((uint32_t)std::max<int64_t>(1, cdiv(T, kPrepLabels))), dim3(1024), 0, (hipStream_t)stream, labels, T, V,
                      ignore_index, shift, row_index, row_label, counts);
   return check_launch("prepare_kernel");
 }

@@ -123,7 +123,7 @@ __device__ __forceinline__ void fwd_final_merge(char* lds, float (&m2)[8], float
 // (deterministic order).
 // guard (non-null): set to 1 when some row's largest logit lies outside
 // [kGuardLo, kGuardHi], the range in which the fused path keeps exp(logit)
-// itself in bf16 (see fused_row_scale_kernel): at a row maximum of -48 the
+// itself in bf16 (see fused_grad_kernel): at a row maximum of -48 the
 // terms within 39 of it (relative weight e^-39 and more) stay normal numbers
 // (e^-87 is about the smallest), and at +48, lse <= 48 + ln V keeps the row
 // factor g exp(-lse) a normal fp32 number for g down to 1e-10 at V = 2^20.
@@ -157,44 +157,6 @@ __global__ __launch_bounds__(256) void fwd_finalize_kernel(const float* part, co
     const float mx = m * kLn2;
     if (guard && !(mx >= kGuardLo && mx <= kGuardHi)) atomicOr(guard, 1);
   }
-}
-
-// Fused path, per row chunk, after the forward stored E = exp(z) (z the
-// bf16-rounded, soft-capped logit; times the softcap derivative 1 - (z/cap)^2)
-// instead of the logits: G = g (softmax - onehot) dz = s E - onehot g dz with
-// the per-row factor s = g exp(-lse).  dX = G W and dW = G^T X then take s as
-// a row scale of dX and of the gathered X^T (gather_t_kernel), and this
-// kernel replaces the label's element by (exp(z_y) - exp(lse)) dz_y, formed
-// in fp32 from the label logit (no cancellation against the rounded E).  When
-// the guard is set the chunk holds G itself (the logits were stored and
-// turned into G by softmax_grad_kernel): s = 1 and no element is touched.
-// Rows cn .. cn_pad get s = 0.  One thread per row; the first n_zero threads
-// also clear zero_words (the dW work queue of the chunk).
-__global__ __launch_bounds__(256) void fused_row_scale_kernel(
-    int32_t cn, int32_t cn_pad, const float* lse, const float* xy, const float* grad,
-    int64_t gstride, const int32_t* row_index, const int32_t* row_label, const int32_t* guard,
-    float softcap, char* E, int64_t lde_b, float* scale, uint32_t* zero_words, int32_t n_zero) {
-  const int32_t t = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (t < n_zero) zero_words[t] = 0u;
-  if (t >= cn_pad) return;
-  if (t >= cn) {
-    scale[t] = 0.f;
-    return;
-  }
-  if (*guard != 0) {
-    scale[t] = 1.f;
-    return;
-  }
-  const float L = lse[t], z = xy[t];
-  const float g = grad[(int64_t)row_index[t] * gstride];
-  float dz = 1.f;
-  if (softcap > 0.f) {
-    const float q = z / softcap;
-    dz = fmaf(-q, q, 1.f);
-  }
-  const float e = (fast_exp2(z * kLog2e) - fast_exp2(L * kLog2e)) * dz;
-  reinterpret_cast<__bf16*>(E + (int64_t)t * lde_b)[row_label[t]] = (__bf16)e;
-  scale[t] = g * fast_exp2(-L * kLog2e);
 }
 
 // ===========================================================================
@@ -378,14 +340,14 @@ constexpr int kDwRows = 0, kDwTiles = 1, kDwNarrow = 2;
 
 // XcT[h][t] = X[row_index[t]][h] for t < Cn, 0 for Cn <= t < t_pad.
 // 64 x 64 element tiles; 16-byte loads along h, 16-byte stores along t.
-// scale (non-null, bf16 only): row t is multiplied by scale[t] in fp32 and
-// rounded to bf16 (the fused path's per-row factor of G, see
-// fused_row_scale_kernel).
-template <typename T>
+// scale (bf16 only): row t is multiplied by scale(t) in fp32 and rounded to
+// bf16 (the fused path's per-row factor of G, see fused_grad_kernel); kScale
+// false: not at all.
+template <typename T, bool kScale, class Scale>
 __device__ __forceinline__ void gather_t_tile(T (&tile)[64][64 + 1], int32_t t0, int32_t hb,
                                               const char* X, int64_t ldx_b, const int32_t* row_index,
                                               int32_t Cn, int32_t H, char* XcT, int64_t ldxt_b,
-                                              const float* scale) {
+                                              Scale scale) {
   constexpr int E = sizeof(T);
   constexpr int PER = 16 / E;  // elements per 16-byte vector
   // load 64 rows (t) x 64 h
@@ -396,9 +358,9 @@ __device__ __forceinline__ void gather_t_tile(T (&tile)[64][64 + 1], int32_t t0,
     if (t < Cn && hb + hc < H)
       val = *reinterpret_cast<const u32x4_t*>(X + (int64_t)row_index[t] * ldx_b +
                                               (int64_t)(hb + hc) * E);
-    if constexpr (sizeof(T) == 2) {
-      if (scale && t < Cn) {
-        const float sc = scale[t];
+    if constexpr (kScale) {
+      if (t < Cn) {
+        const float sc = scale(t);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           val[j] = pack_bf16x2(__builtin_bit_cast(float, val[j] << 16) * sc,
@@ -424,11 +386,10 @@ __device__ __forceinline__ void gather_t_tile(T (&tile)[64][64 + 1], int32_t t0,
 template <typename T>
 __global__ __launch_bounds__(256) void gather_t_kernel(const char* X, int64_t ldx_b,
                                                        const int32_t* row_index, int32_t Cn,
-                                                       int32_t H, char* XcT, int64_t ldxt_b,
-                                                       const float* scale = nullptr) {
+                                                       int32_t H, char* XcT, int64_t ldxt_b) {
   __shared__ T tile[64][64 + 1];
-  gather_t_tile<T>(tile, blockIdx.x * 64, blockIdx.y * 64, X, ldx_b, row_index, Cn, H, XcT, ldxt_b,
-                   scale);
+  gather_t_tile<T, false>(tile, blockIdx.x * 64, blockIdx.y * 64, X, ldx_b, row_index, Cn, H, XcT,
+                          ldxt_b, 0);
 }
 
 // Zero `nrows` rows (ids from rows[]) of a row-major matrix, row_bytes each
@@ -461,97 +422,112 @@ __global__ __launch_bounds__(256) void zero_scatter_f32_kernel(float* loss, cons
     loss[rows[i]] = 0.0f;
 }
 
-// Valid-row compaction in one workgroup of 1024 threads.
+// Valid-row compaction, one workgroup of 1024 threads per 4096 labels.
 //   row_index[0 .. N)    positions t with a valid label, ascending
 //   row_index[N .. T)    every other position (descending from the end)
 //   row_label[0 .. N)    their labels
 //   counts = {N, #labels outside [0, V), first such t or -1, 0}
+// Each workgroup counts the labels before its own by itself (they come from L2;
+// independent loads), so no workgroup waits for another and no scratch is
+// needed; the last one writes counts.  Bound by latency: one workgroup walking
+// all labels, a scan and two barriers per 4096, took 58 us for 53k labels.
+constexpr int kPrepItems = 4, kPrepLabels = 1024 * kPrepItems;
 __global__ __launch_bounds__(1024) void prepare_kernel(const int64_t* labels, int64_t T, int64_t V,
                                                        int64_t ignore, int shift, int32_t* row_index,
                                                        int32_t* row_label, int32_t* counts) {
-  constexpr int kItems = 4;
-  __shared__ int32_t wsum_v[16], wsum_m[16];
-  __shared__ int32_t s_base_v, s_base_m, s_bad, s_first_bad;
+  __shared__ int32_t wsum_v[16], wpre_v[16], wbad[16], wfirst[16];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  if (tid == 0) {
-    s_base_v = 0;
-    s_base_m = 0;
-    s_bad = 0;
-    s_first_bad = INT32_MAX;
+  const int64_t start = (int64_t)blockIdx.x * kPrepLabels;
+  auto label = [&](int64_t t) __attribute__((always_inline)) {
+    return shift ? (t + 1 < T ? labels[t + 1] : ignore) : labels[t];
+  };
+  // 0 ignored, 1 valid, 2 out of range
+  auto kind = [&](int64_t lab) __attribute__((always_inline)) {
+    return lab == ignore ? 0 : (lab < 0 || lab >= V ? 2 : 1);
+  };
+  int32_t pre_v = 0, bad = 0, first = INT32_MAX;
+  auto see_bad = [&](int k, int64_t t) __attribute__((always_inline)) {
+    if (k == 2) {
+      ++bad;
+      first = min(first, (int32_t)t);
+    }
+  };
+  for (int64_t t0 = tid; t0 < start; t0 += 1024 * 8) {
+    int64_t lab[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) lab[j] = t0 + j * 1024 < start ? label(t0 + j * 1024) : ignore;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = kind(lab[j]);
+      pre_v += k == 1;
+      see_bad(k, t0 + j * 1024);
+    }
+  }
+  int32_t y[kPrepItems];
+  uint32_t vmask = 0, mmask = 0;
+#pragma unroll
+  for (int j = 0; j < kPrepItems; ++j) {
+    const int64_t t = start + tid * kPrepItems + j;
+    y[j] = 0;
+    if (t >= T) continue;
+    const int64_t lab = label(t);
+    const int k = kind(lab);
+    see_bad(k, t);
+    if (k == 1) {
+      vmask |= 1u << j;
+      y[j] = (int32_t)lab;
+    } else {
+      mmask |= 1u << j;
+    }
+  }
+  const int cv = __builtin_popcount(vmask);
+  int sv = cv;  // inclusive wave scan of the workgroup's own valid labels
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(sv, o);
+    if (lane >= o) sv += up;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    pre_v += __shfl_xor(pre_v, o);
+    bad += __shfl_xor(bad, o);
+    first = min(first, __shfl_xor(first, o));
+  }
+  if (lane == 63) {
+    wsum_v[wid] = sv;
+    wpre_v[wid] = pre_v;
+    wbad[wid] = bad;
+    wfirst[wid] = first;
   }
   __syncthreads();
-  for (int64_t start = 0; start < T; start += 1024 * kItems) {
-    int32_t y[kItems];
-    uint32_t vmask = 0, mmask = 0;
-#pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const int64_t t = start + tid * kItems + j;
-      y[j] = 0;
-      if (t >= T) continue;
-      int64_t lab;
-      if (shift) lab = (t + 1 < T) ? labels[t + 1] : ignore;
-      else lab = labels[t];
-      if (lab == ignore) {
-        mmask |= 1u << j;
-      } else if (lab < 0 || lab >= V) {
-        mmask |= 1u << j;
-        atomicAdd(&s_bad, 1);
-        atomicMin(&s_first_bad, (int32_t)t);
-      } else {
-        vmask |= 1u << j;
-        y[j] = (int32_t)lab;
-      }
-    }
-    const int cv = __builtin_popcount(vmask), cm = __builtin_popcount(mmask);
-    // inclusive wave scans
-    int sv = cv, sm = cm;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      int tv = __shfl_up(sv, o), tmm = __shfl_up(sm, o);
-      if (lane >= o) {
-        sv += tv;
-        sm += tmm;
-      }
-    }
-    if (lane == 63) {
-      wsum_v[wid] = sv;
-      wsum_m[wid] = sm;
-    }
-    __syncthreads();
-    int pv = 0, pm = 0, tv_all = 0, tm_all = 0;
-    for (int w = 0; w < 16; ++w) {
-      if (w < wid) {
-        pv += wsum_v[w];
-        pm += wsum_m[w];
-      }
-      tv_all += wsum_v[w];
-      tm_all += wsum_m[w];
-    }
-    int ov = s_base_v + pv + sv - cv;
-    int om = s_base_m + pm + sm - cm;
-#pragma unroll
-    for (int j = 0; j < kItems; ++j) {
-      const int64_t t = start + tid * kItems + j;
-      if (vmask & (1u << j)) {
-        row_index[ov] = (int32_t)t;
-        row_label[ov] = y[j];
-        ++ov;
-      } else if (mmask & (1u << j)) {
-        row_index[T - 1 - om] = (int32_t)t;
-        ++om;
-      }
-    }
-    __syncthreads();
-    if (tid == 0) {
-      s_base_v += tv_all;
-      s_base_m += tm_all;
-    }
-    __syncthreads();
+  int32_t before = 0, own = 0, base = 0;  // valid before this wave's labels, in all, before the workgroup
+  for (int w = 0; w < 16; ++w) {
+    if (w < wid) before += wsum_v[w];
+    own += wsum_v[w];
+    base += wpre_v[w];
   }
-  if (tid == 0) {
-    counts[0] = s_base_v;
-    counts[1] = s_bad;
-    counts[2] = s_bad ? s_first_bad : -1;
+  int32_t ov = base + before + sv - cv;
+  int32_t om = (int32_t)(start + (int64_t)tid * kPrepItems) - ov;  // others before this thread's labels
+#pragma unroll
+  for (int j = 0; j < kPrepItems; ++j) {
+    const int32_t t = (int32_t)(start + tid * kPrepItems + j);
+    if (vmask & (1u << j)) {
+      row_index[ov] = t;
+      row_label[ov] = y[j];
+      ++ov;
+    } else if (mmask & (1u << j)) {
+      row_index[T - 1 - om] = t;
+      ++om;
+    }
+  }
+  if (blockIdx.x == gridDim.x - 1 && tid == 0) {
+    for (int w = 1; w < 16; ++w) {
+      bad += wbad[w];
+      first = min(first, wfirst[w]);
+    }
+    counts[0] = base + own;
+    counts[1] = bad;
+    counts[2] = bad ? first : -1;
     counts[3] = 0;
   }
 }

@@ -66,7 +66,7 @@ struct TileSeq {
 // row's lse is known.  kStore = kStoreExp: S receives E = exp(z) (1 - (z /
 // cap)^2) instead, z the soft-capped logit (fwd_epilogue_exp_bf16): G is
 // then s E with a per-row factor s applied downstream (see
-// fused_row_scale_kernel), which saves the pass over S that forms G.
+// fused_grad_kernel), which saves the pass over S that forms G.
 // Row tiles per group of the forward's tile walk: W (the larger operand) is
 // streamed once per group, so wider groups cut its re-reads.  Up to 12 row
 // tiles walk as one group, more in groups of 8.  Measured in same-box
@@ -1213,12 +1213,11 @@ __global__ __launch_bounds__(256) void narrow_tiles_kernel(const float* scale, c
   }
 }
 
-// G = g_t (softmax(cap(S_t)) - onehot(y_t)) (1 - tanh^2), in place over the
-// bf16 logits S written by fwd_bf16_kernel<*, kStoreLogits>: the kept logits
-// of a whole call, or (run_if non-null: nothing unless *run_if != 0) a fused
-// chunk whose exponentials would leave bf16's range.  One workgroup per row;
-// rows >= cn and columns >= V become 0.  HBM-bound: one 16-byte read and one
-// 16-byte write per 8 elements.
+// G = g_t (softmax(cap(S_t)) - onehot(y_t)) (1 - tanh^2), in place over row
+// `row` of the bf16 logits S written by fwd_bf16_kernel<*, kStoreLogits>: kept
+// logits, or a fused chunk whose exponentials would leave bf16's range.  One
+// workgroup per row; rows >= cn and columns >= V become 0.  HBM-bound: one
+// 16-byte read and one 16-byte write per 8 elements.
 template <bool kCap>
 __device__ __forceinline__ void softmax_grad_row(int32_t row, char* S, int64_t lds_b, int32_t cols,
                                                  int32_t cn, int32_t V, const float* lse,
@@ -1267,18 +1266,73 @@ __device__ __forceinline__ void softmax_grad_row(int32_t row, char* S, int64_t l
   for (; c < cols; c += kStep) p[c / 8] = grad8(p[c / 8], c);
 }
 
+// Fused path, per row chunk, after the forward stored E = exp(z) (z the
+// bf16-rounded, soft-capped logit; times the softcap derivative 1 - (z/cap)^2)
+// instead of the logits: G = g (softmax - onehot) dz = s E - onehot g dz with
+// the per-row factor s = g exp(-lse).  dX = G W and dW = G^T X then take s as a
+// row scale of dX and of the gathered X^T, and the label's element becomes
+// (exp(z_y) - exp(lse)) dz_y, formed in fp32 from the label logit (no
+// cancellation against the rounded E).  When the guard is set the chunk holds
+// the logits instead (stored by the guarded launch before this one): they
+// become G itself (softmax_grad_row) and s = 1.  Rows cn .. rows get s = 0.
+// One launch (three serial ones took 15 us a chunk): workgroups [0, rows) do
+// row b, the others gather and transpose X (XcT, see gather_t_tile) with s
+// formed on the way; zero_words[0 .. n_zero) (the chunk's dW work queue) are
+// cleared.
+struct FusedGradArgs {
+  char* S;
+  int64_t lds_b;
+  int32_t cols, cn, rows, V;
+  const float* lse;
+  const float* xy;
+  const float* grad;
+  int64_t gstride;
+  const int32_t* row_index;
+  const int32_t* row_label;
+  const int32_t* guard;
+  float softcap;
+  float* scale;
+  const char* X;
+  int64_t ldx_b;
+  int32_t H;
+  char* XcT;
+  int64_t ldxt_b;
+  uint32_t* zero_words;
+  int32_t n_zero;
+};
 template <bool kCap>
-__global__ __launch_bounds__(256) void softmax_grad_kernel(char* S, int64_t lds_b, int32_t cols,
-                                                           int32_t cn, int32_t V,
-                                                           const float* lse, const float* grad,
-                                                           int64_t gstride,
-                                                           const int32_t* row_index,
-                                                           const int32_t* row_label,
-                                                           float softcap,
-                                                           const int32_t* run_if) {
-  if (run_if && *run_if == 0) return;
-  softmax_grad_row<kCap>((int32_t)blockIdx.x, S, lds_b, cols, cn, V, lse, grad, gstride, row_index,
-                         row_label, softcap);
+__global__ __launch_bounds__(256) void fused_grad_kernel(FusedGradArgs a) {
+  __shared__ __bf16 tile[64][64 + 1];
+  if (blockIdx.x == 0 && (int32_t)threadIdx.x < a.n_zero) a.zero_words[threadIdx.x] = 0u;
+  const bool raised = *a.guard != 0;
+  auto row_scale = [&](int32_t t) __attribute__((always_inline)) {
+    return raised ? 1.f
+                  : a.grad[(int64_t)a.row_index[t] * a.gstride] * fast_exp2(-a.lse[t] * kLog2e);
+  };
+  int32_t b = (int32_t)blockIdx.x;
+  if (b < a.rows) {
+    if (raised)
+      softmax_grad_row<kCap>(b, a.S, a.lds_b, a.cols, a.cn, a.V, a.lse, a.grad, a.gstride, a.row_index,
+                             a.row_label, a.softcap);
+    if (threadIdx.x == 0) {
+      a.scale[b] = b < a.cn ? row_scale(b) : 0.f;
+      if (!raised && b < a.cn) {
+        const float L = a.lse[b], z = a.xy[b];
+        float dz = 1.f;
+        if (kCap) {
+          const float q = z / a.softcap;
+          dz = fmaf(-q, q, 1.f);
+        }
+        const float e = (fast_exp2(z * kLog2e) - fast_exp2(L * kLog2e)) * dz;
+        reinterpret_cast<__bf16*>(a.S + (int64_t)b * a.lds_b)[a.row_label[b]] = (__bf16)e;
+      }
+    }
+    return;
+  }
+  b -= a.rows;
+  const int32_t gm = a.rows / 64;
+  gather_t_tile<__bf16, true>(tile, b % gm * 64, b / gm * 64, a.X, a.ldx_b, a.row_index, a.cn, a.H,
+                              a.XcT, a.ldxt_b, row_scale);
 }
 
 // What the products of the kept-logits backward need first, in one launch (three
@@ -1327,8 +1381,8 @@ __global__ __launch_bounds__(256) void kept_grad_kernel(KeptGradArgs a) {
   b -= a.rows;
   const int32_t tiles = a.gather_m * ((a.H + 63) / 64);
   if (b < tiles) {
-    gather_t_tile<__bf16>(tile, b % a.gather_m * 64, b / a.gather_m * 64, a.X, a.ldx_b, a.row_index,
-                          a.cn, a.H, a.XcT, a.ldxt_b, nullptr);
+    gather_t_tile<__bf16, false>(tile, b % a.gather_m * 64, b / a.gather_m * 64, a.X, a.ldx_b,
+                                 a.row_index, a.cn, a.H, a.XcT, a.ldxt_b, 0);
     return;
   }
   const int32_t nb = (int32_t)gridDim.x - a.rows - tiles;
