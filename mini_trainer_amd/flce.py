@@ -32,7 +32,7 @@ __all__ = [
 ]
 
 # Optional override of the backward workspace budget in bytes (default: 5% of
-# the materialised-logits size T * V * sizeof(dtype)).
+# the materialised-logits size T * V * sizeof(dtype), at least MIN_BUDGET).
 BACKWARD_BUDGET_ENV = "MT_FLCE_BWD_BUDGET_BYTES"
 # bf16: "auto" (default) keeps the logits where they fit (_kept_plan) and takes
 # the fused path when the planner expects it to pay, "1" always takes the fused
@@ -145,7 +145,8 @@ def _kept_plan(T: int, n: int, H: int, V: int,
     that keeps logits from the forward to the backward (mt_flce_logits_plan),
     columns 0 when none fit.  The default budget counts the bytes by which a
     bf16 weight gradient is smaller than the fp32 one of the other paths (no
-    such gradient exists with an accumulator); a budget set by MT_FLCE_BWD_BUDGET_BYTES is taken as it stands."""
+    such gradient exists with an accumulator); a budget set by
+    MT_FLCE_BWD_BUDGET_BYTES is taken as it stands."""
     room = int(int(os.environ.get(BACKWARD_BUDGET_ENV, "0")) == 0)
     cols, lb, sb, pays = ctypes.c_int64(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int()
     check(load().mt_flce_logits_plan(T, n, H, V, MT_DTYPE_BF16, _default_budget(T, V, 2), room,
