@@ -56,7 +56,7 @@
 extern "C" {
 #endif
 
-#define MT_FLCE_ABI_VERSION 8
+#define MT_FLCE_ABI_VERSION 9
 
 typedef struct ihipStream_t* mt_stream_t; /* == hipStream_t */
 
@@ -205,6 +205,18 @@ int mt_flce_backward_narrow_plan(int64_t T, int64_t n_valid, int64_t H,
                                  int64_t V, int dtype, size_t budget_bytes,
                                  int64_t* chunk_rows, int64_t* chunk_vocab,
                                  size_t* workspace_bytes);
+
+/*
+ * Either of the two plans above (narrow != 0: mt_flce_backward_narrow_plan) for
+ * a weight whose rows lie ldw >= H elements apart: a bf16 block's rows, gaps
+ * included, must lie within one buffer's reach (mt_flce_max_buffer_bytes).
+ * The plans above take ldw = H.  (No reference counterpart, as theirs.)
+ */
+int mt_flce_backward_plan_pitch(int64_t T, int64_t n_valid, int64_t H,
+                                int64_t V, int64_t ldw, int dtype,
+                                size_t budget_bytes, int narrow,
+                                int64_t* chunk_rows, int64_t* chunk_vocab,
+                                size_t* workspace_bytes);
 
 /*
  * Backward: dX = G W and dW (+)= G^T X with
@@ -358,8 +370,8 @@ int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V,
  * in blocks of keep_cols in the same buffer (6 H V n_valid flops in all when
  * every column is kept).
  *
- * mt_flce_logits_plan writes keep_cols (a multiple of 256, at most
- * round_up(V, 256)), the bytes of the logits buffer (round_up(n_valid, 256) x
+ * mt_flce_logits_plan (ldw: pitch of the weight's rows) writes keep_cols (a
+ * multiple of 256, at most round_up(V, 256)), the bytes of the logits buffer (round_up(n_valid, 256) x
  * keep_cols bf16) and of the backward's scratch (X^T, the dW work queue, dX's
  * fp32 accumulator or the planes of a dX split over the vocabulary), which fit
  * budget_bytes (0 = 5% of T V 2) -- plus, with count_gradient != 0, the bytes
@@ -386,7 +398,7 @@ int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V,
  * each chunk's logits to form the gradients from).
  */
 int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V,
-                        int dtype, size_t budget_bytes, int count_gradient,
+                        int64_t ldw, int dtype, size_t budget_bytes, int count_gradient,
                         int with_accumulator, int64_t* keep_cols,
                         size_t* logits_bytes, size_t* scratch_bytes, int* pays);
 int mt_flce_forward_logits(const void* X, const void* W, int64_t T, int64_t H,

@@ -14,7 +14,7 @@ import os
 # MT_FLCE_LIB: another build of the same library (the sanitized host-only
 # build of the CPU tests); unset in production.
 LIB_PATH = Path(os.environ.get("MT_FLCE_LIB") or Path(__file__).resolve().parent / "libmt_flce.so")
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 MT_DTYPE_F32 = 0
 MT_DTYPE_BF16 = 1
@@ -71,9 +71,12 @@ SIGNATURES = {
                                         c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p,
                                         c_size_t, c_void_p, c_size_t, c_int64, c_int64, c_void_p,
                                         c_size_t, c_void_p, c_void_p]),
-    "mt_flce_logits_plan": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int, c_size_t, c_int,
-                                    c_int, POINTER(c_int64), POINTER(c_size_t), POINTER(c_size_t),
-                                    POINTER(c_int)]),
+    "mt_flce_backward_plan_pitch": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int,
+                                            c_size_t, c_int, POINTER(c_int64), POINTER(c_int64),
+                                            POINTER(c_size_t)]),
+    "mt_flce_logits_plan": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_size_t,
+                                    c_int, c_int, POINTER(c_int64), POINTER(c_size_t),
+                                    POINTER(c_size_t), POINTER(c_int)]),
     "mt_flce_general_pays": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int, c_size_t, c_size_t,
                                      POINTER(c_int)]),
     "mt_flce_forward_logits": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,

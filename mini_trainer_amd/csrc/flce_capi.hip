@@ -662,11 +662,13 @@ inline bool narrow_scratch_fits(int64_t V, int64_t H, int64_t C) {
 // mt_flce_backward_tiles and the narrowing pass, which the cost includes.
 // blocks (a plan to run, not one to price a path with): the cost model of the
 // blocks, and for a few row blocks also vocabulary blocks a few tiles
-// narrower, whose tiles may fill whole rounds better.
+// narrower, whose tiles may fill whole rounds better.  ldw: pitch of the
+// weight's rows in elements (0: H), which bounds the rows one buffer reaches.
 BwdPlan plan_backward(int64_t T, int64_t N, int64_t H, int64_t V, int es, size_t budget,
-                      bool narrow = false, bool blocks = false) {
+                      bool narrow = false, bool blocks = false, int64_t ldw = 0) {
   BwdPlan best;
   if (N <= 0) return best;
+  ldw = std::min<int64_t>(std::max(ldw, H), INT32_MAX);  // (more is beyond any buffer)
   if (budget == 0) budget = (size_t)((double)T * V * es * 0.05);
   narrow = narrow && es == 2;
   double best_cost = 1e300;
@@ -685,7 +687,7 @@ BwdPlan plan_backward(int64_t T, int64_t N, int64_t H, int64_t V, int es, size_t
     // G, X^T and the block's weight rows (bf16) within one buffer's reach
     const uint64_t lim = buffer_limit();
     if ((uint64_t)C * Cv * es > lim || (uint64_t)H * C * es > lim ||
-        (es == 2 && (uint64_t)Cv * H * es > lim))
+        (es == 2 && (uint64_t)Cv * ldw * es > lim))
       return false;
     if (ws > budget) return false;
     const double cost =
@@ -1535,7 +1537,8 @@ DxSplit kept_split(int64_t cols, int64_t V, int64_t S) {
 // slices keep to XCDs of their own, see fused_split) the columns that fit, and of
 // these the cheapest.  Too few slices and dX, whose tiles contract a whole
 // block, outlasts dW beside it; a plane costs 2 H columns.
-KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bool room, bool acc) {
+KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, int64_t ldw, size_t budget, bool room,
+                   bool acc) {
   KeptPlan best;
   if (N <= 0 || H % 8 != 0) return best;
   if (budget == 0) budget = (size_t)((double)T * V * 2 * 0.05);
@@ -1545,7 +1548,7 @@ KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, size_t budget, bo
   const size_t have = budget + (room ? dw_tiles_bytes(V, H) - dw_lo_bytes(V, H) : 0);
   const size_t fwd = forward_ws(plan_forward(N, V, 2), N);
   // columns one buffer reaches: of the logits, and of the weight's rows
-  const int64_t reach = (int64_t)(std::min(lim / ((uint64_t)C * 2), lim / ((uint64_t)H * 2)) / 256 * 256);
+  const int64_t reach = (int64_t)(std::min(lim / ((uint64_t)C * 2), lim / ((uint64_t)ldw * 2)) / 256 * 256);
   for (int64_t S = 1; S <= 32; S *= 2) {
     for (int blocks = 0; blocks < 2; ++blocks) {
       const size_t other = std::max(kept_scratch(C, H, S, blocks != 0, acc), fwd);
@@ -1933,7 +1936,7 @@ namespace {
 
 int backward_plan_entry(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,
                         size_t budget_bytes, int64_t* chunk_rows, int64_t* chunk_vocab,
-                        size_t* workspace_bytes, bool narrow) {
+                        size_t* workspace_bytes, bool narrow, int64_t ldw = 0) {
   const int es = esize_of(dtype);
   if (!es) return fail(MT_ERR_INVALID_ARGUMENT, "dtype %d is not MT_DTYPE_F32 or MT_DTYPE_BF16", dtype);
   if (T < 0 || n_valid < 0 || n_valid > T || H <= 0 || V <= 0 || T > INT32_MAX || H > INT32_MAX ||
@@ -1944,7 +1947,7 @@ int backward_plan_entry(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dt
     return fail(MT_ERR_INVALID_ARGUMENT, "null output pointer");
   if (narrow && dtype != MT_DTYPE_BF16)
     return fail(MT_ERR_UNSUPPORTED, "the narrowing backward is bf16 only (dtype %d)", dtype);
-  const BwdPlan p = plan_backward(T, n_valid, H, V, es, budget_bytes, narrow, true);
+  const BwdPlan p = plan_backward(T, n_valid, H, V, es, budget_bytes, narrow, true, ldw);
   *chunk_rows = p.C;
   *chunk_vocab = p.Cv;
   *workspace_bytes = p.ws;
@@ -1960,6 +1963,15 @@ int mt_flce_backward_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int 
                           size_t* workspace_bytes) {
   return backward_plan_entry(T, n_valid, H, V, dtype, budget_bytes, chunk_rows, chunk_vocab,
                              workspace_bytes, false);
+}
+
+int mt_flce_backward_plan_pitch(int64_t T, int64_t n_valid, int64_t H, int64_t V, int64_t ldw,
+                                int dtype, size_t budget_bytes, int narrow, int64_t* chunk_rows,
+                                int64_t* chunk_vocab, size_t* workspace_bytes) {
+  if (ldw < H)
+    return fail(MT_ERR_INVALID_ARGUMENT, "ldw=%lld must be >= H=%lld", (long long)ldw, (long long)H);
+  return backward_plan_entry(T, n_valid, H, V, dtype, budget_bytes, chunk_rows, chunk_vocab,
+                             workspace_bytes, narrow != 0, ldw);
 }
 
 int mt_flce_backward_narrow_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,
@@ -2186,7 +2198,7 @@ int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V, int d
   return MT_OK;
 }
 
-int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dtype,
+int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int64_t ldw, int dtype,
                         size_t budget_bytes, int count_gradient, int with_accumulator,
                         int64_t* keep_cols, size_t* logits_bytes, size_t* scratch_bytes, int* pays) {
   if (dtype != MT_DTYPE_BF16)
@@ -2195,10 +2207,13 @@ int mt_flce_logits_plan(int64_t T, int64_t n_valid, int64_t H, int64_t V, int dt
       V > INT32_MAX)
     return fail(MT_ERR_INVALID_ARGUMENT, "bad sizes T=%lld n_valid=%lld H=%lld V=%lld", (long long)T,
                 (long long)n_valid, (long long)H, (long long)V);
+  if (ldw < H)
+    return fail(MT_ERR_INVALID_ARGUMENT, "ldw=%lld must be >= H=%lld", (long long)ldw, (long long)H);
   if (!keep_cols || !logits_bytes || !scratch_bytes || !pays)
     return fail(MT_ERR_INVALID_ARGUMENT, "null output pointer");
   const bool acc = with_accumulator != 0;
-  const KeptPlan p = plan_kept(T, n_valid, H, V, budget_bytes, count_gradient != 0 && !acc, acc);
+  const KeptPlan p = plan_kept(T, n_valid, H, V, std::min<int64_t>(ldw, INT32_MAX), budget_bytes,
+                               count_gradient != 0 && !acc, acc);
   *keep_cols = p.cols;
   *logits_bytes = p.logits;
   *scratch_bytes = p.scratch;

@@ -108,19 +108,22 @@ def prepare_targets(target: torch.Tensor, vocab_size: int, ignore_index: int = -
 
 
 def backward_plan(T: int, n_valid: int, H: int, V: int, dtype: torch.dtype,
-                  budget_bytes: Optional[int] = None, narrow: bool = False) -> Tuple[int, int, int]:
+                  budget_bytes: Optional[int] = None, narrow: bool = False,
+                  ldw: Optional[int] = None) -> Tuple[int, int, int]:
     """(chunk_rows, chunk_vocab, workspace_bytes) of the backward blocking;
     narrow: the plan of a bf16 backward whose weight gradient is wanted in
     bf16 and added into nothing (mt_flce_backward_narrow_plan: chunk_rows >=
     n_valid means one row block through mt_flce_backward_narrow), else of
-    mt_flce_backward."""
+    mt_flce_backward.  ldw: pitch of the weight's rows (default H)
+    (mt_flce_backward_plan_pitch)."""
     lib = load()
     if budget_bytes is None:
         budget_bytes = int(os.environ.get(BACKWARD_BUDGET_ENV, "0"))
     c, cv, ws = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_size_t()
-    fn = "mt_flce_backward_narrow_plan" if narrow else "mt_flce_backward_plan"
-    check(getattr(lib, fn)(T, n_valid, H, V, _dtype_code(dtype), budget_bytes, ctypes.byref(c),
-                           ctypes.byref(cv), ctypes.byref(ws)), fn)
+    check(lib.mt_flce_backward_plan_pitch(T, n_valid, H, V, H if ldw is None else ldw,
+                                          _dtype_code(dtype), budget_bytes, int(narrow),
+                                          ctypes.byref(c), ctypes.byref(cv), ctypes.byref(ws)),
+          "mt_flce_backward_plan_pitch")
     return c.value, cv.value, ws.value
 
 
@@ -140,17 +143,20 @@ def _default_budget(T: int, V: int, es: int) -> int:
 
 
 def _kept_plan(T: int, n: int, H: int, V: int,
-               accumulator: bool = False) -> Tuple[int, int, int, bool]:
+               accumulator: bool = False,
+               ldw: Optional[int] = None) -> Tuple[int, int, int, bool]:
     """(columns, logits bytes, backward scratch bytes, pays) of a bf16 call
     that keeps logits from the forward to the backward (mt_flce_logits_plan),
     columns 0 when none fit.  The default budget counts the bytes by which a
     bf16 weight gradient is smaller than the fp32 one of the other paths (no
     such gradient exists with an accumulator); a budget set by
-    MT_FLCE_BWD_BUDGET_BYTES is taken as it stands."""
+    MT_FLCE_BWD_BUDGET_BYTES is taken as it stands.  ldw: pitch of the weight's
+    rows (default H)."""
     room = int(int(os.environ.get(BACKWARD_BUDGET_ENV, "0")) == 0)
     cols, lb, sb, pays = ctypes.c_int64(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int()
-    check(load().mt_flce_logits_plan(T, n, H, V, MT_DTYPE_BF16, _default_budget(T, V, 2), room,
-                                     int(accumulator), ctypes.byref(cols), ctypes.byref(lb), ctypes.byref(sb),
+    check(load().mt_flce_logits_plan(T, n, H, V, H if ldw is None else ldw, MT_DTYPE_BF16,
+                                     _default_budget(T, V, 2), room, int(accumulator),
+                                     ctypes.byref(cols), ctypes.byref(lb), ctypes.byref(sb),
                                      ctypes.byref(pays)), "mt_flce_logits_plan")
     return cols.value, lb.value, sb.value, bool(pays.value)
 
@@ -302,9 +308,13 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         keep = (dt == MT_DTYPE_BF16 and len(parts) == 1 and n_tot > 0
                 and _fused_mode() == "auto")
         if keep and allow_unit and grad_scale is None:
-            kept = _kept_plan(T, n_tot, H, V)
+            kept = _kept_plan(T, n_tot, H, V, False, W.stride(0))
             kept = kept if kept[3] else None
-        if kept is None and dt == MT_DTYPE_BF16 and n_tot > 0 and (grad_scale is not None or allow_unit):
+        # (the fused path takes the whole weight, gaps between its rows included,
+        # through one buffer; the general one takes it in vocabulary blocks)
+        if (kept is None and dt == MT_DTYPE_BF16 and n_tot > 0
+                and (grad_scale is not None or allow_unit)
+                and V * W.stride(0) * 2 <= lib.mt_flce_max_buffer_bytes()):
             # whether it pays is asked at 5% of the logits, also where
             # MIN_BUDGET gives more: the general path's blocks grow with it,
             # and its dX carries one rounding less than the fused path's
@@ -325,7 +335,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                     elif keep and _general_pays(T, n_tot, H, V):
                         ctx.path = "general"
         if keep and acc and recording and ctx.path == "general":
-            kept = _kept_plan(T, n_tot, H, V, True)
+            kept = _kept_plan(T, n_tot, H, V, True, W.stride(0))
             kept = kept if kept[3] else None
         ctx.dw_accumulator = dw_accumulator
         ctx.meta = (float(softcap), hidden.shape, dt)
@@ -396,7 +406,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                 # it under what the budget leaves of that
                 left = _default_budget(T, V, 2) - ws_bytes
                 if left > 0:
-                    plan = backward_plan(T, n, H, V, X.dtype, budget_bytes=left, narrow=True)
+                    plan = backward_plan(T, n, H, V, X.dtype, left, True, W.stride(0))
             if plan is not None and plan[0] >= n and plan[1] < V:
                 # one row block in the backward: the forward keeps the first
                 # vocabulary block's exponentials in that backward's G block,
@@ -474,7 +484,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             dW = acc if acc is not None else torch.empty((V, H), dtype=torch.float32, device=dev)
             for r, (t0, t1, n, ri, rl, lse) in enumerate(rngs):
                 budget = _default_budget(t1 - t0, V, X.element_size())
-                C, Cv, ws_bytes = backward_plan(t1 - t0, n, H, V, X.dtype, budget)
+                C, Cv, ws_bytes = backward_plan(t1 - t0, n, H, V, X.dtype, budget, ldw=W.stride(0))
                 if dt == MT_DTYPE_F32:  # what the budget leaves holds planes of a split dX
                     ws_bytes = max(ws_bytes, min(budget, ws_bytes + 8 * C * H * 4))
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
@@ -600,7 +610,7 @@ def _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX,
     if one:
         n = rngs[0][2]
         plan = keep[:3] if keep is not None else backward_plan(
-            T, n, H, V, X.dtype, _default_budget(T, V, 2), narrow=True)
+            T, n, H, V, X.dtype, _default_budget(T, V, 2), True, W.stride(0))
     if one and plan[0] >= n:
         (t0, t1, n, ri, rl, lse), (C, Cv, ws) = rngs[0], plan
         if keep is not None:
@@ -631,7 +641,8 @@ def _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX,
         # plan of mt_flce_backward_tiles itself (dX's accumulator and X^T in
         # the workspace)
         C, Cv, ws_bytes = (plan if one else backward_plan(t1 - t0, n, H, V, X.dtype,
-                                                          _default_budget(t1 - t0, V, 2)))
+                                                          _default_budget(t1 - t0, V, 2),
+                                                          ldw=W.stride(0)))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         gr = g[t0:t1] if gstride else g
         check(lib.mt_flce_backward_tiles(_p(X[t0:t1]), _p(W), t1 - t0, H, V, X.stride(0),

@@ -414,3 +414,39 @@ def test_binding_declares_every_argument():
         decl = re.search(r"\b" + name + r"\s*\(([^)]*)\)", text).group(1)
         want = [a for a in decl.split(",") if a.strip() and a.strip() != "void"]
         assert len(args) == len(want), name
+
+
+@pytest.mark.parametrize("T,n,H,V,ldw", [
+    (4096, 2867, 8192, 152064, 16384),   # the whole weight fits one buffer at pitch H, not at ldw
+    (4096, 2868, 4096, 128256, 20480),
+    (256, 200, 4096, 128256, 65536),     # few rows: the budget alone would take every column
+    (300, 200, 64, 5000, 64),
+])
+def test_plans_keep_a_strided_weight_within_one_buffer(T, n, H, V, ldw):
+    """Every plan the host layer makes for rows ldw apart is one that its entry
+    accepts: a block's rows, gaps included, stay within one buffer's reach.
+    (The entries' own checks, reached with a logits buffer too small, tell the
+    two refusals apart before any launch.)"""
+    from mini_trainer_amd.flce import _default_budget, _kept_plan
+
+    lib = _lib.load()
+    reach = lib.mt_flce_max_buffer_bytes()
+    for acc in (False, True):
+        cols, lb, sb, _ = _kept_plan(T, n, H, V, acc, ldw)
+        assert cols % 256 == 0 and min(cols, V) * ldw * 2 <= reach
+        if cols:
+            args = (16, 16, T, H, V, H, ldw, 1, 0.0, 16, 16, n, 16, 16, 16, 1 << 40)
+            assert lib.mt_flce_forward_logits(*args, None, cols, lb, None) == 1
+            assert lib.mt_flce_forward_logits(*args, 16, cols, lb - 1, None) == 1
+    for narrow in (False, True):
+        C, Cv, ws = backward_plan(T, n, H, V, torch.bfloat16, _default_budget(T, V, 2), narrow, ldw)
+        assert C > 0 and min(Cv, -(-V // 256) * 256) * ldw * 2 <= reach
+    # at pitch H the plans are those without a pitch
+    assert _kept_plan(T, n, H, V, False, H) == _kept_plan(T, n, H, V)
+    c, cv, ws = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_size_t()
+    for fn, narrow in ((lib.mt_flce_backward_plan, False), (lib.mt_flce_backward_narrow_plan, True)):
+        assert fn(T, n, H, V, 1, 0, ctypes.byref(c), ctypes.byref(cv), ctypes.byref(ws)) == 0
+        assert (c.value, cv.value, ws.value) == backward_plan(T, n, H, V, torch.bfloat16, 0, narrow)
+    # a pitch below H is refused
+    assert lib.mt_flce_backward_plan_pitch(T, n, H, V, H - 8, 1, 0, 0, ctypes.byref(c),
+                                           ctypes.byref(cv), ctypes.byref(ws)) == 1
