@@ -858,13 +858,16 @@ class _CrossEntropyNone(torch.autograd.Function):
         lse = torch.empty(T, dtype=torch.float32, device=dev)
         # the targets are checked first, so that the host waits for that alone
         # and launches what follows while the logits are being read
-        status = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        status = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
         check(lib.mt_ce_check_targets(_p(tgt), T, V, int(ignore_index), _p(status), _stream(dev)),
               "mt_ce_check_targets")
         checked = torch.cuda.current_stream(dev).record_event()
-        check(lib.mt_ce_forward_checked(_p(L), T, V, L.stride(0), dt, _p(tgt), int(ignore_index),
-                                        _p(loss), _p(lse), _stream(dev)), "mt_ce_forward_checked")
-        checked.synchronize()
+        try:
+            check(lib.mt_ce_forward_checked(_p(L), T, V, L.stride(0), dt, _p(tgt),
+                                            int(ignore_index), _p(loss), _p(lse), _stream(dev)),
+                  "mt_ce_forward_checked")
+        finally:
+            checked.synchronize()  # the check writes `status` until then
         if int(status[0]) != 0:
             bad = tgt[(tgt != ignore_index) & ((tgt < 0) | (tgt >= V))][0].item()
             raise IndexError(f"Target {bad} is out of bounds.")
