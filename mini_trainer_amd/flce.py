@@ -388,17 +388,20 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             ws_bytes = lib.mt_flce_forward_workspace_bytes(t1 - t0, n, H, V, dt)
             if kept is not None:
                 # the logits live from here to the backward (or until the
-                # loss's graph is freed, when no backward follows)
+                # loss's graph is freed, when no backward follows), as a saved
+                # tensor like any activation: hooks that offload or recompute
+                # those (checkpointing) move or drop it
                 cols, logits_bytes, scratch_bytes, _ = kept
-                logits = torch.empty(logits_bytes, dtype=torch.uint8, device=dev)
+                logits = torch.empty((logits_bytes // (2 * cols), cols), dtype=torch.bfloat16,
+                                     device=dev)
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
                 check(lib.mt_flce_forward_logits(_p(Xr), _p(W), T, H, V, X.stride(0), W.stride(0),
                                                  dt, float(softcap), _p(ri), _p(rl), n, _p(lr),
                                                  _p(lse), _p(ws), ws_bytes, _p(logits), cols,
                                                  logits_bytes, _stream(dev)),
                       "mt_flce_forward_logits")
-                ctx.logits = (logits, cols, scratch_bytes)
-                del ws, logits
+                ctx.logits = (cols, scratch_bytes, logits.data_ptr())
+                del ws
                 continue
             if (dt == MT_DTYPE_BF16 and allow_unit and float(softcap) == 0.0 and n > 0
                     and len(parts) == 1):
@@ -427,13 +430,14 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                                           dt, float(softcap), _p(ri), _p(rl), n, _p(lr), _p(lse),
                                           _p(ws), ws_bytes, _stream(dev)), "mt_flce_forward")
             del ws
-        ctx.save_for_backward(X, W, *[t for p, lse in zip(parts, lses) for t in (p[2], p[3], lse)])
+        ctx.save_for_backward(X, W, *[t for p, lse in zip(parts, lses) for t in (p[2], p[3], lse)],
+                              *([] if kept is None else [logits]))
         return loss.view(hidden.shape[:-1])
 
     @staticmethod
-    def _range_tensors(ctx):
-        """X, W and [(t0, t1, n, row_index, row_label, lse)] per range."""
-        saved = ctx.saved_tensors
+    def _range_tensors(ctx, saved):
+        """X, W and [(t0, t1, n, row_index, row_label, lse)] per range of the
+        saved tensors."""
         X, W, rest = saved[0], saved[1], saved[2:]
         out = []
         for i, (t0, t1, n) in enumerate(ctx.ranges):
@@ -446,7 +450,8 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             return _FusedLinearCrossEntropyNone._backward_fused(ctx, grad_loss)
         if ctx.path == "fused_unit":
             return _FusedLinearCrossEntropyNone._backward_fused_unit(ctx, grad_loss)
-        X, W, rngs = _FusedLinearCrossEntropyNone._range_tensors(ctx)
+        saved = ctx.saved_tensors
+        X, W, rngs = _FusedLinearCrossEntropyNone._range_tensors(ctx, saved)
         softcap, hshape, dt = ctx.meta
         need_x, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         acc = ctx.dw_accumulator
@@ -461,18 +466,22 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         dX = torch.empty((T, H), dtype=X.dtype, device=dev)
         logits, ctx.logits = ctx.logits, None
         if logits is not None:
-            # the first backward: G from the logits its forward kept
-            (t0, t1, n, ri, rl, lse), (kept, cols, scratch_bytes) = rngs[0], logits
+            # the first backward: G from the logits its forward kept, in place
+            # (a second one finds G there and recomputes)
+            (t0, t1, n, ri, rl, lse), (cols, scratch_bytes, ptr) = rngs[0], logits
+            kept = saved[-1].contiguous()
             scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
             out = None if acc is not None else torch.empty((V, H), dtype=torch.bfloat16, device=dev)
             check(lib.mt_flce_backward_logits(_p(X), _p(W), T, H, V, X.stride(0), W.stride(0), dt,
                                               softcap, _p(ri), _p(rl), n, _p(lse), _p(g), gstride,
                                               _p(dX), dX.stride(0), _p(out), V * H * 2, _p(acc),
                                               acc.stride(0) if acc is not None else 0, _p(kept),
-                                              cols, kept.numel(), _p(scratch), scratch_bytes,
-                                              _stream(dev)),
+                                              cols, kept.numel() * 2, _p(scratch),
+                                              scratch_bytes, _stream(dev)),
                   "mt_flce_backward_logits")
-            del kept, scratch, logits
+            if kept.data_ptr() == ptr:  # (not a copy that a hook made)
+                kept.untyped_storage().resize_(0)  # graph retained: it would outlive this
+            del kept, scratch
             grad_w = out if need_w else None
         elif acc is None and dt == MT_DTYPE_BF16:
             # dW in bf16; the first backward takes the exponentials its
@@ -544,7 +553,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
 
     @staticmethod
     def _backward_fused_unit(ctx, grad_loss):
-        X, W, rngs = _FusedLinearCrossEntropyNone._range_tensors(ctx)
+        X, W, rngs = _FusedLinearCrossEntropyNone._range_tensors(ctx, ctx.saved_tensors)
         softcap, hshape, dt = ctx.meta
         if ctx.fused_consumed:
             raise RuntimeError(
