@@ -161,6 +161,23 @@ def _kept_plan(T: int, n: int, H: int, V: int,
     return cols.value, lb.value, sb.value, bool(pays.value)
 
 
+def _kept_logits(T: int, n: int, H: int, V: int, accumulator: bool, ldw: int,
+                 dev: torch.device) -> Optional[Tuple[torch.Tensor, int, int, torch.Tensor]]:
+    """(buffer of the logits, columns, backward scratch bytes, forward
+    workspace) where keeping them pays and the device has the room, else None:
+    the other paths then run as if it did not pay."""
+    cols, nbytes, scratch_bytes, pays = _kept_plan(T, n, H, V, accumulator, ldw)
+    if not pays:
+        return None
+    try:
+        logits = torch.empty((nbytes // (2 * cols), cols), dtype=torch.bfloat16, device=dev)
+        ws = torch.empty(load().mt_flce_forward_workspace_bytes(T, n, H, V, MT_DTYPE_BF16),
+                         dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        return None
+    return logits, cols, scratch_bytes, ws
+
+
 def _general_pays(T: int, n: int, H: int, V: int) -> bool:
     """Is the general path in the default budget expected to beat the fused
     one at 5% of the logits (mt_flce_general_pays)?"""
@@ -308,8 +325,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         keep = (dt == MT_DTYPE_BF16 and len(parts) == 1 and n_tot > 0
                 and _fused_mode() == "auto")
         if keep and allow_unit and grad_scale is None:
-            kept = _kept_plan(T, n_tot, H, V, False, W.stride(0))
-            kept = kept if kept[3] else None
+            kept = _kept_logits(T, n_tot, H, V, False, W.stride(0), dev)
         # (the fused path takes the whole weight, gaps between its rows included,
         # through one buffer; the general one takes it in vocabulary blocks)
         if (kept is None and dt == MT_DTYPE_BF16 and n_tot > 0
@@ -335,8 +351,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                     elif keep and _general_pays(T, n_tot, H, V):
                         ctx.path = "general"
         if keep and acc and recording and ctx.path == "general":
-            kept = _kept_plan(T, n_tot, H, V, True, W.stride(0))
-            kept = kept if kept[3] else None
+            kept = _kept_logits(T, n_tot, H, V, True, W.stride(0), dev)
         ctx.dw_accumulator = dw_accumulator
         ctx.meta = (float(softcap), hidden.shape, dt)
         lses = []
@@ -384,25 +399,21 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
             lse = torch.empty(n, dtype=torch.float32, device=dev)
             lses.append(lse)
             Xr, lr = (X, loss) if t1 - t0 == T else (X[t0:t1], loss[t0:t1])
-            plan = None
-            ws_bytes = lib.mt_flce_forward_workspace_bytes(t1 - t0, n, H, V, dt)
             if kept is not None:
                 # the logits live from here to the backward (or until the
                 # loss's graph is freed, when no backward follows), as a saved
                 # tensor like any activation: hooks that offload or recompute
                 # those (checkpointing) move or drop it
-                cols, logits_bytes, scratch_bytes, _ = kept
-                logits = torch.empty((logits_bytes // (2 * cols), cols), dtype=torch.bfloat16,
-                                     device=dev)
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+                logits, cols, scratch_bytes, ws = kept
                 check(lib.mt_flce_forward_logits(_p(Xr), _p(W), T, H, V, X.stride(0), W.stride(0),
                                                  dt, float(softcap), _p(ri), _p(rl), n, _p(lr),
-                                                 _p(lse), _p(ws), ws_bytes, _p(logits), cols,
-                                                 logits_bytes, _stream(dev)),
+                                                 _p(lse), _p(ws), ws.numel(), _p(logits), cols,
+                                                 logits.numel() * 2, _stream(dev)),
                       "mt_flce_forward_logits")
                 ctx.logits = (cols, scratch_bytes, logits.data_ptr())
-                del ws
                 continue
+            plan = None
+            ws_bytes = lib.mt_flce_forward_workspace_bytes(t1 - t0, n, H, V, dt)
             if (dt == MT_DTYPE_BF16 and allow_unit and float(softcap) == 0.0 and n > 0
                     and len(parts) == 1):
                 # the kept block sits beside the forward's own workspace: plan
@@ -431,7 +442,7 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                                           _p(ws), ws_bytes, _stream(dev)), "mt_flce_forward")
             del ws
         ctx.save_for_backward(X, W, *[t for p, lse in zip(parts, lses) for t in (p[2], p[3], lse)],
-                              *([] if kept is None else [logits]))
+                              *([] if kept is None else [kept[0]]))
         return loss.view(hidden.shape[:-1])
 
     @staticmethod
@@ -463,48 +474,27 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         V = W.shape[0]
         dev = X.device
         g, gstride = _grad_vector(grad_loss, T)
-        dX = torch.empty((T, H), dtype=X.dtype, device=dev)
         logits, ctx.logits = ctx.logits, None
+        done = None
         if logits is not None:
             # the first backward: G from the logits its forward kept, in place
             # (a second one finds G there and recomputes)
-            (t0, t1, n, ri, rl, lse), (cols, scratch_bytes, ptr) = rngs[0], logits
-            kept = saved[-1].contiguous()
-            scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
-            out = None if acc is not None else torch.empty((V, H), dtype=torch.bfloat16, device=dev)
-            check(lib.mt_flce_backward_logits(_p(X), _p(W), T, H, V, X.stride(0), W.stride(0), dt,
-                                              softcap, _p(ri), _p(rl), n, _p(lse), _p(g), gstride,
-                                              _p(dX), dX.stride(0), _p(out), V * H * 2, _p(acc),
-                                              acc.stride(0) if acc is not None else 0, _p(kept),
-                                              cols, kept.numel() * 2, _p(scratch),
-                                              scratch_bytes, _stream(dev)),
-                  "mt_flce_backward_logits")
-            if kept.data_ptr() == ptr:  # (not a copy that a hook made)
-                kept.untyped_storage().resize_(0)  # graph retained: it would outlive this
-            del kept, scratch
-            grad_w = out if need_w else None
-        elif acc is None and dt == MT_DTYPE_BF16:
-            # dW in bf16; the first backward takes the exponentials its
-            # forward kept
-            keep, ctx.keep = ctx.keep, None
-            grad_w = _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX, keep=keep)
-            grad_w = grad_w if need_w else None
+            done = _backward_kept_logits(lib, X, W, rngs[0], g, gstride, softcap, acc, saved[-1],
+                                         *logits)
+        saved = logits = None
+        if done is not None:
+            dX, grad_w = done
         else:
-            dW = acc if acc is not None else torch.empty((V, H), dtype=torch.float32, device=dev)
-            for r, (t0, t1, n, ri, rl, lse) in enumerate(rngs):
-                budget = _default_budget(t1 - t0, V, X.element_size())
-                C, Cv, ws_bytes = backward_plan(t1 - t0, n, H, V, X.dtype, budget, ldw=W.stride(0))
-                if dt == MT_DTYPE_F32:  # what the budget leaves holds planes of a split dX
-                    ws_bytes = max(ws_bytes, min(budget, ws_bytes + 8 * C * H * 4))
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-                gr = g[t0:t1] if gstride else g
-                check(lib.mt_flce_backward(_p(X[t0:t1]), _p(W), t1 - t0, H, V, X.stride(0),
-                                           W.stride(0), dt, softcap, _p(ri), _p(rl), n, _p(lse),
-                                           _p(gr), gstride, _p(dX[t0:t1]), dX.stride(0), _p(dW),
-                                           dW.stride(0), int(acc is not None or r > 0), C, Cv,
-                                           _p(ws), ws_bytes, _stream(dev)), "mt_flce_backward")
-                del ws
-            grad_w = _weight_grad_in_dtype(dW, W.dtype) if (need_w and acc is None) else None
+            dX = torch.empty((T, H), dtype=X.dtype, device=dev)
+            if acc is None and dt == MT_DTYPE_BF16:
+                # dW in bf16; the first backward takes the exponentials its
+                # forward kept
+                keep, ctx.keep = ctx.keep, None
+                grad_w = _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX, keep=keep)
+            else:
+                grad_w = _backward_fp32_weight(lib, X, W, rngs, g, gstride, softcap, dX, dt, acc,
+                                               need_w)
+        grad_w = grad_w if need_w else None
         grad_x = dX.view(hshape) if need_x else None
         return (grad_x, grad_w) + none
 
@@ -588,6 +578,42 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
         return (grad_x, grad_w) + (None,) * 9
 
 
+def _backward_kept_logits(lib, X, W, rng, g, gstride, softcap, acc, kept, cols, scratch_bytes,
+                          ptr) -> Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]]:
+    """dX and the weight gradient in bf16 (None with an accumulator) from the
+    logits that the forward kept at `ptr`, whose memory is given back.  None
+    where the device lacks the room beside them: the caller then recomputes,
+    in theirs."""
+    T, H = X.shape
+    V = W.shape[0]
+    dev = X.device
+    t0, t1, n, ri, rl, lse = rng
+    try:
+        dX = torch.empty((T, H), dtype=X.dtype, device=dev)
+        scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
+        out = None if acc is not None else torch.empty((V, H), dtype=torch.bfloat16, device=dev)
+        kept = kept.contiguous()
+    except torch.OutOfMemoryError:
+        _release(kept, ptr)
+        return None
+    check(lib.mt_flce_backward_logits(_p(X), _p(W), T, H, V, X.stride(0), W.stride(0),
+                                      MT_DTYPE_BF16, softcap, _p(ri), _p(rl), n, _p(lse), _p(g),
+                                      gstride, _p(dX), dX.stride(0), _p(out), V * H * 2, _p(acc),
+                                      acc.stride(0) if acc is not None else 0, _p(kept), cols,
+                                      kept.numel() * 2, _p(scratch), scratch_bytes, _stream(dev)),
+          "mt_flce_backward_logits")
+    _release(kept, ptr)
+    return dX, out
+
+
+def _release(kept: torch.Tensor, ptr: int) -> None:
+    """Give back the memory of the logits that the forward kept at `ptr` (the
+    node holds the tensor until it is freed); not of a copy that a saved-tensor
+    hook made."""
+    if kept.data_ptr() == ptr:
+        kept.untyped_storage().resize_(0)
+
+
 def _narrowed_view(dW: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """The [V, H] gradient in `dtype` that mt_flce_scale_grads narrowed into
     the first bytes of the fp32 dW's own storage (bf16 row r at element
@@ -661,6 +687,30 @@ def _backward_bf16_weight(lib, X, W, rngs, g, gstride, softcap, dX,
                                          _stream(dev)), "mt_flce_backward_tiles")
         del ws
     return dWt.narrow(torch.ones(1, dtype=torch.float32, device=dev))
+
+
+def _backward_fp32_weight(lib, X, W, rngs, g, gstride, softcap, dX, dt, acc,
+                          need_w) -> Optional[torch.Tensor]:
+    """The backward into dX and an fp32 weight gradient: added into acc
+    (returns None), or returned in the weight's dtype (None unless need_w)."""
+    T, H = X.shape
+    V = W.shape[0]
+    dev = X.device
+    dW = acc if acc is not None else torch.empty((V, H), dtype=torch.float32, device=dev)
+    for r, (t0, t1, n, ri, rl, lse) in enumerate(rngs):
+        budget = _default_budget(t1 - t0, V, X.element_size())
+        C, Cv, ws_bytes = backward_plan(t1 - t0, n, H, V, X.dtype, budget, ldw=W.stride(0))
+        if dt == MT_DTYPE_F32:  # what the budget leaves holds planes of a split dX
+            ws_bytes = max(ws_bytes, min(budget, ws_bytes + 8 * C * H * 4))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        gr = g[t0:t1] if gstride else g
+        check(lib.mt_flce_backward(_p(X[t0:t1]), _p(W), t1 - t0, H, V, X.stride(0), W.stride(0),
+                                   dt, softcap, _p(ri), _p(rl), n, _p(lse), _p(gr), gstride,
+                                   _p(dX[t0:t1]), dX.stride(0), _p(dW), dW.stride(0),
+                                   int(acc is not None or r > 0), C, Cv, _p(ws), ws_bytes,
+                                   _stream(dev)), "mt_flce_backward")
+        del ws
+    return _weight_grad_in_dtype(dW, W.dtype) if (need_w and acc is None) else None
 
 
 def _weight_grad_in_dtype(dW: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
