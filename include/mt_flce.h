@@ -390,9 +390,9 @@ int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V,
  * or, with dW_acc (fp32 rows of pitch lddw_acc), added into that instead.
  * grad_loss and grad_stride as in mt_flce_backward; one scalar (stride 0) is
  * applied to the fp32 sums when dW goes to dW_out, else it is part of G, as a
- * per-token gradient is.  A scratch
- * smaller than planned (but with X^T, the queue and, for keep_cols < V, the
- * accumulator) means fewer dX slices.  n_valid >= 1, H a multiple of 8.
+ * per-token gradient is.  The scratch's size tells the number of dX slices: the
+ * planned one at the planned size, fewer in less (but X^T, the queue and, for
+ * keep_cols < V, the accumulator must fit).  n_valid >= 1, H a multiple of 8.
  * Replaces the same reference interface as mt_flce_forward and
  * mt_flce_backward (none_reduction_losses.py:16-23, whose Liger forward keeps
  * each chunk's logits to form the gradients from).

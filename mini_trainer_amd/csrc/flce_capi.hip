@@ -1551,8 +1551,9 @@ KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, int64_t ldw, size
   const int64_t reach = (int64_t)(std::min(lim / ((uint64_t)C * 2), lim / ((uint64_t)ldw * 2)) / 256 * 256);
   for (int64_t S = 1; S <= 32; S *= 2) {
     for (int blocks = 0; blocks < 2; ++blocks) {
-      const size_t other = std::max(kept_scratch(C, H, S, blocks != 0, acc), fwd);
-      if (other > have) continue;
+      const size_t own = kept_scratch(C, H, S, blocks != 0, acc), other = std::max(own, fwd);
+      // (slices whose planes are the size of one slice's tiles: see kept_slices_in)
+      if (other > have || (S > 1 && own == kept_scratch(C, H, 1, blocks != 0, acc))) continue;
       int64_t cols = std::min<int64_t>((int64_t)((have - other) / ((size_t)C * 2)) / 256 * 256, reach);
       if (blocks == 0 && cols < Vp) continue;  // several blocks
       cols = std::min(cols, blocks ? Vp - 256 : Vp);
@@ -1572,10 +1573,15 @@ KeptPlan plan_kept(int64_t T, int64_t N, int64_t H, int64_t V, int64_t ldw, size
   return best;
 }
 
-// The most slices (a power of two) whose planes fit a scratch of `bytes`.
-int64_t kept_slices_in(int64_t C, int64_t H, bool blocks, bool acc, size_t bytes) {
+// The slices wanted in a scratch of `bytes`: one where that is one slice's size
+// (its tiled accumulator is wider than H and would hold several planes: 4 at H
+// = 64), else the most (a power of two, 256 columns each) that fit.  Of the
+// planned scratch this is the planned number.
+int64_t kept_slices_in(int64_t C, int64_t H, int64_t V, int64_t cols, bool acc, size_t bytes) {
+  const bool blocks = cols < V;
+  if (bytes == kept_scratch(C, H, 1, blocks, acc)) return 1;
   int64_t S = 32;
-  while (S > 1 && kept_scratch(C, H, S, blocks, acc) > bytes) S /= 2;
+  while (S > 1 && (kept_scratch(C, H, S, blocks, acc) > bytes || std::min(cols, V) / S < 256)) S /= 2;
   return S;
 }
 
@@ -1588,7 +1594,7 @@ int launch_backward_logits(const void* X, const void* W, int64_t Tn, int64_t H, 
   const bool acc = lddw_acc > 0;  // add into fp32 rows of that pitch
   const int64_t C = round_up(N, 256), nb = cdiv(V, cols);
   const int64_t ldg_b = cols * 2, ldxt_b = C * 2;
-  const DxSplit split = kept_split(cols, V, kept_slices_in(C, H, nb > 1, acc, scratch_bytes));
+  const DxSplit split = kept_split(cols, V, kept_slices_in(C, H, V, cols, acc, scratch_bytes));
   char* XcT = scratch;
   uint32_t* queue = reinterpret_cast<uint32_t*>(scratch + align_up((size_t)H * C * 2));
   float* one = reinterpret_cast<float*>(queue + kQueueWords);
