@@ -1756,8 +1756,10 @@ int mt_flce_prepare(const int64_t* labels, int64_t T, int64_t V, int64_t ignore_
   if (V <= 0 || V > INT32_MAX) return fail(MT_ERR_INVALID_ARGUMENT, "V=%lld out of range", (long long)V);
   if (!counts || (T > 0 && (!labels || !row_index || !row_label)))
     return fail(MT_ERR_INVALID_ARGUMENT, "null pointer argument");
-  hipLaunchKernelGGL(prepare_kernel, dim3((uint32_t)std::max<int64_t>(1, cdiv(T, kPrepLabels))), dim3(1024), 0, (hipStream_t)stream, labels, T, V,
-                     ignore_index, shift, row_index, row_label, counts);
+  const int64_t span = round_up(std::max<int64_t>(1, cdiv(T, kPrepBlocks)), kPrepLabels);
+  hipLaunchKernelGGL(prepare_kernel, dim3((uint32_t)std::max<int64_t>(1, cdiv(T, span))), dim3(1024), 0,
+                     (hipStream_t)stream, labels, T, V, ignore_index, shift, span, row_index, row_label,
+                     counts);
   return check_launch("prepare_kernel");
 }
 

@@ -422,7 +422,8 @@ __global__ __launch_bounds__(256) void zero_scatter_f32_kernel(float* loss, cons
     loss[rows[i]] = 0.0f;
 }
 
-// Valid-row compaction, one workgroup of 1024 threads per 4096 labels.
+// Valid-row compaction, one workgroup of 1024 threads per `span` labels (a
+// multiple of 4096).
 //   row_index[0 .. N)    positions t with a valid label, ascending
 //   row_index[N .. T)    every other position (descending from the end)
 //   row_label[0 .. N)    their labels
@@ -430,14 +431,19 @@ __global__ __launch_bounds__(256) void zero_scatter_f32_kernel(float* loss, cons
 // Each workgroup counts the labels before its own by itself (they come from L2;
 // independent loads), so no workgroup waits for another and no scratch is
 // needed; the last one writes counts.  Bound by latency: one workgroup walking
-// all labels, a scan and two barriers per 4096, took 58 us for 53k labels.
-constexpr int kPrepItems = 4, kPrepLabels = 1024 * kPrepItems;
+// all labels, a scan and two barriers per 4096, took 58 us for 53k labels.  The
+// labels read again grow with the workgroups (1/2 T each on average), so there
+// are at most kPrepBlocks, which from 2^20 labels on take longer spans: 16.8M
+// labels 13.0 ms in one workgroup, 34 ms at 4096 apiece, 2.7 ms in 256; 53k
+// labels 41 us in one, 13 us at 4096 apiece.
+constexpr int kPrepItems = 4, kPrepLabels = 1024 * kPrepItems, kPrepBlocks = 256;
 __global__ __launch_bounds__(1024) void prepare_kernel(const int64_t* labels, int64_t T, int64_t V,
-                                                       int64_t ignore, int shift, int32_t* row_index,
-                                                       int32_t* row_label, int32_t* counts) {
+                                                       int64_t ignore, int shift, int64_t span,
+                                                       int32_t* row_index, int32_t* row_label,
+                                                       int32_t* counts) {
   __shared__ int32_t wsum_v[16], wpre_v[16], wbad[16], wfirst[16];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int64_t start = (int64_t)blockIdx.x * kPrepLabels;
+  const int64_t start = (int64_t)blockIdx.x * span, end = min(start + span, T);
   auto label = [&](int64_t t) __attribute__((always_inline)) {
     return shift ? (t + 1 < T ? labels[t + 1] : ignore) : labels[t];
   };
@@ -463,69 +469,77 @@ __global__ __launch_bounds__(1024) void prepare_kernel(const int64_t* labels, in
       see_bad(k, t0 + j * 1024);
     }
   }
-  int32_t y[kPrepItems];
-  uint32_t vmask = 0, mmask = 0;
 #pragma unroll
-  for (int j = 0; j < kPrepItems; ++j) {
-    const int64_t t = start + tid * kPrepItems + j;
-    y[j] = 0;
-    if (t >= T) continue;
-    const int64_t lab = label(t);
-    const int k = kind(lab);
-    see_bad(k, t);
-    if (k == 1) {
-      vmask |= 1u << j;
-      y[j] = (int32_t)lab;
-    } else {
-      mmask |= 1u << j;
+  for (int o = 32; o > 0; o >>= 1) pre_v += __shfl_xor(pre_v, o);
+  if (lane == 63) wpre_v[wid] = pre_v;
+  int32_t base = 0;  // valid before the labels at hand
+  for (int64_t c0 = start; c0 < end || c0 == start; c0 += kPrepLabels) {
+    int32_t y[kPrepItems];
+    uint32_t vmask = 0, mmask = 0;
+#pragma unroll
+    for (int j = 0; j < kPrepItems; ++j) {
+      const int64_t t = c0 + tid * kPrepItems + j;
+      y[j] = 0;
+      if (t >= end) continue;
+      const int64_t lab = label(t);
+      const int k = kind(lab);
+      see_bad(k, t);
+      if (k == 1) {
+        vmask |= 1u << j;
+        y[j] = (int32_t)lab;
+      } else {
+        mmask |= 1u << j;
+      }
     }
-  }
-  const int cv = __builtin_popcount(vmask);
-  int sv = cv;  // inclusive wave scan of the workgroup's own valid labels
+    const int cv = __builtin_popcount(vmask);
+    int sv = cv;  // inclusive wave scan of these 4096 labels' valid ones
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int up = __shfl_up(sv, o);
-    if (lane >= o) sv += up;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(sv, o);
+      if (lane >= o) sv += up;
+    }
+    if (c0 != start) __syncthreads();  // (the sums of the labels before have been read)
+    if (lane == 63) wsum_v[wid] = sv;
+    __syncthreads();
+    int32_t before = 0, own = 0;  // valid before this wave's labels, and in all
+    for (int w = 0; w < 16; ++w) {
+      if (w < wid) before += wsum_v[w];
+      own += wsum_v[w];
+      if (c0 == start) base += wpre_v[w];
+    }
+    int32_t ov = base + before + sv - cv;
+    int32_t om = (int32_t)(c0 + (int64_t)tid * kPrepItems) - ov;  // others before this thread's labels
+#pragma unroll
+    for (int j = 0; j < kPrepItems; ++j) {
+      const int32_t t = (int32_t)(c0 + tid * kPrepItems + j);
+      if (vmask & (1u << j)) {
+        row_index[ov] = t;
+        row_label[ov] = y[j];
+        ++ov;
+      } else if (mmask & (1u << j)) {
+        row_index[T - 1 - om] = t;
+        ++om;
+      }
+    }
+    base += own;
   }
+  if (blockIdx.x != gridDim.x - 1) return;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    pre_v += __shfl_xor(pre_v, o);
     bad += __shfl_xor(bad, o);
     first = min(first, __shfl_xor(first, o));
   }
   if (lane == 63) {
-    wsum_v[wid] = sv;
-    wpre_v[wid] = pre_v;
     wbad[wid] = bad;
     wfirst[wid] = first;
   }
   __syncthreads();
-  int32_t before = 0, own = 0, base = 0;  // valid before this wave's labels, in all, before the workgroup
-  for (int w = 0; w < 16; ++w) {
-    if (w < wid) before += wsum_v[w];
-    own += wsum_v[w];
-    base += wpre_v[w];
-  }
-  int32_t ov = base + before + sv - cv;
-  int32_t om = (int32_t)(start + (int64_t)tid * kPrepItems) - ov;  // others before this thread's labels
-#pragma unroll
-  for (int j = 0; j < kPrepItems; ++j) {
-    const int32_t t = (int32_t)(start + tid * kPrepItems + j);
-    if (vmask & (1u << j)) {
-      row_index[ov] = t;
-      row_label[ov] = y[j];
-      ++ov;
-    } else if (mmask & (1u << j)) {
-      row_index[T - 1 - om] = t;
-      ++om;
-    }
-  }
-  if (blockIdx.x == gridDim.x - 1 && tid == 0) {
+  if (tid == 0) {
     for (int w = 1; w < 16; ++w) {
       bad += wbad[w];
       first = min(first, wfirst[w]);
     }
-    counts[0] = base + own;
+    counts[0] = base;
     counts[1] = bad;
     counts[2] = bad ? first : -1;
     counts[3] = 0;

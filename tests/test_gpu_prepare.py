@@ -33,3 +33,12 @@ def test_compaction_matches_torch(gpu, T, mask, shift):
     assert counts.tolist() == [n, int(wrong.sum()), first, 0]
     assert torch.equal(ri[:n].cpu(), want) and torch.equal(rl[:n].cpu(), src[ok].int())
     assert torch.equal(ri[n:].cpu(), torch.nonzero(~ok).flatten().int().flip(0))
+
+
+@pytest.mark.parametrize("T,shift", [
+    (1 << 20, 0),                # 256 workgroups of 4096 labels
+    ((1 << 20) + 1, 1),          # two 4096s each, the last workgroup with one
+    (3 * (1 << 20) - 4097, 0),   # three each, a last one that ends within its second
+])
+def test_compaction_of_several_chunks_per_workgroup(gpu, T, shift):
+    test_compaction_matches_torch(gpu, T, 0.4, shift)
