@@ -450,3 +450,111 @@ def test_plans_keep_a_strided_weight_within_one_buffer(T, n, H, V, ldw):
     # a pitch below H is refused
     assert lib.mt_flce_backward_plan_pitch(T, n, H, V, H - 8, 1, 0, 0, ctypes.byref(c),
                                            ctypes.byref(cv), ctypes.byref(ws)) == 1
+
+
+def call_forward_logits(**kw):
+    a = dict(X=16, W=16, T=300, H=64, V=1000, ldx=64, ldw=64, dtype=1, softcap=0.0, ri=16, rl=16,
+             n=200, loss=16, lse=16, ws=16, wsb=1 << 30, logits=16, cols=1024,
+             lb=256 * 1024 * 2, stream=None)
+    a.update(kw)
+    return _lib.load().mt_flce_forward_logits(*a.values())
+
+
+def call_backward_logits(**kw):
+    a = dict(X=16, W=16, T=300, H=64, V=1000, ldx=64, ldw=64, dtype=1, softcap=0.0, ri=16, rl=16,
+             n=200, lse=16, grad=16, gstride=0, dX=16, lddx=64, out=16, outb=1000 * 64 * 2, acc=None,
+             lddw=0, logits=16, cols=1024, lb=256 * 1024 * 2, scratch=16, sb=1 << 30, stream=None)
+    a.update(kw)
+    return _lib.load().mt_flce_backward_logits(*a.values())
+
+
+@pytest.mark.parametrize("kw,code", [
+    (dict(dtype=0), 3),                  # bf16 only
+    (dict(dtype=7), 3),
+    (dict(n=301), 1),                    # n_valid > T
+    (dict(ldw=32), 1),
+    (dict(X=18), 1),
+    (dict(loss=None), 1),
+    (dict(lse=None), 1),
+    (dict(wsb=0), 2),
+    (dict(ws=24), 1),                    # misaligned
+    (dict(cols=0), 1),
+    (dict(cols=1000), 1),                # not a multiple of 256
+    (dict(cols=1280), 1),                # beyond V rounded up
+    (dict(lb=256 * 1024 * 2 - 1), 1),
+    (dict(logits=None), 1),
+    (dict(logits=24), 1),
+    (dict(n=1 << 20, T=1 << 20, V=1 << 20, cols=1 << 20, lb=1 << 62, wsb=1 << 50), 3),  # reach
+])
+def test_forward_logits_host_checks(kw, code):
+    assert call_forward_logits(**kw) == code
+    assert _lib.load().mt_flce_last_error()
+
+
+@pytest.mark.parametrize("kw,code", [
+    (dict(dtype=0), 3),
+    (dict(n=0), 1),                      # nothing was kept
+    (dict(n=301), 1),
+    (dict(lddx=56), 1),
+    (dict(lddx=68), 1),                  # pitch not whole 16-byte chunks
+    (dict(gstride=-1), 1),
+    (dict(outb=1000 * 64 * 2 - 1), 1),
+    (dict(out=None), 1),
+    (dict(acc=16, lddw=32), 1),          # accumulator pitch below H
+    (dict(acc=16, lddw=66), 1),
+    (dict(acc=24, lddw=64), 1),          # misaligned
+    (dict(dX=24), 1),
+    (dict(dX=None), 1),
+    (dict(grad=None), 1),
+    (dict(lse=None), 1),
+    (dict(cols=1000), 1),
+    (dict(lb=0), 1),
+    (dict(logits=None), 1),
+    (dict(scratch=None), 2),
+    (dict(sb=64 * 256 * 2), 2),          # X^T without the work queue
+    (dict(cols=512, sb=64 * 256 * 2 + 256 + 65536 * 4 - 1), 2),  # blocks: dX's tiles too
+    (dict(cols=512, acc=16, lddw=64, sb=64 * 256 * 2 + 256 + 64 * 256 * 4 - 1), 2),  # or rows
+])
+def test_backward_logits_host_checks(kw, code):
+    assert call_backward_logits(**kw) == code
+    assert _lib.load().mt_flce_last_error()
+
+
+def test_logits_plan_and_target_check_host_checks():
+    lib = _lib.load()
+    cols, lb, sb, pays = ctypes.c_int64(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int()
+    out = [ctypes.byref(x) for x in (cols, lb, sb, pays)]
+    assert lib.mt_flce_logits_plan(300, 200, 64, 1000, 64, 1, 0, 0, 0, *out) == 0
+    assert lib.mt_flce_logits_plan(300, 200, 64, 1000, 64, 0, 0, 0, 0, *out) == 3
+    assert lib.mt_flce_logits_plan(300, 301, 64, 1000, 64, 1, 0, 0, 0, *out) == 1
+    assert lib.mt_flce_logits_plan(300, 200, 64, 1000, 56, 1, 0, 0, 0, *out) == 1
+    assert lib.mt_flce_logits_plan(300, 200, 64, 1000, 64, 1, 0, 0, 0, *out[:3], None) == 1
+    # nothing to keep, or a width the kernels do not take: no columns
+    for n, H in ((0, 64), (200, 60)):
+        assert lib.mt_flce_logits_plan(300, n, H, 1000, H, 1, 1 << 30, 0, 0, *out) == 0
+        assert (cols.value, lb.value, sb.value, pays.value) == (0, 0, 0, 0)
+    assert lib.mt_flce_general_pays(300, 200, 64, 1000, 0, 0, 0, out[3]) == 3
+    assert lib.mt_flce_general_pays(300, 301, 64, 1000, 1, 0, 0, out[3]) == 1
+    assert lib.mt_flce_general_pays(300, 200, 64, 1000, 1, 0, 0, None) == 1
+    assert lib.mt_ce_check_targets(None, 4, 10, -100, 16, None) == 1
+    assert lib.mt_ce_check_targets(16, 4, 10, -100, None, None) == 1
+    assert lib.mt_ce_check_targets(16, -1, 10, -100, 16, None) == 1
+    assert lib.mt_ce_check_targets(None, 0, 10, -100, 16, None) == 0
+    assert lib.mt_ce_forward_checked(16, 4, 10, 10, 7, 16, -100, 16, 16, None) == 1
+    assert lib.mt_ce_forward_checked(16, 4, 10, 9, 1, 16, -100, 16, 16, None) == 1
+    assert lib.mt_ce_forward_checked(16, 4, 10, 10, 1, None, -100, 16, 16, None) == 1
+
+
+def test_general_path_is_preferred_where_its_blocks_gain():
+    """mt_flce_general_pays: a small vocabulary whose 5% of the logits holds a
+    few rows of exponentials, while the workspace floor holds the general
+    path's logits block whole; not under the same 5%, and not at a size whose
+    5% already holds long chunks."""
+    from mini_trainer_amd.flce import _general_pays
+
+    lib, pays = _lib.load(), ctypes.c_int()
+    assert _general_pays(11217, 10350, 760, 10337)
+    assert not _general_pays(65536, 45875, 4096, 128256)
+    for size in ((11217, 10350, 760, 10337), (65536, 45875, 4096, 128256)):
+        assert lib.mt_flce_general_pays(*size, 1, 0, 0, ctypes.byref(pays)) == 0
+        assert pays.value == 0

@@ -79,3 +79,21 @@ def test_slices_are_those_of_the_scratch(gpu, monkeypatch, H, slices):
     assert ("dx_bf16_kernel<split>" in rep) == (slices > 1)
     assert float((dX - rdX).norm()) <= 1e-2 * float(rdX.norm())
     assert float((dW - rdW).norm()) <= 1e-2 * float(rdW.norm())
+
+
+@pytest.mark.parametrize("T,H,V,cols,slices,acc", [
+    (3, 8, 1, 256, 1, False),           # the smallest: one row tile, one column
+    (700, 200, 1300, 1536, 1, False),   # all kept, tails in every dimension
+    (700, 200, 1300, 1536, 4, False),   # the same with dX slices
+    (700, 200, 1300, 1536, 4, True),
+    (300, 136, 5000, 1024, 1, False),   # blocks, a short last one
+    (300, 136, 5000, 1024, 1, True),
+    (520, 264, 12500, 6144, 8, False),  # a last block (212 columns) with fewer stages than slices
+    (520, 264, 12500, 6144, 8, True),
+])
+def test_guards_and_results(gpu, T, H, V, cols, slices, acc):
+    """Against the same roundings of the logits in 64 bits: G is rounded to
+    bf16 (2^-9 of each entry), so is a bf16 result."""
+    dX, dW, rdX, rdW = _call(gpu, T, H, V, cols, slices, acc)
+    assert float((dX - rdX).norm()) <= 2.0 ** -8 * float(rdX.norm())
+    assert float((dW - rdW).norm()) <= 2.0 ** -8 * float(rdW.norm())

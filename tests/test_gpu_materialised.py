@@ -72,3 +72,56 @@ def test_failed_launch_after_the_check(gpu, monkeypatch):
     assert waited
     monkeypatch.delenv("MT_FLCE_TEST_FAIL_LAUNCH")
     _matches(z, y, gpu)
+
+
+@pytest.mark.parametrize("dtype,T,V", [
+    (torch.float32, 24, 4099),        # one round of four vectors a thread and three columns
+    (torch.float32, 24, 12291),       # three rounds and three columns
+    (torch.float32, 24, 8192),        # whole rounds, rows aligned
+    (torch.bfloat16, 24, 8191),       # every alignment of a row, one column short of a round
+    (torch.bfloat16, 24, 8193),
+    (torch.bfloat16, 24, 32003),
+    (torch.bfloat16, 24, 16384),
+    (torch.float32, 5, 1),            # rows shorter than a vector
+    (torch.bfloat16, 24, 3),
+    (torch.float32, 1000, 64003),     # 256,012,000 bytes: past the caches, odd rows
+    (torch.bfloat16, 1000, 128001),   # 256,002,000 bytes: just past them
+    (torch.bfloat16, 1000, 127999),   # 255,998,000 bytes: just short of that
+])
+def test_row_lengths(gpu, dtype, T, V):
+    """Labels at a row's first and last columns and in between."""
+    z, y = _case(T, V, dtype, seed=V)
+    for t, c in enumerate((0, V - 1, min(1, V - 1), V // 2, max(0, V - 2))):
+        y[t] = c
+    _matches(z, y, gpu)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("ld,ldd", [(0, 0), (0, 1), (1, 0), (3, 2), (8, 16), (0, 5)])
+def test_gradient_of_another_pitch(gpu, dtype, ld, ldd):
+    """Logits and gradient rows of different pitches: those that start alike
+    within 16 bytes, and those that do not; what lies between the gradient's
+    rows is untouched."""
+    T, V = 24, 8193
+    z, y = _case(T, V, dtype, seed=1)
+    es = z.element_size()
+    code = {torch.float32: _lib.MT_DTYPE_F32, torch.bfloat16: _lib.MT_DTYPE_BF16}[dtype]
+    lib, s = _lib.load(), torch.cuda.current_stream(gpu).cuda_stream
+    src = torch.full((T, V + ld), float("nan"), dtype=dtype, device=gpu)
+    src[:, :V] = z.to(gpu)
+    out = torch.full((T, V + ldd), 7.0, dtype=dtype, device=gpu)
+    yd, w = y.to(gpu), torch.rand(T, device=gpu)
+    loss, lse = torch.empty(T, device=gpu), torch.empty(T, device=gpu)
+    _lib.check(lib.mt_ce_forward_checked(src.data_ptr(), T, V, V + ld, code, yd.data_ptr(), -100,
+                                         loss.data_ptr(), lse.data_ptr(), s), "ce_forward")
+    _lib.check(lib.mt_ce_backward(src.data_ptr(), T, V, V + ld, code, yd.data_ptr(), -100,
+                                  lse.data_ptr(), w.data_ptr(), 1, out.data_ptr(), V + ldd, s),
+               "ce_backward")
+    torch.cuda.synchronize()
+    ref = z.double().requires_grad_(True)
+    want = torch.nn.functional.cross_entropy(ref, y, reduction="none")
+    (want * w.double().cpu()).sum().backward()
+    torch.testing.assert_close(loss.double().cpu(), want.detach(), rtol=1e-5, atol=1e-5)
+    diff = (out[:, :V].double().cpu() - ref.grad).norm()
+    assert float(diff) <= (1e-5 if es == 4 else 2.0 ** -8) * float(ref.grad.norm())
+    assert bool((out[:, V:] == 7.0).all())
