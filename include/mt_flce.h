@@ -169,6 +169,8 @@ uint64_t mt_flce_max_buffer_bytes(void);
  * from different host threads -- race; serialise them.
  */
 size_t mt_flce_noalloc_scratch_bytes(void);
+/* The most of it that a call with n_valid valid rows uses (0: bad arguments). */
+size_t mt_flce_noalloc_used_bytes(int64_t n_valid, int64_t V, int dtype);
 int mt_flce_forward_noalloc(const void* X, const void* W, int64_t T, int64_t H,
                             int64_t V, int64_t ldx, int64_t ldw, int dtype,
                             float softcap, const int32_t* row_index,

@@ -1889,11 +1889,36 @@ int64_t noalloc_rows(int64_t n_valid, int64_t V, int es) {
   return lo;
 }
 
+// The plan of a chunk of cn <= rows = noalloc_rows() rows.  An fp32 chunk's
+// splits depend on its rows, and a shorter chunk may want so many more that its
+// partials outgrow the scratch (V = 143753: 45184 rows take 10.7 MB, the 42345
+// after three of them 42.5 MB): it then takes the splits of a full chunk, whose
+// partials fit.
+FwdPlan noalloc_plan(int64_t cn, int64_t rows, int64_t V, int es) {
+  FwdPlan p = plan_forward(cn, V, es);
+  if (forward_ws(p, cn) > kScratchBytes) {
+    const FwdPlan full = plan_forward(rows, V, es);
+    p.per = full.per;
+    p.splits = full.splits;
+  }
+  return p;
+}
+
 }  // namespace
 
 extern "C" {
 
 size_t mt_flce_noalloc_scratch_bytes(void) { return kScratchBytes; }
+
+size_t mt_flce_noalloc_used_bytes(int64_t n_valid, int64_t V, int dtype) {
+  const int es = esize_of(dtype);
+  if (!es || n_valid <= 0 || V <= 0 || n_valid > INT32_MAX || V > INT32_MAX) return 0;
+  const int64_t rows = noalloc_rows(n_valid, V, es);
+  size_t used = 0;
+  for (const int64_t cn : {std::min(rows, n_valid), rows > 0 ? n_valid % rows : 0})
+    if (cn > 0) used = std::max(used, forward_ws(noalloc_plan(cn, rows, V, es), cn));
+  return used;
+}
 
 uint64_t mt_flce_max_buffer_bytes(void) { return buffer_limit(); }
 
@@ -1927,7 +1952,7 @@ int mt_flce_forward_noalloc(const void* X, const void* W, int64_t T, int64_t H, 
   // own forward kernel first, so the scratch needs no clearing between calls
   for (int64_t c0 = 0; c0 < n_valid; c0 += rows) {
     const int64_t cn = std::min(rows, n_valid - c0);
-    const FwdPlan p = plan_forward(cn, V, es);
+    const FwdPlan p = noalloc_plan(cn, rows, V, es);
     if (dtype == MT_DTYPE_BF16)
       MT_TRY(launch_forward<__bf16>(X, W, T, H, V, ldx, ldw, softcap, row_index + c0, row_label + c0,
                                     cn, loss, lse + c0, p, ws, s));

@@ -558,3 +558,20 @@ def test_general_path_is_preferred_where_its_blocks_gain():
     for size in ((11217, 10350, 760, 10337), (65536, 45875, 4096, 128256)):
         assert lib.mt_flce_general_pays(*size, 1, 0, 0, ctypes.byref(pays)) == 0
         assert pays.value == 0
+
+
+def test_noalloc_chunks_fit_the_scratch():
+    """Every row chunk of the forward without allocation, the last and shorter
+    one included, keeps its partials within the static scratch: in fp32 a
+    chunk's splits of the vocabulary depend on its rows."""
+    lib = _lib.load()
+    scratch = lib.mt_flce_noalloc_scratch_bytes()
+    rng = np.random.default_rng(0)
+    sizes = [(177897, 143753), (745107, 954), (494664, 133465), (1, 1), (300, 1 << 20)]
+    sizes += [(int(np.exp(rng.uniform(0, np.log(3e6)))), int(np.exp(rng.uniform(0, np.log(3e5)))))
+              for _ in range(400)]
+    for n, V in sizes:
+        for dtype in (0, 1):
+            assert 0 < lib.mt_flce_noalloc_used_bytes(n, V, dtype) <= scratch, (n, V, dtype)
+    for bad in ((0, 10, 0), (-1, 10, 0), (10, 0, 1), (10, 10, 7), (1 << 40, 10, 0)):
+        assert lib.mt_flce_noalloc_used_bytes(*bad) == 0
