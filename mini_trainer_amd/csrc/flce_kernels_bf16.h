@@ -81,8 +81,8 @@ __device__ __forceinline__ uint32_t fwd_group(uint32_t tiles_m) { return tiles_m
 // registers; the unrolled whole-tile form spilled): the lane's 32 logits of
 // the row are rounded to bf16 once, stored to S (kStore = kStoreLogits,
 // before the softcap), soft-capped, masked past V, merged into the row's
-// running (max, sum) and scanned for the label (same arithmetic as
-// fwd_tile_epilogue).
+// running (max, sum) and scanned for the label (the arithmetic of
+// fwd_tile_f32, on rounded logits).
 enum FwdStore : int { kStoreNone = 0, kStoreLogits = 1, kStoreExp = 2 };
 template <bool kCap, int kStore, bool kTail>
 __device__ __forceinline__ void fwd_epilogue_bf16(const f32x4_t (&acc)[8][8], float (&m2)[8],

@@ -266,12 +266,13 @@ class _FusedLinearCrossEntropyNone(torch.autograd.Function):
                 its GEMM -- the forward then also keeps the first vocabulary
                 block's exponentials for it, mt_flce_forward_keep, softcap
                 off -- else mt_flce_backward_tiles, dW as 256 x 256 fp32
-                tiles narrowed by mt_flce_narrow_tiles).  Where it pays
-                (bf16, no dw_accumulator, _kept_plan: every column fits up
-                to about H counted tokens) the forward keeps logits
-                (mt_flce_forward_logits) and the first backward recomputes
-                only the columns not kept (mt_flce_backward_logits): 6 H V n
-                flops instead of 8 when it keeps them all.
+                tiles narrowed by mt_flce_narrow_tiles).  Where it pays and
+                the device has the room (bf16, _kept_logits: without a
+                dw_accumulator every column fits up to about H counted
+                tokens) the forward keeps logits (mt_flce_forward_logits) as
+                a saved tensor and the first backward recomputes only the
+                columns not kept (mt_flce_backward_logits): 6 H V n flops
+                instead of 8 when it keeps them all.
     fused       grad_scale promised the upstream gradient at the forward and
                 the planner expects the fused path to pay (bf16,
                 mt_flce_fused_plan): the forward also forms dX and dW for it
@@ -832,7 +833,11 @@ def fused_linear_cross_entropy(hidden_states: torch.Tensor, lm_head_weight: torc
     the gradients for a unit upstream gradient and the backward rescales
     them when the gradient it receives is one scalar for every token (what
     train.py:97-104's sum and scaling produce), or recomputes for a per-token
-    one -- see _FusedLinearCrossEntropyNone.
+    one -- see _FusedLinearCrossEntropyNone.  Shorter bf16 calls (up to about H
+    counted tokens) keep the counted tokens' bf16 logits from the forward to
+    the backward instead of recomputing them: at most V H 2 bytes plus the
+    workspace budget, saved like any activation.  A budget set with
+    MT_FLCE_BWD_BUDGET_BYTES bounds them too.
 
     grad_scale (a float, or a [T] tensor of per-token values) promises the
     upstream gradient of the returned loss -- train.py:97-104 knows it before
