@@ -394,7 +394,7 @@ int mt_flce_general_pays(int64_t T, int64_t n_valid, int64_t H, int64_t V,
  * applied to the fp32 sums when dW goes to dW_out, else it is part of G, as a
  * per-token gradient is.  The scratch's size tells the number of dX slices: the
  * planned one at the planned size, fewer in less (but X^T, the queue and, for
- * keep_cols < V, the accumulator must fit).  n_valid >= 1, H a multiple of 8.
+ * keep_cols < V, one slice's accumulator or several slices' planes must fit).  n_valid >= 1, H a multiple of 8.
  * Replaces the same reference interface as mt_flce_forward and
  * mt_flce_backward (none_reduction_losses.py:16-23, whose Liger forward keeps
  * each chunk's logits to form the gradients from).

@@ -2345,7 +2345,11 @@ int mt_flce_backward_logits(const void* X, const void* W, int64_t T, int64_t H, 
        reinterpret_cast<uintptr_t>(scratch)) % 16 != 0)
     return fail(MT_ERR_INVALID_ARGUMENT, "dX, dW and scratch must be 16-byte aligned");
   MT_TRY(logits_args(n_valid, H, V, ldw, logits, keep_cols, logits_bytes));
-  const size_t need = kept_scratch(round_up(n_valid, 256), H, 1, keep_cols < V, dW_acc != nullptr);
+  // (below H = 256 several slices' planes may be smaller than one slice's tiles)
+  const int64_t C = round_up(n_valid, 256);
+  const size_t need = kept_scratch(
+      C, H, kept_slices_in(C, H, V, keep_cols, dW_acc != nullptr, scratch_bytes), keep_cols < V,
+      dW_acc != nullptr);
   if (!scratch || scratch_bytes < need)
     return fail(MT_ERR_WORKSPACE_TOO_SMALL, "logits scratch %zu bytes < required %zu", scratch_bytes, need);
   hipStream_t s = (hipStream_t)stream;

@@ -512,7 +512,7 @@ def test_forward_logits_host_checks(kw, code):
     (dict(logits=None), 1),
     (dict(scratch=None), 2),
     (dict(sb=64 * 256 * 2), 2),          # X^T without the work queue
-    (dict(cols=512, sb=64 * 256 * 2 + 256 + 65536 * 4 - 1), 2),  # blocks: dX's tiles too
+    (dict(cols=256, sb=64 * 256 * 2 + 256 + 65536 * 4 - 1), 2),  # blocks: dX's tiles too
     (dict(cols=512, acc=16, lddw=64, sb=64 * 256 * 2 + 256 + 64 * 256 * 4 - 1), 2),  # or rows
 ])
 def test_backward_logits_host_checks(kw, code):
@@ -575,3 +575,40 @@ def test_noalloc_chunks_fit_the_scratch():
             assert 0 < lib.mt_flce_noalloc_used_bytes(n, V, dtype) <= scratch, (n, V, dtype)
     for bad in ((0, 10, 0), (-1, 10, 0), (10, 0, 1), (10, 10, 7), (1 << 40, 10, 0)):
         assert lib.mt_flce_noalloc_used_bytes(*bad) == 0
+
+
+def test_planned_logits_scratch_is_accepted():
+    """Every plan of mt_flce_logits_plan passes the checks of both entries (the
+    call then fails at its first launch, in a process without a GPU): narrow
+    weights too, whose dX slices need less room than one slice's 256-column
+    tiles."""
+    if torch.cuda.is_available():
+        pytest.skip("launches with dummy pointers: a process without a GPU only")
+    lib, p = _lib.load(), 1 << 20
+    cols, lb, sb, pays = ctypes.c_int64(), ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_int()
+    rng = np.random.default_rng(4)
+
+    def log_int(lo, hi):
+        return int(round(np.exp(rng.uniform(np.log(lo), np.log(hi)))))
+
+    sizes = [(7809, 6758, 16, 115360), (580, 556, 8, 1151), (1362, 641, 8, 135855)]
+    sizes += [(T, int(rng.integers(1, T + 1)), log_int(8, 600) // 8 * 8, log_int(1, 160000))
+              for T in (log_int(1, 130000) for _ in range(1500))]
+    kept = 0
+    for T, n, H, V in sizes:
+        for budget, room, acc in ((max(192 << 20, T * V // 10), 1, 0), (3 << 20, 0, 0), (3 << 20, 0, 1)):
+            assert lib.mt_flce_logits_plan(T, n, H, V, H, 1, budget, room, acc, ctypes.byref(cols),
+                                           ctypes.byref(lb), ctypes.byref(sb), ctypes.byref(pays)) == 0
+            if not cols.value:
+                continue
+            kept += 1
+            size = dict(T=T, n=n, H=H, V=V, ldx=H, ldw=H, cols=cols.value, lb=lb.value)
+            ptr = dict(X=p, W=p, ri=p, rl=p, lse=p, logits=p)
+            assert call_forward_logits(**size, **ptr, loss=p, ws=p, wsb=1 << 40) == 4
+            out = dict(out=None, acc=p, lddw=H) if acc else dict(out=p, outb=V * H * 2)
+            assert call_backward_logits(**size, **ptr, **out, grad=p, dX=p, lddx=H, scratch=p,
+                                        sb=sb.value) == 4, (T, n, H, V, budget, acc)
+            # and no less than one slice's or the slices' room is
+            assert call_backward_logits(**size, **ptr, **out, grad=p, dX=p, lddx=H, scratch=p,
+                                        sb=H * -(-n // 256) * 512) == 2
+    assert kept > 1000

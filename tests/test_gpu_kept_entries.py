@@ -90,6 +90,8 @@ def test_slices_are_those_of_the_scratch(gpu, monkeypatch, H, slices):
     (300, 136, 5000, 1024, 1, True),
     (520, 264, 12500, 6144, 8, False),  # a last block (212 columns) with fewer stages than slices
     (520, 264, 12500, 6144, 8, True),
+    (511, 16, 5000, 2304, 8, False),    # slices' planes smaller than one slice's tiles
+    (511, 16, 5000, 512, 2, False),
 ])
 def test_guards_and_results(gpu, T, H, V, cols, slices, acc):
     """Against the same roundings of the logits in 64 bits: G is rounded to
